@@ -118,7 +118,7 @@ KERNEL_NAMES = {
     "lp_b4096": "pcd::k_lp_block<512, 8192, 1u, pcd::RangeSrc, false, 4, unsigned short>",
     "lp_hub_partition": "pcd::k_hub_partition<1u, false>",
     "lp_hub_count": "pcd::k_hub_count_listed<1u, 512, 4096, false>",
-    "stats_items": "pcd::k_stats_items_cached<1024>",
+    "stats_items": "pcd::k_stats_rows",
 }
 PMC_SUMMARY = os.path.join(ROOT, "profiles", "rmat22_mod_pmc.md")
 FETCH_FACTOR, WRITE_FACTOR = 2.0, 1.0  # stream-copy calibration of FETCH_SIZE / WRITE_SIZE

@@ -24,10 +24,39 @@ __global__ void k_first_init(int bound, const int32_t *labels, const int32_t *fi
     }
 }
 
-__global__ void k_first_occurrence(int n, const int32_t *labels, int32_t *first) {
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-        int l = labels[v];
-        if (l >= 0 && first[l] > v) atomicMin(&first[l], v);
+// The least vertex of every label.  A workgroup keeps the labels it meets
+// first in LDS (as StatsAcc does) and sends each one's least vertex to
+// memory at its end, so the members of a large community neither read its
+// word of `first` nor queue on it; other labels go to memory (R-MAT-20 under
+// a partition of hub neighbourhoods: 0.29 -> 0.05 ms; R-MAT-22 from many
+// small communities unchanged).  What bounds it is then the labels' read and
+// one random read per vertex of a small community.  A small table and four
+// vertices a thread: the flush of a full table costs as much as the reads it
+// saved.
+constexpr int FO_LOG = 7, FO_NT = 512;
+__global__ __launch_bounds__(FO_NT) void k_first_occurrence(int n, const int32_t *labels, int32_t *first) {
+    __shared__ int key[1 << FO_LOG], low[1 << FO_LOG];
+    for (int i = threadIdx.x; i < (1 << FO_LOG); i += FO_NT) {
+        key[i] = EMPTY_KEY;
+        low[i] = INT32_MAX;
+    }
+    __syncthreads();
+    for (int v = blockIdx.x * FO_NT + threadIdx.x; v < n; v += gridDim.x * FO_NT) {
+        const int l = labels[v];
+        if (l < 0) continue;
+        const int h = (int)(((uint32_t)l * 0x9E3779B1u) >> (32 - FO_LOG));
+        int k = __hip_atomic_load(&key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (k == EMPTY_KEY) {
+            k = atomicCAS(&key[h], EMPTY_KEY, l);
+            if (k == EMPTY_KEY) k = l;
+        }
+        if (k == l) atomicMin(&low[h], v);
+        else if (first[l] > v) atomicMin(&first[l], v);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < (1 << FO_LOG); i += FO_NT) {
+        const int l = key[i];
+        if (l != EMPTY_KEY && first[l] > low[i]) atomicMin(&first[l], low[i]);
     }
 }
 
@@ -91,8 +120,8 @@ int compress_labels_dev(pcd_ctx *ctx, bool defer_k) {
                            ctx->label_bound, ctx->d_labels, ctx->d_firstv, ctx->d_first);
     else if (ctx->label_bound > 0)
         PCD_TRY(fill_i32(ctx, ctx->d_first, INT32_MAX, ctx->label_bound));
-    hipLaunchKernelGGL(k_first_occurrence, dim3(grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, n, ctx->d_labels,
-                       ctx->d_first);
+    hipLaunchKernelGGL(k_first_occurrence, dim3(grid_for(ctx, n, FO_NT * 4, 4)), dim3(FO_NT), 0, ctx->stream, n,
+                       ctx->d_labels, ctx->d_first);
     // statistics of these labels (full count, or updated by the last
     // propagation step) are renumbered with them
     const bool renumber = ctx->stats_pending || ctx->has_stats;
@@ -143,128 +172,121 @@ __global__ void k_clear_stats(CommStats *st, const int32_t *kp) {
         st[c] = CommStats{0, 0, 0, 0};
 }
 
-// G lanes per vertex, vertices at positions [p0, p1) (all with degree <= G
-// is the fast case; larger degrees are still correct).
+// The whole recount in one launch: every wave takes work items {v, begin,
+// end, first} of the long rows (each lane PF gathers in flight), then its
+// share of the small bins, G lanes per vertex.  The labels of vertices
+// [0, ncache) are staged in LDS (ids are degree-descending: the most frequent
+// gather targets), and the sums go through the workgroup's accumulators, for
+// large communities' records are what the pass waited for: a recount of
+// R-MAT-20 (31 M entries) under a partition of hub neighbourhoods took 2.5 ms
+// with an atomic pair per row and takes 0.17 ms; from singletons, where the
+// label gathers bound it, R-MAT-22 (128 M entries) takes 0.62 ms either way.
+struct StatsRows {
+    int start[6];  // small bins G64..G4: positions [start[b], start[b + 1])
+    int nitems, ncache;
+    const int4 *items;
+    const int32_t *order, *indices, *adj, *labels;
+    CommStats *st;
+};
+constexpr int STATS_NT = 1024, STATS_LOG = 9;  // 64 + 8 KB of LDS: two workgroups per CU
+
+// A label from LDS or memory without a branch: both reads are issued (lanes
+// served by LDS all read word 0 in memory), so a row's gathers stay in flight
+// together.
+struct HotLabels {
+    const int32_t *hot, *labels;
+    int n;
+    __device__ int operator()(int v) const {
+        const bool in = v < n;
+        const int32_t g = labels[in ? 0 : v], h = hot[in ? v : 0];
+        return in ? h : g;
+    }
+};
+
 template <int G>
-__global__ __launch_bounds__(256) void k_stats_small(int p0, int p1, const int32_t *order, const int32_t *indices,
-                                                     const int32_t *adj, const int32_t *labels, CommStats *st) {
+__device__ inline void stats_small(const StatsRows &r, int b, int wave_g, int nwaves, const HotLabels &label,
+                                   StatsAcc<STATS_LOG> &acc) {
     const int lane = __lane_id(), glane = lane & (G - 1);
-    const int per_wave = WAVE / G;
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int count = p1 - p0;
+    constexpr int per_wave = WAVE / G;
+    const int p0 = r.start[b], count = r.start[b + 1] - p0;
     for (int base = wave_g * per_wave; base < count; base += nwaves * per_wave) {
-        int gi = base + lane / G;
-        bool has = gi < count;
-        int v = 0, start = 0, deg = 0, l = 0;
+        const int gi = base + lane / G;
+        const bool has = gi < count;
+        int start = 0, deg = 0, l = 0;
         if (has) {
-            int p = p0 + gi;
-            v = order ? order[p] : p;
-            start = indices[v];
-            deg = indices[v + 1] - start;
-            l = labels[v];
+            const int v = r.order ? r.order[p0 + gi] : p0 + gi;
+            start = r.indices[v];
+            deg = r.indices[v + 1] - start;
+            l = r.labels[v];
         }
         int same = 0;
-        for (int j = glane; j < deg; j += G) same += (labels[adj[start + j]] == l) ? 1 : 0;
+        for (int j = glane; j < deg; j += G) same += label(r.adj[start + j]) == l ? 1 : 0;
 #pragma unroll
         for (int d = G / 2; d > 0; d >>= 1) same += __shfl_xor(same, d, WAVE);
-        if (has && glane == 0) add_stats(st, l, 1, same, deg - same);
+        if (has && glane == 0) acc.add(r.st, l, 1, same, deg - same);
     }
 }
 
-// one wave per work item {v, begin, end, first} (rows longer than 64); each
-// lane keeps PF gathers in flight
-__global__ __launch_bounds__(256) void k_stats_items(int nitems, const int4 *items, const int32_t *adj,
-                                                     const int32_t *labels, CommStats *st) {
-    constexpr int PF = 8;
-    const int lane = __lane_id();
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    for (int it = wave_g; it < nitems; it += nwaves) {
-        int4 w = items[it];
-        int l = labels[w.x];
-        int same = 0;
-        for (int j0 = w.y + lane; j0 < w.z; j0 += PF * WAVE) {
-            int nb[PF];
-#pragma unroll
-            for (int e = 0; e < PF; e++) {
-                int j = j0 + e * WAVE;
-                nb[e] = j < w.z ? adj[j] : -1;
-            }
-#pragma unroll
-            for (int e = 0; e < PF; e++) same += (nb[e] >= 0 && labels[nb[e]] == l) ? 1 : 0;
-        }
-        same = wave_sum(same);
-        if (lane == 0) add_stats(st, l, w.w ? 1 : 0, same, (w.z - w.y) - same);
-    }
-}
-
-// Same work with the labels of vertices [0, ncache) staged in LDS: ids are
-// degree-descending, so those are the most frequent gather targets.  One
-// 1024-thread workgroup per CU pair of slots; each wave takes items as above.
-template <int NT>
-__global__ __launch_bounds__(NT) void k_stats_items_cached(int nitems, const int4 *items, const int32_t *adj,
-                                                           const int32_t *labels, CommStats *st, int ncache) {
+__global__ __launch_bounds__(STATS_NT) void k_stats_rows(StatsRows r) {
     constexpr int PF = 8;
     __shared__ int32_t hot[STATS_CACHE];
-    for (int i = threadIdx.x; i < ncache; i += NT) hot[i] = labels[i];
+    __shared__ StatsAcc<STATS_LOG> acc;
+    for (int i = threadIdx.x; i < r.ncache; i += STATS_NT) hot[i] = r.labels[i];
+    acc.init();
     __syncthreads();
+    const HotLabels label{hot, r.labels, r.ncache};
     const int lane = __lane_id();
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    for (int it = wave_g; it < nitems; it += nwaves) {
-        int4 w = items[it];
-        int l = labels[w.x];
+    const int wave_g = (blockIdx.x * STATS_NT + threadIdx.x) / WAVE;
+    const int nwaves = gridDim.x * STATS_NT / WAVE;
+    for (int it = wave_g; it < r.nitems; it += nwaves) {
+        const int4 w = r.items[it];
+        const int l = r.labels[w.x];
         int same = 0;
         for (int j0 = w.y + lane; j0 < w.z; j0 += PF * WAVE) {
             int nb[PF];
 #pragma unroll
             for (int e = 0; e < PF; e++) {
-                int j = j0 + e * WAVE;
-                nb[e] = j < w.z ? adj[j] : -1;
+                const int j = j0 + e * WAVE;
+                nb[e] = j < w.z ? r.adj[j] : -1;
             }
             int lab[PF];
 #pragma unroll
-            for (int e = 0; e < PF; e++) lab[e] = nb[e] < 0 ? -2 : (nb[e] < ncache ? hot[nb[e]] : labels[nb[e]]);
+            for (int e = 0; e < PF; e++) lab[e] = nb[e] < 0 ? -2 : label(nb[e]);
 #pragma unroll
             for (int e = 0; e < PF; e++) same += lab[e] == l ? 1 : 0;
         }
         same = wave_sum(same);
-        if (lane == 0) add_stats(st, l, w.w ? 1 : 0, same, (w.z - w.y) - same);
+        if (lane == 0) acc.add(r.st, l, w.w ? 1 : 0, same, (w.z - w.y) - same);
     }
-}
-
-template <int G>
-static void launch_stats_small(pcd_ctx *ctx, int p0, int p1) {
-    if (p1 <= p0) return;
-    int per_block = 256 / G;
-    hipLaunchKernelGGL(k_stats_small<G>, dim3(grid_for(ctx, p1 - p0, per_block, 16)), dim3(256), 0, ctx->stream, p0,
-                       p1, ctx->d_order, ctx->d_indices, ctx->d_adj, ctx->d_labels, ctx->d_stats);
+    stats_small<64>(r, 0, wave_g, nwaves, label, acc);
+    stats_small<32>(r, 1, wave_g, nwaves, label, acc);
+    stats_small<16>(r, 2, wave_g, nwaves, label, acc);
+    stats_small<8>(r, 3, wave_g, nwaves, label, acc);
+    stats_small<4>(r, 4, wave_g, nwaves, label, acc);
+    __syncthreads();
+    acc.flush(r.st);
 }
 
 int collect_statistics_dev(pcd_ctx *ctx) {
     const BinLayout &b = ctx->bins;
     hipLaunchKernelGGL(k_clear_stats, dim3(grid_for(ctx, ctx->k, 256)), dim3(256), 0, ctx->stream, ctx->d_stats,
                        ctx->d_k);
-    if (ctx->num_stat_items > 0) {
-        kt_begin(ctx, KS_STATS_ITEMS);
-        if (ctx->tune.stats_cache)
-            hipLaunchKernelGGL(k_stats_items_cached<1024>, dim3(std::min(ctx->cu_count * 2, ctx->num_stat_items)),
-                               dim3(1024), 0, ctx->stream, ctx->num_stat_items, ctx->d_stat_items, ctx->d_adj,
-                               ctx->d_labels, ctx->d_stats, std::min(ctx->n, STATS_CACHE));
-        else
-            hipLaunchKernelGGL(k_stats_items, dim3(grid_for(ctx, ctx->num_stat_items, 4, 16)), dim3(256), 0,
-                               ctx->stream, ctx->num_stat_items, ctx->d_stat_items, ctx->d_adj, ctx->d_labels,
-                               ctx->d_stats);
-        kt_end(ctx, KS_STATS_ITEMS);
-    }
-    kt_begin(ctx, KS_STATS_SMALL);
-    launch_stats_small<64>(ctx, b.start[BIN_G64], b.start[BIN_G64 + 1]);
-    launch_stats_small<32>(ctx, b.start[BIN_G32], b.start[BIN_G32 + 1]);
-    launch_stats_small<16>(ctx, b.start[BIN_G16], b.start[BIN_G16 + 1]);
-    launch_stats_small<8>(ctx, b.start[BIN_G8], b.start[BIN_G8 + 1]);
-    launch_stats_small<4>(ctx, b.start[BIN_G4], b.start[BIN_G4 + 1]);
-    kt_end(ctx, KS_STATS_SMALL);
+    StatsRows r;
+    for (int i = 0; i < 6; i++) r.start[i] = b.start[BIN_G64 + i];
+    r.nitems = ctx->num_stat_items;
+    r.ncache = ctx->tune.stats_cache ? std::min(ctx->n, STATS_CACHE) : 0;
+    r.items = ctx->d_stat_items;
+    r.order = ctx->d_order;
+    r.indices = ctx->d_indices;
+    r.adj = ctx->d_adj;
+    r.labels = ctx->d_labels;
+    r.st = ctx->d_stats;
+    // two workgroups per CU, at most one per 8192 entries: each stages its
+    // own copy of the cached labels
+    kt_begin(ctx, KS_STATS_ITEMS);
+    const int grid = std::max(grid_for(ctx, 2 * (int64_t)ctx->m, 8192, 2), grid_for(ctx, ctx->n, STATS_NT, 2) / 4);
+    hipLaunchKernelGGL(k_stats_rows, dim3(std::max(grid, 1)), dim3(STATS_NT), 0, ctx->stream, r);
+    kt_end(ctx, KS_STATS_ITEMS);
     PCD_HIP(hipGetLastError());
     ctx->has_stats = true;
     return PCD_OK;
@@ -334,7 +356,6 @@ struct MovedStore {
     }
 };
 
-// G lanes per moved vertex of one small bin (degree <= 64)
 // Moved bitmap: bit v of M is set when vertex v's label changed in the step
 // (L[v] != N[v]).  One wave writes one 64-bit word.
 __global__ __launch_bounds__(256) void k_moved_bits(int n, const int32_t *L, const int32_t *N, uint64_t *M) {
@@ -356,157 +377,166 @@ __device__ inline int label_before(const uint64_t *M, const int32_t *L, int w, i
     return ((M[w >> 6] >> (w & 63)) & 1) ? L[w] : after;
 }
 
+// Moved vertices of one small bin, G lanes each.  A wave takes up to
+// DELTA_BATCH entries of the list at once, one lane each, loads their rows
+// and labels together, and then runs through them two groups of 64 / G at a
+// time: what bounds it is the chain of dependent loads per row, which this
+// shortens from five to two for two rows.
+constexpr int DELTA_BATCH = 16, DELTA_LOG = 7;
 template <int G>
-__device__ inline void delta_small(int wave_g, int nwaves, const int32_t *list_all, const int32_t *bounds,
-                                   const int32_t *indices, const int32_t *adj, const int32_t *L, const int32_t *N,
-                                   const uint64_t *M, CommStats *st) {
+__device__ inline void delta_small(int wave_g, int nwaves, const int32_t *list, int cnt, const int32_t *indices, const int32_t *adj, const int32_t *L, const int32_t *N,
+                                   const HotLabels &after, const uint64_t *M, CommStats *st,
+                                   StatsAcc<DELTA_LOG> &acc) {
     const int lane = __lane_id(), glane = lane & (G - 1);
-    const int per_wave = WAVE / G;
-    const int32_t *list = list_all + bounds[0];
-    const int cnt = bounds[1] - bounds[0];
-    for (int base = wave_g * per_wave; base < cnt; base += nwaves * per_wave) {
-        const int gi = base + lane / G;
-        const bool has = gi < cnt;
-        int start = 0, deg = 0, lo = 0, ln = 0;
-        if (has) {
-            const int v = list[gi];
-            lo = L[v];
-            ln = N[v];
-            start = indices[v];
-            deg = indices[v + 1] - start;
+    constexpr int per_wave = WAVE / G;
+    // entries per batch: a multiple of per_wave that leaves no wave idle
+    const int share = (cnt + nwaves - 1) / nwaves;
+    const int batch = min(max(per_wave, DELTA_BATCH), (share + per_wave - 1) / per_wave * per_wave);
+    for (int base = wave_g * batch; base < cnt; base += nwaves * batch) {
+        const int left = min(batch, cnt - base);
+        int bstart = 0, bdeg = 0, blo = 0, bln = 0;
+        if (lane < left) {
+            const int v = list[base + lane];
+            blo = L[v];
+            bln = N[v];
+            bstart = indices[v];
+            bdeg = indices[v + 1] - bstart;
         }
-        int a = 0, b = 0;
-        for (int j = glane; j < deg; j += G) {
-            const int w = adj[start + j];
-            const int nw = N[w];
-            const int lw = label_before(M, L, w, nw);
-            const int f = lw != nw ? 1 : 2;
-            a += lw == lo ? f : 0;
-            b += nw == ln ? f : 0;
-        }
+        for (int g0 = 0; g0 < left; g0 += 2 * per_wave) {
+            int deg[2], lo[2], ln[2], w[2], nw[2], lw[2], a[2], b[2];
 #pragma unroll
-        for (int d = G / 2; d > 0; d >>= 1) {
-            a += __shfl_xor(a, d, WAVE);
-            b += __shfl_xor(b, d, WAVE);
-        }
-        if (has && glane == 0) {
-            add_stats(st, lo, -1, -a, a - deg);
-            if (ln >= 0) add_stats(st, ln, 1, b, deg - b);
+            for (int t = 0; t < 2; t++) {
+                const int gi = g0 + t * per_wave + lane / G;
+                const int src = gi < left ? gi : 0;
+                const int start = __shfl(bstart, src, WAVE);
+                deg[t] = __shfl(bdeg, src, WAVE);
+                lo[t] = __shfl(blo, src, WAVE);
+                ln[t] = __shfl(bln, src, WAVE);
+                if (gi >= left) deg[t] = 0;
+                w[t] = glane < deg[t] ? adj[start + glane] : -1;  // a row of the bin has at most G entries
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++) nw[t] = w[t] < 0 ? -2 : after(w[t]);
+#pragma unroll
+            for (int t = 0; t < 2; t++) lw[t] = w[t] < 0 ? -2 : label_before(M, L, w[t], nw[t]);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int f = lw[t] != nw[t] ? 1 : 2;
+                a[t] = w[t] >= 0 && lw[t] == lo[t] ? f : 0;
+                b[t] = w[t] >= 0 && nw[t] == ln[t] ? f : 0;
+#pragma unroll
+                for (int d = G / 2; d > 0; d >>= 1) {
+                    a[t] += __shfl_xor(a[t], d, WAVE);
+                    b[t] += __shfl_xor(b[t], d, WAVE);
+                }
+                if (g0 + t * per_wave + lane / G < left && glane == 0) {
+                    acc.add(st, lo[t], -1, -a[t], a[t] - deg[t]);
+                    if (ln[t] >= 0) acc.add(st, ln[t], 1, b[t], deg[t] - b[t]);
+                }
+            }
         }
     }
 }
 
-// Moved items {v, begin, end, first} (rows longer than 64): each wave reads
-// 64 list entries at once, lane j taking entry wave + (64 r + j) * waves in
-// round r, and runs their row chunks one after another; one long row's
-// chunks are spread over many waves.
-__device__ inline void delta_items(int wave_g, int nwaves, const int32_t *list_all, const int32_t *bounds,
-                                   const int4 *items, const int32_t *adj, const int32_t *L, const int32_t *N,
-                                   const uint64_t *M, CommStats *st) {
-    constexpr int PF = 4;
+// Moved items {v, begin, end, first} (rows longer than 64), one wave each:
+// workgroup b of nb takes list entries b, b + nb, ..., its waves whichever
+// comes next (rows differ 30-fold in length), and the next item's records are
+// on their way while one is counted.
+__device__ inline void delta_items(int wg, int nwg, int *next, const int32_t *list, int cnt, const int4 *items,
+                                   const int32_t *adj, const int32_t *L, const int32_t *N, const HotLabels &after,
+                                   const uint64_t *M, CommStats *st, StatsAcc<DELTA_LOG> &acc) {
+    constexpr int PF = 8;
     const int lane = __lane_id();
-    const int32_t *list = list_all + bounds[0];
-    const int cnt = bounds[1] - bounds[0];
-    for (int64_t r = 0; wave_g + r * WAVE * nwaves < cnt; r++) {
-        const int64_t i = wave_g + (r * WAVE + lane) * nwaves;
-        int4 w = make_int4(0, 0, 0, 0);
-        int lo = 0, ln = 0;
-        if (i < cnt) {
-            w = items[list[i]];
-            lo = L[w.x];
-            ln = N[w.x];
+    int4 wn = make_int4(0, 0, 0, 0);
+    int lon = 0, lnn = 0;
+    auto fetch = [&]() {
+        int j = 0;
+        if (lane == 0) j = atomicAdd(next, 1);
+        j = __builtin_amdgcn_readfirstlane(j);
+        const int64_t i = wg + (int64_t)j * nwg;
+        if (i >= cnt) return false;
+        wn = items[list[i]];
+        lon = L[wn.x];
+        lnn = N[wn.x];
+        return true;
+    };
+    bool more = fetch();
+    while (more) {
+        const int4 w = wn;
+        const int lo = lon, ln = lnn;
+        more = fetch();
+        int a = 0, b = 0;
+        for (int j0 = w.y + lane; j0 < w.z; j0 += PF * WAVE) {
+            int nb[PF];
+#pragma unroll
+            for (int e = 0; e < PF; e++) {
+                const int j = j0 + e * WAVE;
+                nb[e] = j < w.z ? adj[j] : -1;
+            }
+            int lw[PF], nw[PF];
+#pragma unroll
+            for (int e = 0; e < PF; e++) nw[e] = nb[e] < 0 ? -2 : after(nb[e]);
+#pragma unroll
+            for (int e = 0; e < PF; e++) lw[e] = nb[e] < 0 ? -2 : label_before(M, L, nb[e], nw[e]);
+#pragma unroll
+            for (int e = 0; e < PF; e++) {
+                if (nb[e] < 0) continue;
+                const int f = lw[e] != nw[e] ? 1 : 2;
+                a += lw[e] == lo ? f : 0;
+                b += nw[e] == ln ? f : 0;
+            }
         }
-        uint64_t mv = __ballot(i < cnt);
-        while (mv) {
-            const int src = __builtin_ctzll(mv);
-            mv &= mv - 1;
-            const int xb = __builtin_amdgcn_readlane(w.y, src), xe = __builtin_amdgcn_readlane(w.z, src);
-            const int xf = __builtin_amdgcn_readlane(w.w, src);
-            const int xlo = __builtin_amdgcn_readlane(lo, src), xln = __builtin_amdgcn_readlane(ln, src);
-            int a = 0, b = 0;
-            for (int j0 = xb + lane; j0 < xe; j0 += PF * WAVE) {
-                int nb[PF];
-#pragma unroll
-                for (int e = 0; e < PF; e++) {
-                    const int j = j0 + e * WAVE;
-                    nb[e] = j < xe ? adj[j] : -1;
-                }
-                int lw[PF], nw[PF];
-#pragma unroll
-                for (int e = 0; e < PF; e++) nw[e] = nb[e] < 0 ? -2 : N[nb[e]];
-#pragma unroll
-                for (int e = 0; e < PF; e++) lw[e] = nb[e] < 0 ? -2 : label_before(M, L, nb[e], nw[e]);
-#pragma unroll
-                for (int e = 0; e < PF; e++) {
-                    if (nb[e] < 0) continue;
-                    const int f = lw[e] != nw[e] ? 1 : 2;
-                    a += lw[e] == xlo ? f : 0;
-                    b += nw[e] == xln ? f : 0;
-                }
-            }
-            a = wave_sum(a);
-            b = wave_sum(b);
-            if (lane == 0) {
-                const int len = xe - xb;
-                add_stats(st, xlo, xf ? -1 : 0, -a, a - len);
-                if (xln >= 0) add_stats(st, xln, xf ? 1 : 0, b, len - b);
-            }
+        a = wave_sum(a);
+        b = wave_sum(b);
+        if (lane == 0) {
+            const int len = w.z - w.y;
+            acc.add(st, lo, w.w ? -1 : 0, -a, a - len);
+            if (ln >= 0) acc.add(st, ln, w.w ? 1 : 0, b, len - b);
         }
     }
 }
 
-// All six moved lists in one launch, so the short dependent-load chains of
-// the lists overlap instead of running one kernel after another.  Every
-// workgroup reads the six list lengths and computes the same split of the
-// grid into contiguous ranges, one per list, proportional to the list's
-// entries (at most G per small-bin vertex, DELTA_ITEM_COST per long-row
-// item), with at least one workgroup for a list that is not empty.  The
-// lists are disjoint and the updates are atomic adds.
-constexpr int DELTA_ITEM_COST = 512;
-__global__ __launch_bounds__(256) void k_delta_all(const int32_t *list_all, const int32_t *bounds, const int4 *items,
-                                                   const int32_t *indices, const int32_t *adj, const int32_t *L,
-                                                   const int32_t *N, const uint64_t *M, CommStats *st) {
-    __shared__ int s_lo[7];
-    if (threadIdx.x == 0) {
-        constexpr int cost[6] = {64, 32, 16, 8, 4, DELTA_ITEM_COST};
-        double w[6], tot = 0.0;
-        int nonempty = 0;
-        for (int l = 0; l < 6; l++) {
-            const int c = bounds[l + 1] - bounds[l];
-            w[l] = (double)c * cost[l];
-            tot += w[l];
-            nonempty += c > 0;
-        }
-        // one workgroup reserved per non-empty list, the rest by weight
-        const int spare = (int)gridDim.x - nonempty;
-        int at = 0;
-        double acc = 0.0;
-        for (int l = 0; l < 6; l++) {
-            s_lo[l] = at;
-            if (w[l] > 0) {
-                const int before = tot > 0 ? (int)(spare * (acc / tot)) : 0;
-                acc += w[l];
-                const int after = tot > 0 ? (int)(spare * (acc / tot)) : 0;
-                at += 1 + (after - before);
-            }
-        }
-        s_lo[6] = at;  // <= gridDim.x
-    }
+// All six moved lists in one launch: every wave takes its share of each list
+// in turn, from a place in the list that differs by list, so that short
+// lists fall to different waves and the lists' dependent-load chains overlap.
+// The sums go through the workgroup's accumulators: in a step that moves many
+// vertices into few communities the atomics on their records were the bound
+// (first step of CPM 0.01 on R-MAT-20, 15.7 M entries: 1.28 ms, now 0.22).
+// One resident round of workgroups: more of them measured slower once few
+// vertices move (24 us at twice as many, 12 us here), because every
+// workgroup pays the accumulators' start and flush.
+constexpr int DELTA_NT = 1024, DELTA_HOT_ITEMS = 2;
+__global__ __launch_bounds__(DELTA_NT) void k_delta_all(int n, const int32_t *list, const int32_t *bounds, const int4 *items,
+                                                        const int32_t *indices, const int32_t *adj, const int32_t *L,
+                                                        const int32_t *N, const uint64_t *M, CommStats *st) {
+    int bd[7];  // read at once: a read per list would lengthen every wave's chain
+#pragma unroll
+    for (int i = 0; i < 7; i++) bd[i] = bounds[i];
+    if (bd[0] == bd[6]) return;  // nothing moved
+    __shared__ int32_t hot[STATS_CACHE];
+    __shared__ StatsAcc<DELTA_LOG> acc;
+    const int nwaves = gridDim.x * DELTA_NT / WAVE;
+    // with several long-row items a wave, the labels of the most frequent
+    // neighbours are staged in LDS (as in k_stats_rows)
+    const HotLabels after{hot, N, bd[6] - bd[5] >= DELTA_HOT_ITEMS * nwaves ? min(n, STATS_CACHE) : 0};
+    for (int i = threadIdx.x; i < after.n; i += DELTA_NT) hot[i] = N[i];
+    __shared__ int next;
+    if (threadIdx.x == 0) next = 0;
+    acc.init();
     __syncthreads();
-    int l = 0;
-    while (l < 6 && !(s_lo[l] <= (int)blockIdx.x && (int)blockIdx.x < s_lo[l + 1])) l++;
-    if (l == 6) return;  // beyond the last range (rounding) or no moved rows
-    const int wpb = blockDim.x / WAVE;
-    const int wave_g = ((int)blockIdx.x - s_lo[l]) * wpb + (int)threadIdx.x / WAVE;
-    const int nwaves = (s_lo[l + 1] - s_lo[l]) * wpb;
-    switch (l) {
-    case 0: delta_small<64>(wave_g, nwaves, list_all, bounds + 0, indices, adj, L, N, M, st); break;
-    case 1: delta_small<32>(wave_g, nwaves, list_all, bounds + 1, indices, adj, L, N, M, st); break;
-    case 2: delta_small<16>(wave_g, nwaves, list_all, bounds + 2, indices, adj, L, N, M, st); break;
-    case 3: delta_small<8>(wave_g, nwaves, list_all, bounds + 3, indices, adj, L, N, M, st); break;
-    case 4: delta_small<4>(wave_g, nwaves, list_all, bounds + 4, indices, adj, L, N, M, st); break;
-    default: delta_items(wave_g, nwaves, list_all, bounds + 5, items, adj, L, N, M, st); break;
-    }
+    const int wave_g = (blockIdx.x * DELTA_NT + threadIdx.x) / WAVE;
+    auto place = [&](int i) {
+        const int w = wave_g + i * (nwaves / 6);
+        return w < nwaves ? w : w - nwaves;
+    };
+    delta_items(blockIdx.x, gridDim.x, &next, list + bd[5], bd[6] - bd[5], items, adj, L, N, after, M, st, acc);
+    delta_small<64>(place(1), nwaves, list + bd[0], bd[1] - bd[0], indices, adj, L, N, after, M, st, acc);
+    delta_small<32>(place(2), nwaves, list + bd[1], bd[2] - bd[1], indices, adj, L, N, after, M, st, acc);
+    delta_small<16>(place(3), nwaves, list + bd[2], bd[3] - bd[2], indices, adj, L, N, after, M, st, acc);
+    delta_small<8>(place(4), nwaves, list + bd[3], bd[4] - bd[3], indices, adj, L, N, after, M, st, acc);
+    delta_small<4>(place(5), nwaves, list + bd[4], bd[5] - bd[4], indices, adj, L, N, after, M, st, acc);
+    __syncthreads();
+    acc.flush(st);
 }
 
 int statistics_delta_dev(pcd_ctx *ctx, const int32_t *before, const int32_t *after) {
@@ -526,8 +556,9 @@ int statistics_delta_dev(pcd_ctx *ctx, const int32_t *before, const int32_t *aft
     uint64_t *M = ctx->d_moved_bits;
     hipLaunchKernelGGL(k_moved_bits, dim3(grid_for(ctx, (ctx->n + WAVE - 1) / WAVE, 4, 8)), dim3(256), 0, ctx->stream,
                        ctx->n, before, after, M);
-    // the lists of empty bins (and no items) are empty: their workgroups exit
-    hipLaunchKernelGGL(k_delta_all, dim3(ctx->cu_count * 24), dim3(256), 0, ctx->stream, list, bounds,
+    // two workgroups per CU, fewer for a small graph
+    const int delta_grid = std::max(8, grid_for(ctx, 2 * (int64_t)ctx->m, 2048, 2));
+    hipLaunchKernelGGL(k_delta_all, dim3(delta_grid), dim3(DELTA_NT), 0, ctx->stream, ctx->n, list, bounds,
                        ctx->d_stat_items, ctx->d_indices, ctx->d_adj, before, after, M, ctx->d_stats);
     kt_end(ctx, KS_STATS_DELTA);
     PCD_HIP(hipGetLastError());

@@ -1,0 +1,60 @@
+"""GPU parity where kernels share an address or a workgroup: partitions with
+a few large communities (every member's update falls on the same records),
+and sizes at the edges of tiles, tables and launch forms."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import gpu_graphs as GG
+
+pytestmark = pytest.mark.gpu
+
+parcd = pytest.importorskip("parcd")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    if parcd.device_count() < 1:
+        pytest.fail("no GPU visible to the HIP runtime")
+    c = parcd.Context(0)
+    yield c
+    c.close()
+
+
+def crowded(kind, n):
+    """Labels whose communities are few and large, or both large and many."""
+    rng = np.random.default_rng(11)
+    v = np.arange(n)
+    if kind == "one":
+        return np.full(n, n - 1, np.int32)
+    if kind == "half":  # one community of half the vertices among singletons
+        return np.where(rng.random(n) < 0.5, n // 2, v).astype(np.int32)
+    if kind == "table":  # more communities than a workgroup's accumulators, some of them large
+        return np.where(rng.random(n) < 0.7, rng.integers(0, 3, n), rng.integers(0, 900, n)).astype(np.int32)
+    return np.where(rng.random(n) < 0.1, -1, v % 7).astype(np.int32)  # seven communities and NEW_LABEL vertices
+
+
+@pytest.mark.parametrize("kind", ["one", "half", "table", "seven_new"])
+@pytest.mark.parametrize("graph", ["bin_zoo", "unsorted", "rmat12", "star"])
+def test_statistics_of_crowded_partitions(ctx, graph, kind):
+    """Compression, the full count, and the statistics updated from the moved
+    rows over four steps (crowded communities lose and gain many members at
+    once) equal the oracle's full count, for both tie orders."""
+    g = {"bin_zoo": GG.bin_zoo, "unsorted": lambda: GG.unsorted_copy(GG.bin_zoo()), "rmat12": lambda: GG.rmat(12),
+         "star": lambda: GG.csr_direct(700, [(0, i) for i in range(1, 700)])}[graph]()
+    n, m, ind, adj = g[:4]
+    ctx.upload_graph(n, m, ind, adj)
+    lab_in = crowded(kind, n)
+    ctx.upload_labels(lab_in)
+    for step, (rule, lam, tie) in enumerate([(O.MOD, 0.0, 1), (O.CPM, 0.01, 1), (O.CPM, 0.2, 0), (O.MOD, 0.0, 0)]):
+        k = ctx.compress()
+        want, k_o = O.compress_labels(lab_in)
+        assert k == k_o
+        lab = ctx.labels()
+        assert np.array_equal(lab, want)
+        assert ctx.statistics() == k
+        _, so, ivo, evo = O.collect_statistics(n, ind, adj, lab)
+        for got, w in zip(ctx.stats(k), (so, ivo, evo)):
+            assert np.array_equal(got, w), (graph, kind, step)
+        ctx.propagate(rule, lam, frac=0.9, seed=21, step=step, tie=tie)
+        lab_in = ctx.labels()
