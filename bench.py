@@ -837,16 +837,14 @@ def main():
         per_kernel[slot] = {"kernel": KERNEL_NAMES[slot], "bytes_per_launch": byt / launches,
                             "avg_ms": tms / launches, "entries_per_launch": sum(w[1] for w in work) / launches,
                             "gathers_per_launch": gathers / launches}
-    # statistics over rows longer than 64 (work items, the full count of the
-    # first iteration): per entry the neighbour id and its label, per row its
-    # extent and label and one 12-byte record update
-    deg = np.diff(ind)
-    big = deg > 64
+    # statistics (the full count of the first iteration, every row in one
+    # launch): per entry the neighbour id and its label, per row its extent
+    # and label and one 12-byte record update
     st_ms, st_launches = timers.get("stats_items", (0.0, 0))
     if st_ms > 0 and st_launches:
         per_kernel["stats_items"] = {"kernel": KERNEL_NAMES["stats_items"],
-                                     "bytes_per_launch": 8 * int(deg[big].sum()) + 20 * int(big.sum()),
-                                     "avg_ms": st_ms / st_launches, "entries_per_launch": int(deg[big].sum())}
+                                     "bytes_per_launch": 8 * E + 20 * n,
+                                     "avg_ms": st_ms / st_launches, "entries_per_launch": E}
     # the roofline kernel's average launch comes from the roofline pass
     if dom_probe in per_kernel:
         t_ms, t_launches = timed_dom.get(dom_probe, (0.0, 0))
