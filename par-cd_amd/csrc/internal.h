@@ -241,7 +241,9 @@ struct pcd_ctx {
 
     // triangles
     bool has_triangles = false;
-    int32_t *d_tri = nullptr, *d_tri_deg = nullptr, *d_et = nullptr;
+    int32_t *d_tri = nullptr, *d_tri_deg = nullptr;
+    uint8_t *d_tri_flag = nullptr;  // per entry: on a counted triangle
+    int32_t *d_tri_list = nullptr;  // number of vertices with long prefixes, then the vertices
     int32_t *d_lowpos = nullptr, *d_it = nullptr, *d_itd = nullptr;
     double cc = 0.0;
 

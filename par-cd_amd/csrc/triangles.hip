@@ -1,21 +1,27 @@
 // Triangle counting (Graph::count_triangles, graph.cpp:107-175) and the
 // internal-triangle pass of WCCRule::calculate (rules.cpp:150-235).
 //
-// For each vertex v and each neighbour u < v at row position r, the
-// reference intersects N(v) ∩ [0,u) -- which, rows being ascending, is the
-// row prefix of v before r -- with N(u) ∩ [0,u), and for every common w adds
-// one to the entry counters of (v,w), (u,w) and (v,u).  Here one wave owns
-// a vertex v: the row prefix of v (ids < v) and its entry counters are
-// staged in LDS, the wave walks u over that prefix, and for each u its lanes
-// take the entries of N(u) ∩ [0,u) and binary-search them in the staged
-// prefix.  Counters of row v stay in LDS and are added to memory once;
-// counters of (u,w) go to memory with atomics.  With labels given, only
-// edges and triangles inside one community count (rules.cpp:172,185).
+// For each vertex v and each neighbour u < v, the reference intersects
+// N(v) ∩ [0,u) with N(u) ∩ [0,u), and for every common w adds one to the
+// entry counters of (v,w), (u,w) and (v,u); then every entry (x,y), y < x,
+// with a positive counter adds it to both ends' totals and one edge to both
+// ends' degrees.  Here v's prefix (its neighbours below v) goes into an LDS
+// hash table and the entries of N(u) ∩ [0,u) are looked up in it, one LDS
+// read for most that are not there.  The counters of (v,·) live beside the
+// table, and they give every vertex total: the triangles of (v,p), v the
+// highest corner, add two to p each and two to v each.  Of (u,w) only "some
+// triangle uses this entry" matters, so a hit stores a flag byte instead of
+// adding to a counter in memory.  R-MAT-18 (3.8 M edges, 660 M lookups):
+// 6.4 ms with binary searches, an atomic per hit and a pass that summed the
+// counters with two atomics per edge; 1.2 ms so, 540 G lookups/s, bound by the
+// instructions and LDS reads of a lookup.  With labels given, only edges and triangles inside one
+// community count (rules.cpp:172,185): neighbours of other communities are
+// left out of the prefix.
+#include <algorithm>
+
 #include "prims.h"
 
 namespace pcd {
-
-constexpr int TRI_STAGE = 2048;  // staged prefix entries per wave
 
 // lowpos[v] = number of neighbours of v with a smaller id
 __global__ void k_lowpos(int n, const int32_t *indices, const int32_t *adj, int32_t *lowpos) {
@@ -30,215 +36,318 @@ __global__ void k_lowpos(int n, const int32_t *indices, const int32_t *adj, int3
     }
 }
 
+// prefixes of at most TRI_WAVE entries: one wave per vertex; longer ones,
+// listed once per graph: one workgroup per vertex
+constexpr int TRI_WAVE = 64, TRI_WAVE_LOG = 9;
+constexpr int TRI_BLOCK_LOG = 11, TRI_CHUNK = 1 << (TRI_BLOCK_LOG - 1);
+// vertices whose totals a workgroup sums in LDS: the lowest ids are the
+// highest degrees, and their words are what the additions queue on
+constexpr int TRI_HOT = 1024;
+constexpr int TRI_PF = 3;  // row entries a lane looks up at once
+
+struct TriArgs {
+    int n;
+    const int32_t *indices, *adj, *lowpos, *labels;
+    const int32_t *list, *listed;  // vertices with longer prefixes, their number
+    uint8_t *flag;                 // per entry (x,y), y < x: some counted triangle uses it
+    int32_t *tri;
+};
+
+struct LongPrefix {
+    const int32_t *lowpos;
+    __device__ int operator()(int64_t v) const { return lowpos[v] > TRI_WAVE ? 1 : 0; }
+};
+struct LongStore {
+    int32_t *list, *listed;
+    int64_t n;
+    __device__ void operator()(int64_t v, int ex, int flag) const {
+        if (flag) list[ex] = (int)v;
+        if (v == n - 1) *listed = ex + flag;
+    }
+};
+
 __device__ inline void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ inline int find_sorted(const int32_t *a, int len, int x) {
-    int lo = 0, hi = len;
-    while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (a[mid] < x) lo = mid + 1;
-        else hi = mid;
-    }
-    return (lo < len && a[lo] == x) ? lo : -1;
+// Table of at least 8 slots per entry (2 at the cap): what is not there is
+// then mostly told by one read (R-MAT-18: 1.46 ms at 4 slots, 1.23 at 8).
+__device__ inline int tri_log(int len) { return max(6, 32 - __clz(8 * len - 1)); }
+
+__device__ inline int tri_insert(int *keys, int log, int x) {
+    const int mask = (1 << log) - 1;
+    int h = (int)(((uint32_t)x * 0x9E3779B1u) >> (32 - log));
+    while (atomicCAS(&keys[h], EMPTY_KEY, x) != EMPTY_KEY) h = (h + 1) & mask;  // the keys of a row differ
+    return h;
 }
 
-// Vertices whose prefix exceeds FLAT_TS: one wave walks u over the prefix
-// and its lanes take the entries of N(u) ∩ [0,u).
-__global__ __launch_bounds__(256) void k_triangles(int n, const int32_t *indices, const int32_t *adj,
-                                                   const int32_t *lowpos, const int32_t *labels, int32_t *et,
-                                                   int min_len) {
-    __shared__ int32_t s_val[4][TRI_STAGE];
-    __shared__ int32_t s_cnt[4][TRI_STAGE];
-    const int lane = __lane_id(), w = threadIdx.x / WAVE;
-    int32_t *sval = s_val[w], *scnt = s_cnt[w];
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    for (int v = wave_g; v < n; v += nwaves) {
-        const int lenv = lowpos[v];
-        if (lenv < 2 || lenv <= min_len) continue;  // a triangle needs two smaller neighbours
-        const int sv = indices[v];
-        const int l = labels ? labels[v] : 0;
-        const bool staged = lenv <= TRI_STAGE;
-        const int32_t *vals = staged ? sval : adj + sv;
-        if (staged) {
-            for (int i = lane; i < lenv; i += WAVE) { sval[i] = adj[sv + i]; scnt[i] = 0; }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (int r = 1; r < lenv; r++) {
-            const int u = vals[r];
-            if (labels && labels[u] != l) continue;
-            const int su = indices[u], lenu = lowpos[u];
-            int found = 0;
-            for (int y = lane; y < lenu; y += WAVE) {
-                int wv = adj[su + y];
-                int x = find_sorted(vals, r, wv);
-                if (x >= 0 && (!labels || labels[wv] == l)) {
-                    found++;
-                    if (staged) atomicAdd(&scnt[x], 1);
-                    else atomicAdd(&et[sv + x], 1);
-                    atomicAdd(&et[su + y], 1);
-                }
-            }
-            found = wave_sum(found);
-            if (lane == 0 && found) {
-                if (staged) scnt[r] += found;
-                else atomicAdd(&et[sv + r], found);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (staged) {
-            for (int i = lane; i < lenv; i += WAVE)
-                if (scnt[i]) atomicAdd(&et[sv + i], scnt[i]);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// slot of x, or -1, given the key k of its first slot h; a table is never full
+__device__ inline int tri_probe(const int *keys, int log, int x, int h, int k) {
+    const int mask = (1 << log) - 1;
+    while (k != x && k != EMPTY_KEY) {
+        h = (h + 1) & mask;
+        k = keys[h];
     }
+    return k == x ? h : -1;
+}
+__device__ inline int tri_find(const int *keys, int log, int x) {
+    const int h = (int)(((uint32_t)x * 0x9E3779B1u) >> (32 - log));
+    return tri_probe(keys, log, x, h, keys[h]);
 }
 
-// Vertices with prefixes up to TS: the wedge checks (r, y) of vertex v --
-// u = the r-th prefix entry, w = the y-th entry of N(u) ∩ [0,u) -- are
-// flattened over the lanes (an exclusive scan of the per-r lengths in LDS,
-// a binary search of the lane's item in it), so a wave stays busy however
-// short the rows are.  Same checks and counts as k_triangles.
-constexpr int FLAT_TS = 256;  // 16 KB of LDS per workgroup: eight workgroups (32 waves) per CU
-
-template <int TS>
-__global__ __launch_bounds__(256) void k_triangles_flat(int n, const int32_t *indices, const int32_t *adj,
-                                                        const int32_t *lowpos, const int32_t *labels, int32_t *et) {
-    __shared__ int32_t s_val[4][TS];
-    __shared__ int32_t s_cnt[4][TS];
-    __shared__ int32_t s_su[4][TS];
-    __shared__ int32_t s_pre[4][TS + 1];
-    const int lane = __lane_id(), w = threadIdx.x / WAVE;
-    int32_t *sval = s_val[w], *scnt = s_cnt[w], *ssu = s_su[w], *spre = s_pre[w];
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    for (int v = wave_g; v < n; v += nwaves) {
-        const int lenv = lowpos[v];
-        if (lenv < 2 || lenv > TS) continue;
-        const int sv = indices[v];
-        const int l = labels ? labels[v] : 0;
-        int run = 0;
-        for (int base = 0; base < lenv; base += WAVE) {
-            const int i = base + lane;
-            int len = 0;
-            if (i < lenv) {
-                const int u = adj[sv + i];
-                int su = 0;
-                if (i >= 1 && (!labels || labels[u] == l)) {
-                    su = indices[u];
-                    len = lowpos[u];
-                }
-                sval[i] = u;
-                scnt[i] = 0;
-                ssu[i] = su;
-            }
-            const int inc = wave_incl_scan(len);
-            if (i < lenv) spre[i] = run + inc - len;
-            run += __shfl(inc, WAVE - 1, WAVE);
-        }
-        if (lane == 0) spre[lenv] = run;
-        wave_sync_lds();
-        for (int t = lane; t < run; t += WAVE) {
-            int lo = 0, hi = lenv;  // largest r with spre[r] <= t; its range holds t
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (spre[mid] <= t) lo = mid;
-                else hi = mid;
-            }
-            const int r = lo, y = t - spre[r];
-            const int su = ssu[r];
-            const int wv = adj[su + y];
-            const int x = find_sorted(sval, r, wv);
-            if (x >= 0 && (!labels || labels[wv] == l)) {
-                atomicAdd(&scnt[x], 1);
-                atomicAdd(&scnt[r], 1);
-                atomicAdd(&et[su + y], 1);
-            }
-        }
-        wave_sync_lds();
-        for (int i = lane; i < lenv; i += WAVE)
-            if (scnt[i]) atomicAdd(&et[sv + i], scnt[i]);
-        wave_sync_lds();
-    }
-}
-
-// graph.cpp:146-159 (rules.cpp:197-211): per entry (v,u) with t > 0,
-// t is added to both endpoints and each endpoint counts one edge.
-// Prefixes of at most ACC_G * 8 entries: ACC_G lanes per vertex, 64 / ACC_G
-// vertices per wave; longer prefixes: k_tri_accumulate, one wave each.
-constexpr int ACC_G = 8, ACC_SMALL = ACC_G * 8;
-__global__ __launch_bounds__(256) void k_tri_accumulate_small(int n, const int32_t *indices, const int32_t *adj,
-                                                              const int32_t *lowpos, const int32_t *et, int32_t *tri,
-                                                              int32_t *tdeg) {
-    const int lane = __lane_id(), glane = lane & (ACC_G - 1);
-    const int gid = (blockIdx.x * blockDim.x + threadIdx.x) / ACC_G;
-    const int ngroups = gridDim.x * blockDim.x / ACC_G;
-    // the lanes of a group share v, so the group's shuffles stay inside
-    // lanes that are active together
-    for (int v = gid; v < n; v += ngroups) {
-        const int lenv = lowpos[v];
-        const bool mine = lenv <= ACC_SMALL;
-        const int sv = mine ? indices[v] : 0;
-        int ts = 0, tc = 0;
-        for (int i = glane; mine && i < lenv; i += ACC_G) {
-            int t = et[sv + i];
-            if (t > 0) {
-                int u = adj[sv + i];
-                ts += t;
-                tc++;
-                atomicAdd(&tri[u], t);
-                atomicAdd(&tdeg[u], 1);
-            }
-        }
+// W lanes look the entries [s, s + len) up, PF a lane in flight; returns
+// this lane's hits
+template <int W, int PF>
+__device__ inline int tri_row(const TriArgs &a, const int *keys, int *cnts, int log, int s, int len, int glane) {
+    int found = 0;
+    for (int y = glane; y < len; y += PF * W) {
+        int x[PF], k[PF];
 #pragma unroll
-        for (int d = ACC_G / 2; d > 0; d >>= 1) {
-            ts += __shfl_xor(ts, d, WAVE);
-            tc += __shfl_xor(tc, d, WAVE);
-        }
-        if (glane == 0 && tc) {
-            atomicAdd(&tri[v], ts);
-            atomicAdd(&tdeg[v], tc);
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_tri_accumulate(int n, const int32_t *indices, const int32_t *adj,
-                                                        const int32_t *lowpos, const int32_t *et, int32_t *tri,
-                                                        int32_t *tdeg) {
-    const int lane = __lane_id();
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    for (int v = wave_g; v < n; v += nwaves) {
-        const int lenv = lowpos[v];
-        if (lenv <= ACC_SMALL) continue;  // k_tri_accumulate_small
-        const int sv = indices[v];
-        int ts = 0, tc = 0;
-        for (int i = lane; i < lenv; i += WAVE) {
-            int t = et[sv + i];
-            if (t > 0) {
-                int u = adj[sv + i];
-                ts += t;
-                tc++;
-                atomicAdd(&tri[u], t);
-                atomicAdd(&tdeg[u], 1);
+        for (int e = 0; e < PF; e++) x[e] = a.adj[s + min(y + e * W, len - 1)];
+#pragma unroll
+        for (int e = 0; e < PF; e++) k[e] = keys[((uint32_t)x[e] * 0x9E3779B1u) >> (32 - log)];
+#pragma unroll
+        for (int e = 0; e < PF; e++) {
+            if (y + e * W >= len || k[e] == EMPTY_KEY) continue;
+            const int h = tri_probe(keys, log, x[e], (int)(((uint32_t)x[e] * 0x9E3779B1u) >> (32 - log)), k[e]);
+            if (h >= 0) {
+                found++;
+                atomicAdd(&cnts[h], 1);
+                a.flag[s + y + e * W] = 1;
             }
         }
-        ts = wave_sum(ts);
-        tc = wave_sum(tc);
-        if (lane == 0 && tc) {
-            atomicAdd(&tri[v], ts);
-            atomicAdd(&tdeg[v], tc);
+    }
+    return found;
+}
+
+__device__ inline void tri_add(const TriArgs &a, int *hot, int x, int c) {
+    if (x < TRI_HOT) atomicAdd(&hot[x], c);
+    else atomicAdd(&a.tri[x], c);
+}
+
+template <int NT>
+__device__ inline void tri_flush(const TriArgs &a, const int *hot) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < TRI_HOT; i += NT)
+        if (hot[i]) atomicAdd(&a.tri[i], hot[i]);
+}
+
+// A wave looks at eight vertices at once, eight lanes each, and takes those
+// with at least two (same-label) neighbours below them one by one.  Rows
+// u are read 64 lanes wide, or four at a time 16 lanes wide where they are
+// short on average (Chung-Lu rows hold 30-60 entries, R-MAT rows 150-190).
+__global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a) {
+    __shared__ int s_keys[256 / WAVE][1 << TRI_WAVE_LOG], s_cnts[256 / WAVE][1 << TRI_WAVE_LOG];
+    __shared__ int s_row[256 / WAVE][3][TRI_WAVE];
+    __shared__ int hot[TRI_HOT];
+    for (int i = threadIdx.x; i < TRI_HOT; i += 256) hot[i] = 0;
+    __syncthreads();
+    const int lane = __lane_id(), w = threadIdx.x / WAVE, oct = lane & 7;
+    const uint64_t below = (1ULL << lane) - 1;
+    int *keys = s_keys[w], *cnts = s_cnts[w];
+    int *rsu = s_row[w][0], *rlen = s_row[w][1], *rcnt = s_row[w][2];
+    const int wave_g = (blockIdx.x * 256 + threadIdx.x) / WAVE;
+    const int nwaves = gridDim.x * (256 / WAVE);
+    for (int64_t base = (int64_t)wave_g * 8; base < a.n; base += (int64_t)nwaves * 8) {
+        const int vo = (int)min((int64_t)a.n - 1, base + lane / 8);
+        int plen = base + lane / 8 < a.n ? a.lowpos[vo] : 0;
+        if (plen > TRI_WAVE) plen = 0;
+        const int pstart = a.indices[vo], plab = a.labels ? a.labels[vo] : 0;
+        int mine = plen;
+        if (a.labels) {
+            mine = 0;
+            for (int i = oct; i < plen; i += 8) mine += a.labels[a.adj[pstart + i]] == plab;
+#pragma unroll
+            for (int d = 4; d > 0; d >>= 1) mine += __shfl_xor(mine, d, WAVE);
         }
+        uint64_t todo = __ballot(oct == 0 && mine >= 2);
+        while (todo) {
+            const int src = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int v = (int)base + src / 8;
+            const int len = __builtin_amdgcn_readlane(plen, src), sv = __builtin_amdgcn_readlane(pstart, src);
+            const int lab = __builtin_amdgcn_readlane(plab, src);
+            const int log = tri_log(len);
+            for (int i = lane; i < (1 << log); i += WAVE) {
+                keys[i] = EMPTY_KEY;
+                cnts[i] = 0;
+            }
+            int u = -1, su = 0, lu = 0, slot = 0;
+            if (lane < len) {
+                u = a.adj[sv + lane];
+                if (a.labels && a.labels[u] != lab) u = -1;
+                if (u >= 0) {
+                    su = a.indices[u];
+                    lu = a.lowpos[u];
+                }
+            }
+            wave_sync_lds();
+            if (u >= 0) slot = tri_insert(keys, log, u);
+            if (lane == 0) lu = 0;  // no neighbour lies below the lowest
+            wave_sync_lds();
+            uint64_t rows = __ballot(lu > 0);
+            const int nrows = __popcll(rows), total = wave_sum(lu);
+            int found = 0;  // of this lane's row
+            if (total > 32 * nrows) {
+                while (rows) {
+                    const int r = __builtin_ctzll(rows);
+                    rows &= rows - 1;
+                    const int f = wave_sum(tri_row<WAVE, TRI_PF>(a, keys, cnts, log, __builtin_amdgcn_readlane(su, r),
+                                                         __builtin_amdgcn_readlane(lu, r), lane));
+                    if (lane == r) found = f;
+                }
+            } else {
+                const int at = __popcll(rows & below);
+                if (lu > 0) {
+                    rsu[at] = su;
+                    rlen[at] = lu;
+                }
+                wave_sync_lds();
+                for (int i = lane / 16; i < nrows; i += WAVE / 16) {
+                    int f = tri_row<16, 2>(a, keys, cnts, log, rsu[i], rlen[i], lane & 15);
+#pragma unroll
+                    for (int d = 8; d > 0; d >>= 1) f += __shfl_xor(f, d, WAVE);
+                    if ((lane & 15) == 0) rcnt[i] = f;
+                }
+                wave_sync_lds();
+                if (lu > 0) found = rcnt[at];
+            }
+            wave_sync_lds();
+            const int c = u >= 0 ? cnts[slot] + found : 0;
+            if (c) {
+                a.flag[sv + lane] = 1;
+                tri_add(a, hot, u, 2 * c);
+            }
+            const int tv = wave_sum(c);
+            if (lane == 0 && tv) tri_add(a, hot, v, tv);
+            wave_sync_lds();
+        }
+    }
+    tri_flush<256>(a, hot);
+}
+
+// One workgroup per listed vertex: its prefix goes into the table in chunks,
+// and for each chunk the waves take the rows behind the chunk's first entry
+// (64 rows' extents loaded at once, one lane each).
+__global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
+    constexpr int NT = 256, NW = NT / WAVE;
+    __shared__ int keys[1 << TRI_BLOCK_LOG], cnts[1 << TRI_BLOCK_LOG];
+    __shared__ int hot[TRI_HOT];
+    for (int i = threadIdx.x; i < TRI_HOT; i += NT) hot[i] = 0;
+    const int lane = __lane_id(), w = threadIdx.x / WAVE;
+    const int nlist = *a.listed;
+    for (int it = blockIdx.x; it < nlist; it += gridDim.x) {
+        const int v = a.list[it];
+        const int sv = a.indices[v], len = a.lowpos[v], lab = a.labels ? a.labels[v] : 0;
+        int tv = 0;
+        for (int c0 = 0; c0 < len; c0 += TRI_CHUNK) {
+            const int c1 = min(len, c0 + TRI_CHUNK);
+            const int log = min(TRI_BLOCK_LOG, tri_log(c1 - c0));
+            for (int i = threadIdx.x; i < (1 << log); i += NT) {
+                keys[i] = EMPTY_KEY;
+                cnts[i] = 0;
+            }
+            __syncthreads();
+            for (int i = c0 + threadIdx.x; i < c1; i += NT) {
+                const int u = a.adj[sv + i];
+                if (!a.labels || a.labels[u] == lab) tri_insert(keys, log, u);
+            }
+            __syncthreads();
+            // wave w takes rows c0 + 1 + w, + NW, ...
+            for (int r0 = c0 + 1 + w; r0 < len; r0 += NW * WAVE) {
+                const int r = r0 + NW * lane;
+                int u = -1, su = 0, lu = 0;
+                if (r < len) {
+                    u = a.adj[sv + r];
+                    if (!a.labels || a.labels[u] == lab) {
+                        su = a.indices[u];
+                        lu = a.lowpos[u];
+                    }
+                }
+                int found = 0;
+                uint64_t rows = __ballot(lu > 0);
+                while (rows) {
+                    const int i = __builtin_ctzll(rows);
+                    rows &= rows - 1;
+                    const int f = wave_sum(tri_row<WAVE, TRI_PF>(a, keys, cnts, log, __builtin_amdgcn_readlane(su, i),
+                                                         __builtin_amdgcn_readlane(lu, i), lane));
+                    if (lane == i) found = f;
+                }
+                if (found) {
+                    a.flag[sv + r] = 1;
+                    tri_add(a, hot, u, 2 * found);
+                    tv += found;
+                }
+            }
+            __syncthreads();
+            for (int i = threadIdx.x; i < (1 << log); i += NT) {
+                const int c = cnts[i];
+                if (c) {
+                    tri_add(a, hot, keys[i], 2 * c);
+                    tv += c;
+                }
+            }
+            for (int i = c0 + threadIdx.x; i < c1; i += NT) {
+                const int x = tri_find(keys, log, a.adj[sv + i]);
+                if (x >= 0 && cnts[x]) a.flag[sv + i] = 1;
+            }
+            __syncthreads();
+        }
+        tv = wave_sum(tv);
+        if (lane == 0 && tv) tri_add(a, hot, v, tv);
+    }
+    tri_flush<NT>(a, hot);
+}
+
+// Each flagged entry (v,u) counts one edge at both ends (graph.cpp:146-159,
+// rules.cpp:197-211): eight lanes per vertex, one wave per listed vertex.
+constexpr int TDEG_NT = 1024, TDEG_HOT = 4096;
+__global__ __launch_bounds__(TDEG_NT) void k_tri_degrees(TriArgs a, int32_t *tdeg) {
+    __shared__ int hot[TDEG_HOT];
+    for (int i = threadIdx.x; i < TDEG_HOT; i += TDEG_NT) hot[i] = 0;
+    __syncthreads();
+    const int lane = __lane_id();
+    auto add = [&](int x, int c) {
+        if (x < TDEG_HOT) atomicAdd(&hot[x], c);
+        else atomicAdd(&tdeg[x], c);
+    };
+    auto entries = [&](int s, int len, int first, int step) {
+        int c = 0;
+        for (int i = first; i < len; i += step)
+            if (a.flag[s + i]) {
+                c++;
+                add(a.adj[s + i], 1);
+            }
+        return c;
+    };
+    const int64_t g = ((int64_t)blockIdx.x * TDEG_NT + threadIdx.x) / 8, ng = (int64_t)gridDim.x * TDEG_NT / 8;
+    for (int64_t v = g; v < a.n; v += ng) {  // the lanes of a group share v
+        const int len = a.lowpos[v];
+        int c = len <= TRI_WAVE ? entries(a.indices[v], len, lane & 7, 8) : 0;
+#pragma unroll
+        for (int d = 4; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
+        if ((lane & 7) == 0 && c) add((int)v, c);
+    }
+    const int nlist = *a.listed;
+    for (int it = (blockIdx.x * TDEG_NT + threadIdx.x) / WAVE; it < nlist; it += gridDim.x * TDEG_NT / WAVE) {
+        const int v = a.list[it];
+        const int c = wave_sum(entries(a.indices[v], a.lowpos[v], lane, WAVE));
+        if (lane == 0 && c) add(v, c);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < TDEG_HOT; i += TDEG_NT)
+        if (hot[i]) atomicAdd(&tdeg[i], hot[i]);
+}
+
+// flags of E entries (padded to words) and both totals, cleared
+__global__ void k_tri_clear(int64_t words, uint32_t *flag, int n, int32_t *tri, int32_t *tdeg) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (int64_t i = t; i < words; i += stride) flag[i] = 0;
+    for (int64_t i = t; i < n; i += stride) {
+        tri[i] = 0;
+        tdeg[i] = 0;
     }
 }
 
@@ -305,35 +414,40 @@ __global__ __launch_bounds__(256) void k_sum_partials_plain(const double *part, 
 static int ensure_tri_buffers(pcd_ctx *ctx) {
     if (ctx->d_tri) return PCD_OK;
     const int64_t E = (int64_t)2 * ctx->m;
-    PCD_TRY(dev_alloc_t(ctx, &ctx->d_tri, ctx->n + 1));
+    int32_t *tri = nullptr;
+    PCD_TRY(dev_alloc_t(ctx, &tri, ctx->n + 1));
     PCD_TRY(dev_alloc_t(ctx, &ctx->d_tri_deg, ctx->n + 1));
-    PCD_TRY(dev_alloc_t(ctx, &ctx->d_et, E + 1));
+    PCD_TRY(dev_alloc_t(ctx, &ctx->d_tri_flag, E + 4));
     PCD_TRY(dev_alloc_t(ctx, &ctx->d_lowpos, ctx->n + 1));
     PCD_TRY(dev_alloc_t(ctx, &ctx->d_it, ctx->n + 1));
     PCD_TRY(dev_alloc_t(ctx, &ctx->d_itd, ctx->n + 1));
+    // prefixes above 64 entries: at most E / 65 vertices, and their number
+    const int64_t cap = std::min<int64_t>(ctx->n, E / (TRI_WAVE + 1)) + 1;
+    PCD_TRY(dev_alloc_t(ctx, &ctx->d_tri_list, cap + 1));
     hipLaunchKernelGGL(k_lowpos, dim3(grid_for(ctx, ctx->n, 256)), dim3(256), 0, ctx->stream, ctx->n, ctx->d_indices,
                        ctx->d_adj, ctx->d_lowpos);
+    PCD_TRY(device_scan(ctx, ctx->n, LongPrefix{ctx->d_lowpos},
+                        LongStore{ctx->d_tri_list + 1, ctx->d_tri_list, ctx->n}, nullptr));
     PCD_HIP(hipGetLastError());
+    ctx->d_tri = tri;  // set last: the others are there
     return PCD_OK;
 }
 
-// Runs the counting pass (labels: nullptr for all triangles) into et and
-// accumulates per-vertex totals into (t, td).
+// Runs the counting pass (labels: nullptr for all triangles) and leaves the
+// per-vertex totals in (t, td).
 static int count_pass(pcd_ctx *ctx, const int32_t *labels, int32_t *t, int32_t *td) {
     const int n = ctx->n;
     const int64_t E = (int64_t)2 * ctx->m;
+    const TriArgs a{n,      ctx->d_indices,      ctx->d_adj,      ctx->d_lowpos,   labels,
+                    ctx->d_tri_list + 1, ctx->d_tri_list, ctx->d_tri_flag, t};
     kt_begin(ctx, KS_TRIANGLES);
-    PCD_TRY(fill_i32(ctx, ctx->d_et, 0, E));
-    PCD_TRY(fill_i32(ctx, t, 0, n));
-    PCD_TRY(fill_i32(ctx, td, 0, n));
-    hipLaunchKernelGGL(k_triangles_flat<FLAT_TS>, dim3(grid_for(ctx, n, 4, 8)), dim3(256), 0, ctx->stream, n,
-                       ctx->d_indices, ctx->d_adj, ctx->d_lowpos, labels, ctx->d_et);
-    hipLaunchKernelGGL(k_triangles, dim3(grid_for(ctx, n, 4, 2)), dim3(256), 0, ctx->stream, n, ctx->d_indices,
-                       ctx->d_adj, ctx->d_lowpos, labels, ctx->d_et, FLAT_TS);
-    hipLaunchKernelGGL(k_tri_accumulate_small, dim3(grid_for(ctx, n, 256 / ACC_G, 8)), dim3(256), 0, ctx->stream, n,
-                       ctx->d_indices, ctx->d_adj, ctx->d_lowpos, ctx->d_et, t, td);
-    hipLaunchKernelGGL(k_tri_accumulate, dim3(grid_for(ctx, n, 4, 8)), dim3(256), 0, ctx->stream, n, ctx->d_indices,
-                       ctx->d_adj, ctx->d_lowpos, ctx->d_et, t, td);
+    const int64_t words = (E + 3) / 4;
+    hipLaunchKernelGGL(k_tri_clear, dim3(grid_for(ctx, std::max<int64_t>(words, n), 256 * 4)), dim3(256), 0,
+                       ctx->stream, words, (uint32_t *)ctx->d_tri_flag, n, t, td);
+    // several rounds of workgroups: vertices differ a hundredfold in work
+    hipLaunchKernelGGL(k_triangles_block, dim3(ctx->cu_count * 24), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL(k_triangles_wave, dim3(grid_for(ctx, n, 4 * 8, 24)), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL(k_tri_degrees, dim3(grid_for(ctx, n, TDEG_NT / 8, 2)), dim3(TDEG_NT), 0, ctx->stream, a, td);
     kt_end(ctx, KS_TRIANGLES);
     PCD_HIP(hipGetLastError());
     return PCD_OK;

@@ -58,3 +58,42 @@ def test_statistics_of_crowded_partitions(ctx, graph, kind):
             assert np.array_equal(got, w), (graph, kind, step)
         ctx.propagate(rule, lam, frac=0.9, seed=21, step=step, tie=tie)
         lab_in = ctx.labels()
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 66, 130, 1025, 1026, 2051])
+def test_triangles_of_cliques(ctx, n):
+    """Prefixes at the edges of the wave table (64), of a workgroup table's
+    chunk (1024) and over several chunks: in a clique of n with one pendant
+    vertex every vertex is on C(n-1, 2) triangles and every edge but the
+    pendant's on one."""
+    i, j = np.triu_indices(n, 1)
+    g = GG.csr_from_edges(np.append(i, 0), np.append(j, n))
+    ctx.upload_graph(*g[:4])
+    tri, tdeg, cc = ctx.triangles()
+    deg = np.diff(g[2])
+    inside = deg > 1 if n > 2 else np.zeros(n + 1, bool)
+    assert np.array_equal(tri, np.where(inside, (n - 1) * (n - 2), 0))
+    assert np.array_equal(tdeg, np.where(inside, n - 1, 0))
+    want = (tri / np.maximum(deg * (deg - 1.0), 1.0)).sum() / (n + 1)
+    assert cc == pytest.approx(want, rel=1e-12, abs=1e-300)
+
+
+@pytest.mark.parametrize("labels", [1, 2, 7])
+@pytest.mark.parametrize("graph", ["bin_zoo", "dense", "unsorted"])
+def test_internal_triangles(ctx, graph, labels):
+    """WCC of partitions with long and short prefixes inside and across
+    communities, over several passes that reuse the flags."""
+    g = {"bin_zoo": GG.bin_zoo, "dense": GG.dense_blocks, "unsorted": lambda: GG.unsorted_copy(GG.bin_zoo())}[graph]()
+    n, m, ind, adj = g[:4]
+    ctx.upload_graph(n, m, ind, adj)
+    tri, tdeg, _ = ctx.triangles()
+    _, t_o, td_o, _ = O.count_triangles(n, ind, adj)
+    assert np.array_equal(tri, t_o) and np.array_equal(tdeg, td_o)
+    for seed in (1, 2):
+        lab, _ = O.compress_labels(np.random.default_rng(seed).integers(0, labels, n).astype(np.int32))
+        ctx.upload_labels(lab)
+        ctx.compress()
+        ctx.statistics()
+        s, _, _ = O.collect_statistics(n, ind, adj, lab)[1:]
+        want = O.wcc_calculate(n, ind, adj, lab, s, t_o, td_o)[0]
+        assert ctx.metric(O.WCC) == pytest.approx(want, rel=1e-9, abs=1e-12)
