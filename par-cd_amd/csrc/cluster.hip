@@ -83,42 +83,83 @@ __global__ void k_order_of(int n, const uint64_t *sorted, int32_t *order, uint8_
     }
 }
 
-// One round, one wave per vertex in order.  *open is set when a vertex stays
+// Rows up to OCT_ROW entries are read by eight lanes, eight vertices to a
+// wave; the longer ones among the eight by the whole wave afterwards.  Most
+// vertices a round meets are decided already, and most rows are short: with a
+// wave per vertex a round of the 1 M vertex Chung-Lu graph took 63 us when
+// hardly any vertex was left, 99 us on average; eight to a wave 8 and 35 us.
+constexpr int OCT_ROW = 128;
+
+// any lane of the aligned group of eight / of the wave
+__device__ inline bool oct_any(bool x) { return ((__ballot(x) >> (__lane_id() & ~7)) & 0xff) != 0; }
+
+// Among the W lanes' entries of row [b, e): a center with an earlier key, an
+// open vertex with an earlier key (this lane's view).
+template <int W>
+__device__ inline void center_scan(int b, int e, int first, uint64_t kv, const int32_t *adj, const uint64_t *key,
+                                   const uint8_t *state, bool &center_before, bool &open_before) {
+    for (int j = b + first; j < e && !center_before; j += W) {
+        const int u = adj[j];
+        if (key[u] < kv) {
+            const uint8_t s = state[u];
+            center_before |= s == ST_CENTER;
+            open_before |= s == ST_OPEN;
+        }
+    }
+}
+
+// One round over the vertices in order.  *open is set when a vertex stays
 // undecided.
 __global__ __launch_bounds__(256) void k_center_round(int n, const int32_t *order, const int32_t *indices,
                                                       const int32_t *adj, const uint64_t *key, uint8_t *state,
                                                       int32_t *open) {
-    const int lane = __lane_id();
+    const int lane = __lane_id(), oct = lane & 7;
     const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
     const int nwaves = gridDim.x * blockDim.x / WAVE;
     bool left = false;
-    for (int t = wave_g; t < n; t += nwaves) {
-        const int v = order[t];
-        if (state[v] != ST_OPEN) continue;
-        const uint64_t kv = key[v];
-        const int b = indices[v], e = indices[v + 1];
+    for (int64_t base = (int64_t)wave_g * 8; base < n; base += (int64_t)nwaves * 8) {
+        const int64_t t = base + lane / 8;
+        const int v = t < n ? order[t] : 0;
+        const bool mine = t < n && state[v] == ST_OPEN;
+        if (!__ballot(mine)) continue;
+        uint64_t kv = 0;
+        int b = 0, e = 0;
+        if (mine) {
+            kv = key[v];
+            b = indices[v];
+            e = indices[v + 1];
+        }
+        const bool small = e - b <= OCT_ROW;
         bool center_before = false, open_before = false;
-        for (int j0 = b; j0 < e; j0 += WAVE) {
-            const int j = j0 + lane;
-            if (j < e) {
-                const int u = adj[j];
-                if (key[u] < kv) {
-                    const uint8_t s = state[u];
-                    center_before |= s == ST_CENTER;
-                    open_before |= s == ST_OPEN;
-                }
+        if (mine && small) center_scan<8>(b, e, oct, kv, adj, key, state, center_before, open_before);
+        const bool any_center = oct_any(center_before), any_open = oct_any(open_before);
+        if (mine && small) {
+            if (oct == 0 && any_center) state[v] = ST_MEMBER;
+            else if (oct == 0 && !any_open) state[v] = ST_CENTER;
+            left |= !any_center && any_open;
+        }
+        uint64_t todo = __ballot(mine && !small && oct == 0);
+        while (todo) {
+            const int src = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int lv = __builtin_amdgcn_readlane(v, src), lb = __builtin_amdgcn_readlane(b, src);
+            const int le = __builtin_amdgcn_readlane(e, src);
+            const uint64_t lk = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(kv >> 32), src) << 32) |
+                                (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)kv, src);
+            bool c = false, o = false;
+            for (int j0 = lb; j0 < le; j0 += 4 * WAVE) {  // a few chunks between the checks for an end
+                center_scan<WAVE>(j0, min(le, j0 + 4 * WAVE), lane, lk, adj, key, state, c, o);
+                if (__ballot(c)) break;
             }
-            if (__ballot(center_before)) break;
+            const bool ac = __ballot(c) != 0, ao = __ballot(o) != 0;
+            if (lane == 0) {
+                if (ac) state[lv] = ST_MEMBER;
+                else if (!ao) state[lv] = ST_CENTER;
+            }
+            left |= !ac && ao;
         }
-        const bool any_center = __ballot(center_before) != 0;
-        const bool any_open = __ballot(open_before) != 0;
-        if (lane == 0) {
-            if (any_center) state[v] = ST_MEMBER;
-            else if (!any_open) state[v] = ST_CENTER;
-        }
-        left |= !any_center && any_open;
     }
-    if (lane == 0 && left) *open = 1;
+    if (__ballot(left) && lane == 0) *open = 1;
 }
 
 // center ids: exclusive scan of "is a center" over the order
@@ -136,23 +177,49 @@ struct CenterStore {
 };
 
 // every other vertex: the id of its center neighbour with the smallest key
+// (eight lanes per short row, a wave per longer one, as above)
+__device__ inline uint64_t min_xor(uint64_t x, int d) {
+    return min(x, (uint64_t)__shfl_xor((unsigned long long)x, d, WAVE));
+}
+template <int W>
+__device__ inline uint64_t first_center(int b, int e, int first, const int32_t *adj, const uint64_t *key,
+                                        const uint8_t *state) {
+    uint64_t best = ~0ULL;
+    for (int j = b + first; j < e; j += W) {
+        const int u = adj[j];
+        if (state[u] == ST_CENTER) best = min(best, key[u]);
+    }
+    return best;
+}
+
 __global__ __launch_bounds__(256) void k_member_labels(int n, const int32_t *indices, const int32_t *adj,
                                                        const uint64_t *key, const uint8_t *state, int32_t *labels) {
-    const int lane = __lane_id();
+    const int lane = __lane_id(), oct = lane & 7;
     const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
     const int nwaves = gridDim.x * blockDim.x / WAVE;
-    for (int v = wave_g; v < n; v += nwaves) {
-        if (state[v] != ST_MEMBER) continue;
-        uint64_t best = ~0ULL;
-        for (int j = indices[v] + lane; j < indices[v + 1]; j += WAVE) {
-            const int u = adj[j];
-            if (state[u] == ST_CENTER) best = min(best, key[u]);
-        }
+    // a member always has an earlier center neighbour; the tests keep a
+    // corrupt state from writing out of bounds
+    // a wave's eight vertices lie nwaves apart: ids are degree-descending, and
+    // the longest rows would otherwise fall to a few waves
+    for (int64_t base = wave_g; base < n; base += (int64_t)nwaves * 8) {
+        const int64_t v = base + (int64_t)(lane / 8) * nwaves;
+        const bool mine = v < n && state[v] == ST_MEMBER;
+        const int b = mine ? indices[v] : 0, e = mine ? indices[v + 1] : 0;
+        const bool small = e - b <= OCT_ROW;
+        uint64_t best = mine && small ? first_center<8>(b, e, oct, adj, key, state) : ~0ULL;
 #pragma unroll
-        for (int d = WAVE / 2; d > 0; d >>= 1) best = min(best, (uint64_t)__shfl_xor((unsigned long long)best, d, WAVE));
-        // a member always has an earlier center neighbour; the test keeps a
-        // corrupt state from writing out of bounds
-        if (lane == 0 && best != ~0ULL) labels[v] = labels[(int)(uint32_t)best];
+        for (int d = 4; d > 0; d >>= 1) best = min_xor(best, d);
+        if (mine && small && oct == 0 && best != ~0ULL) labels[v] = labels[(int)(uint32_t)best];
+        uint64_t todo = __ballot(mine && !small && oct == 0);
+        while (todo) {
+            const int src = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            uint64_t lb = first_center<WAVE>(__builtin_amdgcn_readlane(b, src), __builtin_amdgcn_readlane(e, src), lane,
+                                             adj, key, state);
+#pragma unroll
+            for (int d = WAVE / 2; d > 0; d >>= 1) lb = min_xor(lb, d);
+            if (lane == 0 && lb != ~0ULL) labels[base + (int64_t)(src / 8) * nwaves] = labels[(int)(uint32_t)lb];
+        }
     }
 }
 
@@ -205,7 +272,7 @@ int clustering_labels_dev(pcd_ctx *ctx, int *num_communities) {
     bool done = false;
     for (int r = 0; r < ctx->tune.cluster_rounds; r++) {
         PCD_CL(fill_i32(ctx, open, 0, 1));
-        hipLaunchKernelGGL(k_center_round, dim3(grid_for(ctx, n, 4, 8)), dim3(256), 0, ctx->stream, n, order,
+        hipLaunchKernelGGL(k_center_round, dim3(grid_for(ctx, n, 4 * 8, 8)), dim3(256), 0, ctx->stream, n, order,
                            ctx->d_indices, ctx->d_adj, fkey, state, open);
         if (hipGetLastError() != hipSuccess) PCD_CL(fail(PCD_E_HIP, "k_center_round launch"));
         if (hipMemcpyAsync(ctx->h_small, open, 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
@@ -246,7 +313,7 @@ int clustering_labels_dev(pcd_ctx *ctx, int *num_communities) {
     }
     int32_t *total = nullptr;
     PCD_CL(device_scan(ctx, n, CenterFlag{order, state}, CenterStore{order, ctx->d_labels}, &total));
-    hipLaunchKernelGGL(k_member_labels, dim3(grid_for(ctx, n, 4, 8)), dim3(256), 0, ctx->stream, n, ctx->d_indices,
+    hipLaunchKernelGGL(k_member_labels, dim3(grid_for(ctx, n, 4 * 8, 8)), dim3(256), 0, ctx->stream, n, ctx->d_indices,
                        ctx->d_adj, fkey, state, ctx->d_labels);
     if (hipGetLastError() != hipSuccess) PCD_CL(fail(PCD_E_HIP, "k_member_labels launch"));
     if (hipMemcpyAsync(ctx->h_small, total, 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
