@@ -205,7 +205,10 @@ int pcd_bin_counters(pcd_ctx *ctx, int bin, int64_t *active, int64_t *entries, i
  * before it gives up and the sort is finished by three-launch passes;
  * default 2^20; 0 makes the second pass of every sort of more than one tile
  * give up, for tests of that fallback) and "scan_tiles_per_cu" (scans use
- * shorter tiles until there are this many per CU; default 8, in [1, 64]).
+ * shorter tiles until there are this many per CU; default 8, in [1, 64]) and
+ * "solo_loop" (0/1: pcd_iterate_many and pcd_refine run the propagation passes
+ * of a graph of at most 4096 vertices and 32768 entries, under modularity or
+ * CPM, in one launch of one workgroup).
  * Results do not depend on them. */
 int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value);
 /* Hub label partitions whose distinct labels overflowed their LDS table

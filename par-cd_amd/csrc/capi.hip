@@ -212,6 +212,7 @@ static void free_graph_state(pcd_ctx *ctx) {
     ctx->d_tri = ctx->d_tri_deg = ctx->d_tri_list = nullptr;
     ctx->d_lowpos = ctx->d_it = ctx->d_itd = nullptr;
     ctx->d_tri_flag = nullptr;
+    ctx->d_solo = nullptr;
     ctx->d_keys0 = ctx->d_keys1 = nullptr;
     ctx->keys_cap = 0;
     ctx->d_pair_links = ctx->d_pair_head = nullptr;
@@ -887,6 +888,8 @@ extern "C" int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value) {
         ctx->tune.merge_sort = value != 0;
     } else if (k == "graph_loop") {
         ctx->tune.graph_loop = value != 0;
+    } else if (k == "solo_loop") {
+        ctx->tune.solo_loop = value != 0;
     } else if (k == "graph_loop_min_entries") {
         if (value < 0) return fail(PCD_E_INVALID, "graph_loop_min_entries must be >= 0");
         ctx->tune.graph_loop_min_entries = value;

@@ -114,6 +114,7 @@ struct Tuning {
                                  // (R-MAT-22 iteration 1.120 ms at 2, 1.102 at 8, 1.131 at 32)
     int graph_loop = 1;          // modularity / CPM with -s 0: passes replayed from one captured
                                  // pass with the stop rule on the device (pcd_iterate_many)
+    int solo_loop = 1;           // the passes of a small graph in one launch of one workgroup (solo.hip)
     int graph_loop_min_entries = 0;  // graphs with fewer CSR entries run pass by pass
     int merge_sort = 0;          // merging picks partners from the sorted unique community pairs
                                  // (1) or counts over community rows, no sort of the entries (0)
@@ -152,6 +153,14 @@ struct HubLayoutHost {
 int build_hub_layout(const std::vector<int4> &rows, int part_entries, HubLayoutHost &L);
 
 struct pcd_ctx_impl;
+
+// What a loop on one workgroup (solo.hip) ended with: the pass it stopped at,
+// whether the stop rule fired there, the communities of that pass, and those
+// and the score of the last completed pass.
+struct SoloResult {
+    int it, done, k, last_k;
+    double score;
+};
 
 }  // namespace pcd
 
@@ -256,6 +265,7 @@ struct pcd_ctx {
     // device-resident loop (loop.hip): one captured pass, replayed
     bool capturing = false;          // a pass is being captured: no host reads, no pointer swaps of stats
     const int *graph_step = nullptr; // the captured pass reads its step number here
+    pcd::SoloResult *d_solo = nullptr;  // result of the one-workgroup loop (solo.hip)
     void *loop = nullptr;            // the captured pass and its device state (loop.hip)
     int64_t alloc_gen = 0;           // counts device allocations and frees (a capture's buffers)
     int64_t tune_gen = 0;            // counts tuning changes (a capture's kernel forms)
@@ -344,6 +354,11 @@ int contract_dev(pcd_ctx *ctx, int64_t *num_pairs);
 int contract_download(pcd_ctx *ctx, int64_t U, int32_t *l, int32_t *k, int32_t *links);
 int triangles_dev(pcd_ctx *ctx);
 int wcc_metric_dev(pcd_ctx *ctx, double *out);
+
+// the loop of a small graph on one workgroup (solo.hip)
+constexpr int SOLO_MAX_N = 4096, SOLO_MAX_E = 32768, SOLO_MAX_PASSES = 4096;
+bool solo_fits(const pcd_ctx *ctx, const pcd_job *job, int strategy);
+int solo_passes(pcd_ctx *ctx, const pcd_job *job, int cap, int it, int count, double prev, SoloResult *res);
 
 RuleParams make_rule(pcd_ctx *ctx, pcd_rule rule);
 

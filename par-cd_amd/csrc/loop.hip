@@ -314,6 +314,23 @@ extern "C" int pcd_iterate_many(pcd_ctx *ctx, const pcd_job *job, int strategy, 
     const int cap = job->iter_cap > 0 ? job->iter_cap : 1000;
     double prev = prev_score;
     int run = 0;
+    if (ctx->tune.graph_loop && ctx->tune.solo_loop && ctx->tune.inc_stats &&
+        2 * (int64_t)ctx->m >= ctx->tune.graph_loop_min_entries && !ctx->counters && !ctx->timing &&
+        solo_fits(ctx, job, strategy)) {
+        // a small graph: the passes in one launch, up to SOLO_MAX_PASSES at a time
+        PCD_HIP(hipSetDevice(ctx->device));
+        while (run < count && !*done) {
+            SoloResult r;
+            PCD_TRY(solo_passes(ctx, job, cap, it + run, std::min(count - run, SOLO_MAX_PASSES), prev, &r));
+            run = r.it - it + (r.done ? 1 : 0);
+            prev = r.score;
+            *passes = run;
+            *score = r.score;
+            *num_labels = r.last_k;
+            *done = r.done;
+        }
+        return PCD_OK;
+    }
     // pass by pass until the statistics follow the labels (the first pass
     // of labels from outside counts them in full), or for the rules and
     // strategies the captured pass does not cover

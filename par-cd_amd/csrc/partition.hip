@@ -596,10 +596,7 @@ __global__ __launch_bounds__(256) void k_metric_sums(const CommStats *st, const 
 }
 
 __global__ void k_metric_final(const unsigned long long *acc, int kind, double lambda, int m, double *out) {
-    long long a = (long long)acc[0], b = (long long)acc[1], c = (long long)acc[2];
-    double two_m = 2.0 * m;
-    if (kind == PCD_RULE_MODULARITY) *out = a / two_m - (double)b / (two_m * two_m);
-    else *out = (a - lambda * (double)c) / (double)(2 * m);
+    *out = score_of_sums((long long)acc[0], (long long)acc[1], (long long)acc[2], kind, lambda, m);
 }
 
 constexpr int FSUM_BLOCKS = 1024;

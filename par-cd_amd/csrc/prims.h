@@ -79,6 +79,14 @@ struct StatsAcc {
     }
 };
 
+// rules.cpp:9-22 (modularity) and rules.cpp:121-129 (CPM) from the exact sums of
+// int_volume, volume^2 and size (size - 1)
+__device__ inline double score_of_sums(long long a, long long b, long long c, int kind, double lambda, int m) {
+    const double two_m = 2.0 * m;
+    if (kind == PCD_RULE_MODULARITY) return a / two_m - (double)b / (two_m * two_m);
+    return (a - lambda * (double)c) / (double)(2 * m);
+}
+
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ROUNDS = 16;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ROUNDS;

@@ -97,3 +97,70 @@ def test_internal_triangles(ctx, graph, labels):
         s, _, _ = O.collect_statistics(n, ind, adj, lab)[1:]
         want = O.wcc_calculate(n, ind, adj, lab, s, t_o, td_o)[0]
         assert ctx.metric(O.WCC) == pytest.approx(want, rel=1e-9, abs=1e-12)
+
+
+def small_graphs():
+    """Sizes at the edges of the one-workgroup loop: degrees in every table
+    class, isolated vertices, unsorted ids, the largest vertex and entry
+    counts it takes and the first it does not."""
+    rng = np.random.default_rng(3)
+    out = {"tiny_" + name: GG.csr_direct(*g) for name, g in GG.TINY.items()}
+    out["sbm"] = GG.sbm(21, 10, 0.5, 0.02)
+    out["rmat9"] = GG.rmat(9)
+    out["rmat10_unsorted"] = GG.unsorted_copy(GG.rmat(10, factor=8))
+    star = [(0, i) for i in range(1, 4096)]
+    out["hub_4095"] = GG.csr_direct(4096, star + [(i, i + 1) for i in range(1, 1200)])
+    for name, n, m in (("n4096", 4096, 12000), ("n4097", 4097, 12000), ("e32768", 3000, 16384), ("e32770", 3000, 16385),
+                       ("degree_70_300", 500, 15000)):
+        a, b = rng.integers(0, n, (2, 4 * m))
+        if name.startswith("degree"):
+            a = np.where(rng.random(a.size) < 0.5, a % 60, a)
+        keep = a < b
+        e = np.unique(np.stack([a[keep], b[keep]], 1), axis=0)
+        e = e[rng.permutation(len(e))[:m]]
+        assert len(e) == m
+        out[name] = GG.csr_direct(n, [tuple(x) for x in e.tolist()])
+    return out
+
+
+SMALL = small_graphs()
+
+
+@pytest.mark.parametrize("name", sorted(SMALL))
+def test_small_graph_loop(ctx, name):
+    """Refinement and ranges of passes equal the pass-by-pass loop: labels,
+    score, passes, communities and statistics, from labels of outside (with
+    NEW_LABEL) and from where another range stopped."""
+    n, m, ind, adj = SMALL[name][:4]
+    rng = np.random.default_rng(n + m)
+    starts = [rng.permutation(n).astype(np.int32), np.where(rng.random(n) < 0.3, -1, rng.integers(0, max(1, n // 9), n))]
+    ctx.upload_graph(n, m, ind, adj)
+    for i, (kind, lam, tie, frac) in enumerate([(O.MOD, 0.0, 0, 0.5), (O.CPM, 0.05, 1, 0.5), (O.CPM, 0.3, 0, 1.0),
+                                                (O.MOD, 0.0, 1, 0.8)]):
+        lab = starts[i % 2].astype(np.int32)
+        got = []
+        for solo, graph in ((1, 1), (0, 1), (0, 0)):
+            ctx.set_tuning("solo_loop", solo)
+            ctx.set_tuning("graph_loop", graph)
+            one = []
+            for job in (parcd.job(kind=kind, lam=lam, frac=frac, tie=tie, seed=5, iter_cap=40),
+                        parcd.job(kind=kind, lam=lam, frac=frac, tie=tie, seed=6, max_iter=7)):
+                ctx.upload_labels(lab)
+                score, it, k = ctx.refine(job)
+                one += [score, it, k, ctx.labels()] + list(ctx.stats(k))
+            job = parcd.job(kind=kind, lam=lam, frac=frac, tie=tie, seed=5, iter_cap=1000, max_iter=900)
+            ctx.upload_labels(lab)
+            at, prev = 0, 0.0
+            for count in (1, 3, 2):
+                p, prev, k, done = ctx.iterate_many(job, at, count, prev)
+                assert p == count and not done
+                at += p
+                one += [prev, k]
+            one += [ctx.iterate(job, at, prev)[0], ctx.compress(), ctx.labels()]
+            got.append(one)
+        ctx.set_tuning("solo_loop", 1)
+        ctx.set_tuning("graph_loop", 1)
+        for other in got[1:]:
+            assert len(other) == len(got[0])
+            for x, y in zip(got[0], other):
+                assert np.array_equal(x, y, equal_nan=True) if isinstance(x, float) else np.array_equal(x, y), (name, i)
