@@ -208,7 +208,9 @@ int pcd_bin_counters(pcd_ctx *ctx, int bin, int64_t *active, int64_t *entries, i
  * shorter tiles until there are this many per CU; default 8, in [1, 64]) and
  * "solo_loop" (0/1: pcd_iterate_many and pcd_refine run the propagation passes
  * of a graph of at most 4096 vertices and 32768 entries, under modularity or
- * CPM, in one launch of one workgroup).
+ * CPM, in one launch of one workgroup) and "fused_pass" (0/1: a
+ * device-resident propagation pass under modularity or CPM shares launches
+ * between compression, metric, stop rule and bookkeeping).
  * Results do not depend on them. */
 int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value);
 /* Hub label partitions whose distinct labels overflowed their LDS table

@@ -888,6 +888,8 @@ extern "C" int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value) {
         ctx->tune.merge_sort = value != 0;
     } else if (k == "graph_loop") {
         ctx->tune.graph_loop = value != 0;
+    } else if (k == "fused_pass") {
+        ctx->tune.fused_pass = value != 0;
     } else if (k == "solo_loop") {
         ctx->tune.solo_loop = value != 0;
     } else if (k == "graph_loop_min_entries") {

@@ -114,6 +114,7 @@ struct Tuning {
                                  // (R-MAT-22 iteration 1.120 ms at 2, 1.102 at 8, 1.131 at 32)
     int graph_loop = 1;          // modularity / CPM with -s 0: passes replayed from one captured
                                  // pass with the stop rule on the device (pcd_iterate_many)
+    int fused_pass = 1;          // a captured propagation pass (modularity, CPM) shares launches between its parts
     int solo_loop = 1;           // the passes of a small graph in one launch of one workgroup (solo.hip)
     int graph_loop_min_entries = 0;  // graphs with fewer CSR entries run pass by pass
     int merge_sort = 0;          // merging picks partners from the sorted unique community pairs
@@ -153,6 +154,27 @@ struct HubLayoutHost {
 int build_hub_layout(const std::vector<int4> &rows, int part_entries, HubLayoutHost &L);
 
 struct pcd_ctx_impl;
+
+// State of the device-resident loop (loop.hip)
+struct LoopState {
+    int it;        // pass the next replay runs (main.cpp's it)
+    int step;      // step number the captured propagation reads: it, or -1 once frozen
+    int it_end;    // first pass not requested
+    int frozen;    // stopped: done, or it_end reached
+    int done;      // the stop rule fired
+    int just;      // frozen in the current pass: the snapshot copies
+    int k_freeze;  // communities after the frozen pass's compression
+    int cur_k;     // communities of the current pass
+    int prev_k;    // communities of the last completed pass
+    int arrived;   // workgroups of the pass's metric that have added their sums
+    double prev;        // score of the last completed pass
+    double cur;         // score of the current pass
+    double score_done;  // score of the pass at which the rule fired
+};
+struct LoopParams {
+    int max_iter, cap;
+    double threshold;
+};
 
 // What a loop on one workgroup (solo.hip) ended with: the pass it stopped at,
 // whether the stop rule fired there, the communities of that pass, and those
@@ -265,6 +287,9 @@ struct pcd_ctx {
     // device-resident loop (loop.hip): one captured pass, replayed
     bool capturing = false;          // a pass is being captured: no host reads, no pointer swaps of stats
     const int *graph_step = nullptr; // the captured pass reads its step number here
+    // set while a pass of the fused form is captured: its state (the statistics
+    // update closes the pass) and the rule whose totals are there already
+    pcd::LoopState *fused = nullptr;
     pcd::SoloResult *d_solo = nullptr;  // result of the one-workgroup loop (solo.hip)
     void *loop = nullptr;            // the captured pass and its device state (loop.hip)
     int64_t alloc_gen = 0;           // counts device allocations and frees (a capture's buffers)
@@ -325,6 +350,11 @@ int ensure_sort_space(pcd_ctx *ctx, int64_t n);
 // memory; resolve_k takes it once the stream has passed the copy.
 int compress_labels_dev(pcd_ctx *ctx, bool defer_k = false);
 void resolve_k(pcd_ctx *ctx);
+// the captured pass's compression, metric (modularity or CPM), stop rule and
+// gain totals, in as few launches as the dependences between them allow
+int fused_compress_dev(pcd_ctx *ctx, pcd_rule rule, const LoopParams &p, LoopState *state);
+// what the first replay finds where a pass leaves it for the next
+int fused_prepare(pcd_ctx *ctx);
 // drops the captured pass of the device-resident loop (loop.hip)
 void loop_release(pcd_ctx *ctx);
 // drops the merging step's row state (merge.hip); its device buffers belong

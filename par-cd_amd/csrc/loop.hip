@@ -15,6 +15,12 @@
 // The host launches a few replays at a time and reads the record once per
 // batch of replays, never once per pass; at the end it puts the kept copy
 // back.  The result equals pcd_iterate called pass by pass.
+//
+// Under modularity and CPM with -s 0 a pass takes the fused form: its
+// compression, metric, rule and bookkeeping share launches (fused_compress_dev),
+// and no copy is kept, since what the replays after the stop leave is the
+// stopped pass's own result: a compression of compressed labels changes
+// nothing and no vertex moves.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -24,53 +30,8 @@
 
 namespace pcd {
 
-struct LoopState {
-    int it;        // pass the next replay runs (main.cpp's it)
-    int step;      // step number the captured propagation reads: it, or -1 once frozen
-    int it_end;    // first pass not requested
-    int frozen;    // stopped: done, or it_end reached
-    int done;      // the stop rule fired
-    int just;      // frozen in the current pass: the snapshot copies
-    int k_freeze;  // communities after the frozen pass's compression
-    int cur_k;     // communities of the current pass
-    int prev_k;    // communities of the last completed pass
-    int pad;
-    double prev;        // score of the last completed pass
-    double cur;         // score of the current pass
-    double score_done;  // score of the pass at which the rule fired
-};
-
-struct LoopParams {
-    int max_iter, cap;
-    double threshold;
-};
-
 __global__ void k_loop_rule(LoopState *s, const double *score, const int32_t *dk, LoopParams p) {
-    if (s->frozen) return;
-    const int it = s->it;
-    const int k = *dk;
-    if (it >= s->it_end) {
-        s->frozen = 1;
-        s->just = 1;
-        s->k_freeze = k;
-        s->step = -1;
-        return;
-    }
-    const double sc = *score;
-    const bool known = (p.max_iter != -1 && it >= p.max_iter) || it >= p.cap;
-    const bool d = known || (p.max_iter == -1 && s->prev > 0 && sc > 0 && sc / s->prev - 1 <= p.threshold);
-    s->cur = sc;
-    s->cur_k = k;
-    if (d) {
-        s->frozen = 1;
-        s->done = 1;
-        s->just = 1;
-        s->k_freeze = k;
-        s->score_done = sc;
-        s->step = -1;
-    } else {
-        s->step = it;
-    }
+    loop_rule(s, *score, *dk, p);
 }
 
 __global__ void k_loop_snapshot(const LoopState *s, int n, const int32_t *labels, const CommStats *stats,
@@ -82,14 +43,7 @@ __global__ void k_loop_snapshot(const LoopState *s, int n, const int32_t *labels
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += stride) snap_stats[c] = stats[c];
 }
 
-__global__ void k_loop_next(LoopState *s) {
-    if (!s->frozen) {
-        s->prev = s->cur;
-        s->prev_k = s->cur_k;
-        s->it++;
-    }
-    s->just = 0;
-}
+__global__ void k_loop_next(LoopState *s) { loop_next(s); }
 
 enum PassKind { PASS_PROPAGATE = 0, PASS_MERGE = 1 };
 
@@ -114,6 +68,7 @@ struct Loop {
     double frac = 0, threshold = 0;
     uint64_t seed = 0;
     int tie = 0, max_iter = 0, cap = 0, rounds = 0;
+    bool fused = false;   // the propagation pass is in its fused form: no copy is kept
     bool broken = false;  // capture failed once: this context runs pass by pass
 };
 
@@ -132,7 +87,8 @@ void loop_release(pcd_ctx *ctx) {
 
 // whether the captured passes of `kinds` (bit per PassKind) were captured
 // for these buffers, tuning, job and merging rounds
-static bool same_key(const Loop *L, pcd_ctx *ctx, const pcd_job *job, int cap, int rounds, unsigned kinds) {
+static bool same_key(const Loop *L, pcd_ctx *ctx, const pcd_job *job, int cap, int rounds, unsigned kinds, bool fused) {
+    if (L->fused != fused) return false;
     const void *p[4] = {ctx->d_labels, ctx->d_labels_alt, ctx->d_stats, ctx->d_stats_alt};
     for (int i = 0; i < 4; i++)
         if (p[i] != L->ptrs[i]) return false;
@@ -147,7 +103,7 @@ static bool same_key(const Loop *L, pcd_ctx *ctx, const pcd_job *job, int cap, i
 // Captures one pass of step kind `kind`.  Nothing runs: the host
 // bookkeeping is put back as it was after the capture.  Any failure leaves
 // no graph behind.
-static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int kind, int rounds) {
+static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int kind, int rounds, bool fused) {
     hipGraphExec_t &exec = L->exec[kind];
     if (exec) {
         (void)hipGraphExecDestroy(exec);
@@ -163,8 +119,8 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
         L->h_state = nullptr;
         return fail(PCD_E_NOMEM, "pinned loop state");
     }
-    if (!L->snap_labels) PCD_TRY(dev_alloc_t(ctx, &L->snap_labels, ctx->n + 1));
-    if (!L->snap_stats) PCD_TRY(dev_alloc_t(ctx, &L->snap_stats, ctx->n + 1));
+    if (!fused && !L->snap_labels) PCD_TRY(dev_alloc_t(ctx, &L->snap_labels, ctx->n + 1));
+    if (!fused && !L->snap_stats) PCD_TRY(dev_alloc_t(ctx, &L->snap_stats, ctx->n + 1));
     // host bookkeeping as it stands (a pass changes it while capturing)
     const bool s_timing = ctx->timing, s_counters = ctx->counters, s_comp = ctx->labels_compressed,
                s_has = ctx->has_stats, s_pend = ctx->stats_pending, s_new = ctx->labels_have_new,
@@ -179,9 +135,18 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
     PCD_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     ctx->capturing = true;
     ctx->graph_step = &L->d_state->step;
-    int rc = compress_labels_dev(ctx, true);
-    if (rc == PCD_OK) rc = metric_enqueue(ctx, rule);
-    if (rc == PCD_OK) {
+    int rc = PCD_OK;
+    if (fused) {
+        ctx->fused = L->d_state;
+        rc = fused_compress_dev(ctx, rule, lp, L->d_state);
+        if (rc == PCD_OK) rc = propagation_launch(ctx, rule, job->frac, job->seed, 0, job->tie);
+        if (rc == PCD_OK) rc = propagation_commit(ctx);
+        ctx->fused = nullptr;
+    } else {
+        rc = compress_labels_dev(ctx, true);
+        if (rc == PCD_OK) rc = metric_enqueue(ctx, rule);
+    }
+    if (rc == PCD_OK && !fused) {
         hipLaunchKernelGGL(k_loop_rule, dim3(1), dim3(1), 0, ctx->stream, L->d_state, ctx->d_result, ctx->d_k, lp);
         hipLaunchKernelGGL(k_loop_snapshot, dim3(grid_for(ctx, ctx->n + 1, 256, 8)), dim3(256), 0, ctx->stream,
                            L->d_state, ctx->n, ctx->d_labels, ctx->d_stats, L->snap_labels, L->snap_stats);
@@ -192,7 +157,7 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
             rc = merging_dev(ctx, rule, rounds, job->seed, 0, job->tie);
         }
     }
-    if (rc == PCD_OK) hipLaunchKernelGGL(k_loop_next, dim3(1), dim3(1), 0, ctx->stream, L->d_state);
+    if (rc == PCD_OK && !fused) hipLaunchKernelGGL(k_loop_next, dim3(1), dim3(1), 0, ctx->stream, L->d_state);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     ctx->capturing = false;
@@ -228,6 +193,7 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
     L->tie = job->tie;
     L->max_iter = job->max_iter;
     L->cap = cap;
+    L->fused = fused;
     if (kind == PASS_MERGE) L->rounds = rounds;
     return PCD_OK;
 }
@@ -243,6 +209,7 @@ static int device_passes(pcd_ctx *ctx, Loop *L, const pcd_job *job, int strategy
     h.prev = prev_score;
     h.prev_k = ctx->k;
     PCD_HIP(hipMemcpyAsync(L->d_state, &h, sizeof(LoopState), hipMemcpyHostToDevice, ctx->stream));
+    if (L->fused) PCD_TRY(fused_prepare(ctx));
     // replays per read of the record: about half a millisecond of passes
     // (one pass at a time for large graphs), never beyond the first pass
     // that can freeze
@@ -263,9 +230,10 @@ static int device_passes(pcd_ctx *ctx, Loop *L, const pcd_job *job, int strategy
         per = std::max(1, std::min(32, (int)(0.5 / std::max(pass_ms, 1e-3))));
     }
     // the labels and statistics of the frozen pass back in place
-    PCD_HIP(hipMemcpyAsync(ctx->d_labels, L->snap_labels, sizeof(int32_t) * (size_t)ctx->n, hipMemcpyDeviceToDevice,
+    if (!L->fused)
+      PCD_HIP(hipMemcpyAsync(ctx->d_labels, L->snap_labels, sizeof(int32_t) * (size_t)ctx->n, hipMemcpyDeviceToDevice,
                            ctx->stream));
-    if (h.k_freeze > 0)
+    if (!L->fused && h.k_freeze > 0)
         PCD_HIP(hipMemcpyAsync(ctx->d_stats, L->snap_stats, sizeof(CommStats) * (size_t)h.k_freeze,
                                hipMemcpyDeviceToDevice, ctx->stream));
     PCD_HIP(hipStreamSynchronize(ctx->stream));
@@ -362,12 +330,14 @@ extern "C" int pcd_iterate_many(pcd_ctx *ctx, const pcd_job *job, int strategy, 
     PCD_HIP(hipSetDevice(ctx->device));
     if (!ctx->loop) ctx->loop = new Loop();
     Loop *L = loop_of(ctx);
-    if (!same_key(L, ctx, job, cap, rounds, kinds)) {
+    const bool fused = strategy == 0 && ctx->tune.fused_pass &&
+                       (job->rule.kind == PCD_RULE_MODULARITY || job->rule.kind == PCD_RULE_CPM);
+    if (!same_key(L, ctx, job, cap, rounds, kinds, fused)) {
         // everything a captured merging step uses is allocated first, so
         // that neither capture allocates
         int rc = (kinds & 2u) ? merge_rows_reserve(ctx) : PCD_OK;
         for (int kd = 0; kd < 2 && rc == PCD_OK; kd++)
-            if ((kinds >> kd) & 1u) rc = capture_pass(ctx, L, job, cap, kd, rounds);
+            if ((kinds >> kd) & 1u) rc = capture_pass(ctx, L, job, cap, kd, rounds, fused);
         if (rc != PCD_OK) {
             // this context runs pass by pass from now on
             L->broken = true;

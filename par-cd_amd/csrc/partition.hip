@@ -161,6 +161,133 @@ int compress_labels_dev(pcd_ctx *ctx, bool defer_k) {
     return PCD_OK;
 }
 
+// ------------------------------------------------------------ the fused pass
+// The numbering of first occurrences in one launch: every workgroup counts the
+// first occurrences of all vertices before its tile itself, which for n up to
+// DIRECT_N vertices costs less than the two launches and their gaps that a scan
+// of tile sums takes (n = 10,000: 3 us instead of 9).
+constexpr int DIRECT_N = 1 << 16, NUMBER_NT = 1024;
+__global__ __launch_bounds__(NUMBER_NT) void k_number_direct(int n, FirstFlag flag, FirstStore store, int32_t *total) {
+    __shared__ int lds[NUMBER_NT / WAVE];
+    const int tile = blockIdx.x * NUMBER_NT;
+    int before = 0;
+#pragma unroll 4
+    for (int v = threadIdx.x; v < tile; v += NUMBER_NT) before += flag(v);
+    int run;
+    block_excl_scan_n<NUMBER_NT>(before, &run, lds);
+    const int v = tile + threadIdx.x;
+    const int x = v < n ? flag(v) : 0;
+    int tot;
+    const int ex = block_excl_scan_n<NUMBER_NT>(x, &tot, lds);
+    if (v < n) store(v, run + ex, x);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = run + tot;
+}
+
+// What follows the numbering, elementwise: the new labels (into both label
+// buffers: the step's result starts as a copy), the records back in place,
+// the total each gain reads, and the metric's sums; the workgroup that adds
+// its sums last scores the partition and applies the stop rule.
+struct PassTail {
+    int n, m, kind;
+    double lambda;
+    const int32_t *total;  // k
+    const int32_t *newid;
+    int32_t *labels;       // before the compression; the copy
+    int32_t *out;          // compressed
+    const CommStats *st_in;
+    CommStats *st;
+    int32_t *tot, *dk;
+    unsigned long long *acc;  // zero between passes
+    LoopState *state;
+    LoopParams rule;
+};
+constexpr int TAIL_NT = 512;
+__global__ __launch_bounds__(TAIL_NT) void k_pass_tail(PassTail a) {
+    __shared__ long long lds[3][TAIL_NT / WAVE];
+    const int k = *a.total;
+    const int stride = gridDim.x * TAIL_NT, t0 = blockIdx.x * TAIL_NT + threadIdx.x;
+    long long s0 = 0, s1 = 0, s2 = 0;
+    for (int c = t0; c < k; c += stride) {
+        const CommStats r = a.st_in[c];
+        const int v = r.int_vol + r.ext_vol;
+        a.st[c] = r;
+        a.tot[c] = a.kind == PCD_RULE_MODULARITY ? v : r.size;
+        const long long vol = (long long)r.int_vol + r.ext_vol;
+        s0 += r.int_vol;
+        s1 += vol * vol;
+        s2 += (long long)r.size * (r.size - 1);
+    }
+    for (int v = t0; v < a.n; v += stride) {
+        const int l = a.labels[v];
+        const int x = l < 0 ? a.out[v] : a.newid[l];
+        a.out[v] = x;
+        a.labels[v] = x;
+    }
+    s0 = wave_sum64(s0);
+    s1 = wave_sum64(s1);
+    s2 = wave_sum64(s2);
+    const int w = threadIdx.x / WAVE;
+    if (__lane_id() == 0) {
+        lds[0][w] = s0;
+        lds[1][w] = s1;
+        lds[2][w] = s2;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int i = 1; i < TAIL_NT / WAVE; i++) {
+        s0 += lds[0][i];
+        s1 += lds[1][i];
+        s2 += lds[2][i];
+    }
+    atomicAdd(&a.acc[0], (unsigned long long)s0);
+    atomicAdd(&a.acc[1], (unsigned long long)s1);
+    atomicAdd(&a.acc[2], (unsigned long long)s2);
+    __threadfence();
+    if (atomicAdd(&a.state->arrived, 1) != (int)gridDim.x - 1) return;
+    __threadfence();
+    // atomics read what the others added, and leave zeros for the next pass
+    const long long x0 = (long long)atomicExch(&a.acc[0], 0ULL), x1 = (long long)atomicExch(&a.acc[1], 0ULL),
+                    x2 = (long long)atomicExch(&a.acc[2], 0ULL);
+    a.state->arrived = 0;
+    *a.dk = k;
+    loop_rule(a.state, score_of_sums(x0, x1, x2, a.kind, a.lambda, a.m), k, a.rule);
+}
+
+int fused_prepare(pcd_ctx *ctx) {
+    if (ctx->label_bound > 0)
+        hipLaunchKernelGGL(k_first_init, dim3(grid_for(ctx, ctx->label_bound, 256)), dim3(256), 0, ctx->stream,
+                           ctx->label_bound, ctx->d_labels, ctx->d_firstv, ctx->d_first);
+    PCD_TRY(fill_u64(ctx, (uint64_t *)ctx->d_acc, 0, 4));
+    PCD_HIP(hipGetLastError());
+    return PCD_OK;
+}
+
+int fused_compress_dev(pcd_ctx *ctx, pcd_rule rule, const LoopParams &p, LoopState *state) {
+    const int n = ctx->n;
+    hipLaunchKernelGGL(k_first_occurrence, dim3(grid_for(ctx, n, FO_NT * 4, 4)), dim3(FO_NT), 0, ctx->stream, n,
+                       ctx->d_labels, ctx->d_first);
+    const FirstFlag flag{ctx->d_labels, ctx->d_first};
+    const FirstStore store{ctx->d_labels, ctx->d_labels_alt, ctx->d_newid, ctx->d_stats,
+                           ctx->d_stats_alt, ctx->d_indices, ctx->d_firstv};
+    int32_t *total = ctx->d_scan_part;
+    if (n <= DIRECT_N)
+        hipLaunchKernelGGL(k_number_direct, dim3((n + NUMBER_NT - 1) / NUMBER_NT), dim3(NUMBER_NT), 0, ctx->stream, n,
+                           flag, store, total);
+    else
+        PCD_TRY(device_scan(ctx, n, flag, store, &total));
+    const PassTail t{n, ctx->m, rule.kind, rule.lambda, total, ctx->d_newid, ctx->d_labels, ctx->d_labels_alt,
+                     ctx->d_stats_alt, ctx->d_stats, ctx->d_tot, ctx->d_k, (unsigned long long *)ctx->d_acc, state, p};
+    // up to two workgroups per CU: each adds its sums with three atomics
+    hipLaunchKernelGGL(k_pass_tail, dim3(grid_for(ctx, n, TAIL_NT, 2)), dim3(TAIL_NT), 0, ctx->stream, t);
+    PCD_HIP(hipGetLastError());
+    std::swap(ctx->d_labels, ctx->d_labels_alt);
+    ctx->k_deferred = true;
+    ctx->labels_compressed = true;
+    ctx->has_stats = true;
+    ctx->stats_pending = false;
+    return PCD_OK;
+}
+
 // ------------------------------------------------------------ statistics
 // framework.cpp:69-143: per vertex, count neighbours with the same label;
 // sizes[l] += 1, int_volume[l] += same, ext_volume[l] += deg - same.
@@ -358,7 +485,17 @@ struct MovedStore {
 
 // Moved bitmap: bit v of M is set when vertex v's label changed in the step
 // (L[v] != N[v]).  One wave writes one 64-bit word.
-__global__ __launch_bounds__(256) void k_moved_bits(int n, const int32_t *L, const int32_t *N, uint64_t *M) {
+// With dk set (a captured pass) it also starts the next compression's
+// first-occurrence table, as k_first_init does.
+__global__ __launch_bounds__(256) void k_moved_bits(int n, const int32_t *L, const int32_t *N, uint64_t *M,
+                                                    const int32_t *dk, const int32_t *firstv, int32_t *first) {
+    if (dk) {
+        const int k = *dk;
+        for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += gridDim.x * blockDim.x) {
+            const int w = firstv[c];
+            first[c] = N[w] == c ? w : INT32_MAX;
+        }
+    }
     const int lane = __lane_id();
     const int nwords = (n + WAVE - 1) / WAVE;
     const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
@@ -370,82 +507,124 @@ __global__ __launch_bounds__(256) void k_moved_bits(int n, const int32_t *L, con
     }
 }
 
-// A neighbour's label before the step: its label after the step (already
+// A neighbour's label before the step is its label after the step (already
 // gathered) unless the bitmap says it moved, so unmoved neighbours cost one
 // random gather instead of two (the bitmap itself stays in L2).
-__device__ inline int label_before(const uint64_t *M, const int32_t *L, int w, int after) {
-    return ((M[w >> 6] >> (w & 63)) & 1) ? L[w] : after;
-}
 
-// Moved vertices of one small bin, G lanes each.  A wave takes up to
-// DELTA_BATCH entries of the list at once, one lane each, loads their rows
-// and labels together, and then runs through them two groups of 64 / G at a
-// time: what bounds it is the chain of dependent loads per row, which this
-// shortens from five to two for two rows.
+// Moved vertices of one small bin, G lanes each.  The first `left` lanes hold
+// one vertex's row and labels each; the wave runs through them two groups of
+// 64 / G at a time.  What bounds it is the chain of dependent loads per row,
+// which this shortens from five to two for two rows.
 constexpr int DELTA_BATCH = 16, DELTA_LOG = 7;
+struct DeltaArgs {
+    const int32_t *indices, *adj, *L, *N;
+    const uint64_t *M;  // moved bitmap, or nullptr: L is read for every neighbour
+    CommStats *st;
+};
+__device__ inline int label_before(const DeltaArgs &a, int w, int after) {
+    return !a.M || ((a.M[w >> 6] >> (w & 63)) & 1) ? a.L[w] : after;
+}
 template <int G>
-__device__ inline void delta_small(int wave_g, int nwaves, const int32_t *list, int cnt, const int32_t *indices, const int32_t *adj, const int32_t *L, const int32_t *N,
-                                   const HotLabels &after, const uint64_t *M, CommStats *st,
+__device__ inline void delta_batch(const DeltaArgs &d, int left, int v, const HotLabels &after,
                                    StatsAcc<DELTA_LOG> &acc) {
     const int lane = __lane_id(), glane = lane & (G - 1);
     constexpr int per_wave = WAVE / G;
+    int bstart = 0, bdeg = 0, blo = 0, bln = 0;
+    if (lane < left) {
+        blo = d.L[v];
+        bln = d.N[v];
+        bstart = d.indices[v];
+        bdeg = d.indices[v + 1] - bstart;
+    }
+    for (int g0 = 0; g0 < left; g0 += 2 * per_wave) {
+        int deg[2], lo[2], ln[2], w[2], nw[2], lw[2], a[2], b[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int gi = g0 + t * per_wave + lane / G;
+            const int src = gi < left ? gi : 0;
+            const int start = __shfl(bstart, src, WAVE);
+            deg[t] = __shfl(bdeg, src, WAVE);
+            lo[t] = __shfl(blo, src, WAVE);
+            ln[t] = __shfl(bln, src, WAVE);
+            if (gi >= left) deg[t] = 0;
+            w[t] = glane < deg[t] ? d.adj[start + glane] : -1;  // a row of the bin has at most G entries
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++) nw[t] = w[t] < 0 ? -2 : after(w[t]);
+#pragma unroll
+        for (int t = 0; t < 2; t++) lw[t] = w[t] < 0 ? -2 : label_before(d, w[t], nw[t]);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int f = lw[t] != nw[t] ? 1 : 2;
+            a[t] = w[t] >= 0 && lw[t] == lo[t] ? f : 0;
+            b[t] = w[t] >= 0 && nw[t] == ln[t] ? f : 0;
+#pragma unroll
+            for (int x = G / 2; x > 0; x >>= 1) {
+                a[t] += __shfl_xor(a[t], x, WAVE);
+                b[t] += __shfl_xor(b[t], x, WAVE);
+            }
+            if (g0 + t * per_wave + lane / G < left && glane == 0) {
+                acc.add(d.st, lo[t], -1, -a[t], a[t] - deg[t]);
+                if (ln[t] >= 0) acc.add(d.st, ln[t], 1, b[t], deg[t] - b[t]);
+            }
+        }
+    }
+}
+// a wave takes up to DELTA_BATCH entries of the bin's list at once
+template <int G>
+__device__ inline void delta_small(const DeltaArgs &d, int wave_g, int nwaves, const int32_t *list, int cnt,
+                                   const HotLabels &after, StatsAcc<DELTA_LOG> &acc) {
+    constexpr int per_wave = WAVE / G;
+    const int lane = __lane_id();
     // entries per batch: a multiple of per_wave that leaves no wave idle
     const int share = (cnt + nwaves - 1) / nwaves;
     const int batch = min(max(per_wave, DELTA_BATCH), (share + per_wave - 1) / per_wave * per_wave);
     for (int base = wave_g * batch; base < cnt; base += nwaves * batch) {
         const int left = min(batch, cnt - base);
-        int bstart = 0, bdeg = 0, blo = 0, bln = 0;
-        if (lane < left) {
-            const int v = list[base + lane];
-            blo = L[v];
-            bln = N[v];
-            bstart = indices[v];
-            bdeg = indices[v + 1] - bstart;
-        }
-        for (int g0 = 0; g0 < left; g0 += 2 * per_wave) {
-            int deg[2], lo[2], ln[2], w[2], nw[2], lw[2], a[2], b[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int gi = g0 + t * per_wave + lane / G;
-                const int src = gi < left ? gi : 0;
-                const int start = __shfl(bstart, src, WAVE);
-                deg[t] = __shfl(bdeg, src, WAVE);
-                lo[t] = __shfl(blo, src, WAVE);
-                ln[t] = __shfl(bln, src, WAVE);
-                if (gi >= left) deg[t] = 0;
-                w[t] = glane < deg[t] ? adj[start + glane] : -1;  // a row of the bin has at most G entries
-            }
-#pragma unroll
-            for (int t = 0; t < 2; t++) nw[t] = w[t] < 0 ? -2 : after(w[t]);
-#pragma unroll
-            for (int t = 0; t < 2; t++) lw[t] = w[t] < 0 ? -2 : label_before(M, L, w[t], nw[t]);
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int f = lw[t] != nw[t] ? 1 : 2;
-                a[t] = w[t] >= 0 && lw[t] == lo[t] ? f : 0;
-                b[t] = w[t] >= 0 && nw[t] == ln[t] ? f : 0;
-#pragma unroll
-                for (int d = G / 2; d > 0; d >>= 1) {
-                    a[t] += __shfl_xor(a[t], d, WAVE);
-                    b[t] += __shfl_xor(b[t], d, WAVE);
-                }
-                if (g0 + t * per_wave + lane / G < left && glane == 0) {
-                    acc.add(st, lo[t], -1, -a[t], a[t] - deg[t]);
-                    if (ln[t] >= 0) acc.add(st, ln[t], 1, b[t], deg[t] - b[t]);
-                }
-            }
-        }
+        delta_batch<G>(d, left, lane < left ? list[base + lane] : 0, after, acc);
     }
 }
 
-// Moved items {v, begin, end, first} (rows longer than 64), one wave each:
-// workgroup b of nb takes list entries b, b + nb, ..., its waves whichever
-// comes next (rows differ 30-fold in length), and the next item's records are
-// on their way while one is counted.
-__device__ inline void delta_items(int wg, int nwg, int *next, const int32_t *list, int cnt, const int4 *items,
-                                   const int32_t *adj, const int32_t *L, const int32_t *N, const HotLabels &after,
-                                   const uint64_t *M, CommStats *st, StatsAcc<DELTA_LOG> &acc) {
+// One long-row item {v, begin, end, first} of a moved vertex, the whole wave
+__device__ inline void delta_item(const DeltaArgs &d, const int4 &w, int lo, int ln, const HotLabels &after,
+                                  StatsAcc<DELTA_LOG> &acc) {
     constexpr int PF = 8;
+    const int lane = __lane_id();
+    int a = 0, b = 0;
+    for (int j0 = w.y + lane; j0 < w.z; j0 += PF * WAVE) {
+        int nb[PF];
+#pragma unroll
+        for (int e = 0; e < PF; e++) {
+            const int j = j0 + e * WAVE;
+            nb[e] = j < w.z ? d.adj[j] : -1;
+        }
+        int lw[PF], nw[PF];
+#pragma unroll
+        for (int e = 0; e < PF; e++) nw[e] = nb[e] < 0 ? -2 : after(nb[e]);
+#pragma unroll
+        for (int e = 0; e < PF; e++) lw[e] = nb[e] < 0 ? -2 : label_before(d, nb[e], nw[e]);
+#pragma unroll
+        for (int e = 0; e < PF; e++) {
+            if (nb[e] < 0) continue;
+            const int f = lw[e] != nw[e] ? 1 : 2;
+            a += lw[e] == lo ? f : 0;
+            b += nw[e] == ln ? f : 0;
+        }
+    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (lane == 0) {
+        const int len = w.z - w.y;
+        acc.add(d.st, lo, w.w ? -1 : 0, -a, a - len);
+        if (ln >= 0) acc.add(d.st, ln, w.w ? 1 : 0, b, len - b);
+    }
+}
+
+// Moved items, one wave each: workgroup wg of nwg takes list entries wg,
+// wg + nwg, ..., its waves whichever comes next (rows differ 30-fold in
+// length), and the next item's records are on their way while one is counted.
+__device__ inline void delta_items(const DeltaArgs &d, int wg, int nwg, int *next, const int32_t *list, int cnt,
+                                   const int4 *items, const HotLabels &after, StatsAcc<DELTA_LOG> &acc) {
     const int lane = __lane_id();
     int4 wn = make_int4(0, 0, 0, 0);
     int lon = 0, lnn = 0;
@@ -456,8 +635,8 @@ __device__ inline void delta_items(int wg, int nwg, int *next, const int32_t *li
         const int64_t i = wg + (int64_t)j * nwg;
         if (i >= cnt) return false;
         wn = items[list[i]];
-        lon = L[wn.x];
-        lnn = N[wn.x];
+        lon = d.L[wn.x];
+        lnn = d.N[wn.x];
         return true;
     };
     bool more = fetch();
@@ -465,34 +644,7 @@ __device__ inline void delta_items(int wg, int nwg, int *next, const int32_t *li
         const int4 w = wn;
         const int lo = lon, ln = lnn;
         more = fetch();
-        int a = 0, b = 0;
-        for (int j0 = w.y + lane; j0 < w.z; j0 += PF * WAVE) {
-            int nb[PF];
-#pragma unroll
-            for (int e = 0; e < PF; e++) {
-                const int j = j0 + e * WAVE;
-                nb[e] = j < w.z ? adj[j] : -1;
-            }
-            int lw[PF], nw[PF];
-#pragma unroll
-            for (int e = 0; e < PF; e++) nw[e] = nb[e] < 0 ? -2 : after(nb[e]);
-#pragma unroll
-            for (int e = 0; e < PF; e++) lw[e] = nb[e] < 0 ? -2 : label_before(M, L, nb[e], nw[e]);
-#pragma unroll
-            for (int e = 0; e < PF; e++) {
-                if (nb[e] < 0) continue;
-                const int f = lw[e] != nw[e] ? 1 : 2;
-                a += lw[e] == lo ? f : 0;
-                b += nw[e] == ln ? f : 0;
-            }
-        }
-        a = wave_sum(a);
-        b = wave_sum(b);
-        if (lane == 0) {
-            const int len = w.z - w.y;
-            acc.add(st, lo, w.w ? -1 : 0, -a, a - len);
-            if (ln >= 0) acc.add(st, ln, w.w ? 1 : 0, b, len - b);
-        }
+        delta_item(d, w, lo, ln, after, acc);
     }
 }
 
@@ -506,21 +658,21 @@ __device__ inline void delta_items(int wg, int nwg, int *next, const int32_t *li
 // vertices move (24 us at twice as many, 12 us here), because every
 // workgroup pays the accumulators' start and flush.
 constexpr int DELTA_NT = 1024, DELTA_HOT_ITEMS = 2;
-__global__ __launch_bounds__(DELTA_NT) void k_delta_all(int n, const int32_t *list, const int32_t *bounds, const int4 *items,
-                                                        const int32_t *indices, const int32_t *adj, const int32_t *L,
-                                                        const int32_t *N, const uint64_t *M, CommStats *st) {
+__global__ __launch_bounds__(DELTA_NT) void k_delta_all(int n, const int32_t *list, const int32_t *bounds,
+                                                        const int4 *items, DeltaArgs d, LoopState *state) {
+    if (state && blockIdx.x == 0 && threadIdx.x == 0) loop_next(state);  // a captured pass ends here
     int bd[7];  // read at once: a read per list would lengthen every wave's chain
 #pragma unroll
     for (int i = 0; i < 7; i++) bd[i] = bounds[i];
     if (bd[0] == bd[6]) return;  // nothing moved
     __shared__ int32_t hot[STATS_CACHE];
     __shared__ StatsAcc<DELTA_LOG> acc;
+    __shared__ int next;
     const int nwaves = gridDim.x * DELTA_NT / WAVE;
     // with several long-row items a wave, the labels of the most frequent
     // neighbours are staged in LDS (as in k_stats_rows)
-    const HotLabels after{hot, N, bd[6] - bd[5] >= DELTA_HOT_ITEMS * nwaves ? min(n, STATS_CACHE) : 0};
-    for (int i = threadIdx.x; i < after.n; i += DELTA_NT) hot[i] = N[i];
-    __shared__ int next;
+    const HotLabels after{hot, d.N, bd[6] - bd[5] >= DELTA_HOT_ITEMS * nwaves ? min(n, STATS_CACHE) : 0};
+    for (int i = threadIdx.x; i < after.n; i += DELTA_NT) hot[i] = d.N[i];
     if (threadIdx.x == 0) next = 0;
     acc.init();
     __syncthreads();
@@ -529,14 +681,74 @@ __global__ __launch_bounds__(DELTA_NT) void k_delta_all(int n, const int32_t *li
         const int w = wave_g + i * (nwaves / 6);
         return w < nwaves ? w : w - nwaves;
     };
-    delta_items(blockIdx.x, gridDim.x, &next, list + bd[5], bd[6] - bd[5], items, adj, L, N, after, M, st, acc);
-    delta_small<64>(place(1), nwaves, list + bd[0], bd[1] - bd[0], indices, adj, L, N, after, M, st, acc);
-    delta_small<32>(place(2), nwaves, list + bd[1], bd[2] - bd[1], indices, adj, L, N, after, M, st, acc);
-    delta_small<16>(place(3), nwaves, list + bd[2], bd[3] - bd[2], indices, adj, L, N, after, M, st, acc);
-    delta_small<8>(place(4), nwaves, list + bd[3], bd[4] - bd[3], indices, adj, L, N, after, M, st, acc);
-    delta_small<4>(place(5), nwaves, list + bd[4], bd[5] - bd[4], indices, adj, L, N, after, M, st, acc);
+    delta_items(d, blockIdx.x, gridDim.x, &next, list + bd[5], bd[6] - bd[5], items, after, acc);
+    delta_small<64>(d, place(1), nwaves, list + bd[0], bd[1] - bd[0], after, acc);
+    delta_small<32>(d, place(2), nwaves, list + bd[1], bd[2] - bd[1], after, acc);
+    delta_small<16>(d, place(3), nwaves, list + bd[2], bd[3] - bd[2], after, acc);
+    delta_small<8>(d, place(4), nwaves, list + bd[3], bd[4] - bd[3], after, acc);
+    delta_small<4>(d, place(5), nwaves, list + bd[4], bd[5] - bd[4], after, acc);
     __syncthreads();
-    acc.flush(st);
+    acc.flush(d.st);
+}
+
+// The same without lists, in one launch, for graphs whose rows are looked at
+// sooner than the lists are made: a wave takes 64 positions of a small bin at
+// a time and runs through the moved ones, then its share of the items.  Also
+// starts the next compression's first-occurrence table (see k_first_init) and
+// closes a captured pass.
+constexpr int DIRECT_MAX_N = 1 << 16, DIRECT_NT = 512;
+template <int G>
+__device__ inline void delta_positions(const DeltaArgs &d, const MovedArgs &m, int b, int wave_g, int nwaves,
+                                       const HotLabels &after, int *list, StatsAcc<DELTA_LOG> &acc) {
+    const int lane = __lane_id();
+    // no wider than the bin leaves every wave busy
+    const int count = m.s[b + 1] - m.s[b];
+    const int share = min(WAVE, max(2 * WAVE / G, (count + nwaves - 1) / nwaves));
+    for (int base = wave_g * share; base < count; base += nwaves * share) {
+        const int p = m.s[b] + base + lane;
+        const bool in = lane < share && base + lane < count;
+        const int v = in ? (m.order ? m.order[p] : p) : 0;
+        const bool moved = in && d.L[v] != d.N[v];
+        const uint64_t mm = __ballot(moved);
+        if (!mm) continue;
+        if (moved) list[__popcll(mm & ((1ULL << lane) - 1))] = v;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int left = __popcll(mm);
+        delta_batch<G>(d, left, lane < left ? list[lane] : 0, after, acc);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+__global__ __launch_bounds__(DIRECT_NT) void k_delta_direct(MovedArgs m, DeltaArgs d, const int32_t *dk,
+                                                            const int32_t *firstv, int32_t *first, LoopState *state) {
+    __shared__ int s_list[DIRECT_NT / WAVE][WAVE];
+    __shared__ StatsAcc<DELTA_LOG> acc;
+    if (blockIdx.x == 0 && threadIdx.x == 0) loop_next(state);
+    const int k = *dk;
+    for (int c = blockIdx.x * DIRECT_NT + threadIdx.x; c < k; c += gridDim.x * DIRECT_NT) {
+        const int w = firstv[c];
+        first[c] = d.N[w] == c ? w : INT32_MAX;
+    }
+    acc.init();
+    __syncthreads();
+    const int lane = __lane_id(), w = threadIdx.x / WAVE;
+    const int nwaves = gridDim.x * DIRECT_NT / WAVE, wave_g = blockIdx.x * DIRECT_NT / WAVE + w;
+    auto place = [&](int i) { return (wave_g + i * (nwaves / 6)) % nwaves; };
+    const HotLabels after{s_list[w], d.N, 0};
+    for (int i = wave_g; i < m.nitems; i += nwaves) {
+        const int4 it = m.items[i];
+        const int lo = d.L[it.x], ln = d.N[it.x];
+        if (lo != ln) delta_item(d, it, lo, ln, after, acc);
+    }
+    delta_positions<64>(d, m, 0, place(1), nwaves, after, s_list[w], acc);
+    delta_positions<32>(d, m, 1, place(2), nwaves, after, s_list[w], acc);
+    delta_positions<16>(d, m, 2, place(3), nwaves, after, s_list[w], acc);
+    delta_positions<8>(d, m, 3, place(4), nwaves, after, s_list[w], acc);
+    delta_positions<4>(d, m, 4, place(5), nwaves, after, s_list[w], acc);
+    (void)lane;
+    __syncthreads();
+    acc.flush(d.st);
 }
 
 int statistics_delta_dev(pcd_ctx *ctx, const int32_t *before, const int32_t *after) {
@@ -549,17 +761,28 @@ int statistics_delta_dev(pcd_ctx *ctx, const int32_t *before, const int32_t *aft
     m.items = ctx->d_stat_items;
     m.L = before;
     m.N = after;
+    const DeltaArgs d{ctx->d_indices, ctx->d_adj, before, after, ctx->d_moved_bits, ctx->d_stats};
+    if (ctx->fused && ctx->n <= DIRECT_MAX_N) {
+        DeltaArgs dd = d;
+        dd.M = nullptr;
+        const int64_t rows = std::max<int64_t>(m.s[5] - m.s[0], (int64_t)m.nitems * 16);
+        hipLaunchKernelGGL(k_delta_direct, dim3(grid_for(ctx, rows, 64, 4)), dim3(DIRECT_NT), 0, ctx->stream, m, dd,
+                           ctx->d_k, ctx->d_firstv, ctx->d_first, ctx->fused);
+        kt_end(ctx, KS_STATS_DELTA);
+        PCD_HIP(hipGetLastError());
+        return PCD_OK;
+    }
     int32_t *bounds = ctx->d_moved;
     int32_t *list = ctx->d_moved + 8;
     const int64_t len = (int64_t)(m.s[5] - m.s[0]) + m.nitems + 1;
     PCD_TRY(device_scan(ctx, len, MovedFlag{m}, MovedStore{m, bounds, list}, nullptr));
-    uint64_t *M = ctx->d_moved_bits;
     hipLaunchKernelGGL(k_moved_bits, dim3(grid_for(ctx, (ctx->n + WAVE - 1) / WAVE, 4, 8)), dim3(256), 0, ctx->stream,
-                       ctx->n, before, after, M);
+                       ctx->n, before, after, ctx->d_moved_bits, ctx->fused ? ctx->d_k : nullptr, ctx->d_firstv,
+                       ctx->d_first);
     // two workgroups per CU, fewer for a small graph
     const int delta_grid = std::max(8, grid_for(ctx, 2 * (int64_t)ctx->m, 2048, 2));
     hipLaunchKernelGGL(k_delta_all, dim3(delta_grid), dim3(DELTA_NT), 0, ctx->stream, ctx->n, list, bounds,
-                       ctx->d_stat_items, ctx->d_indices, ctx->d_adj, before, after, M, ctx->d_stats);
+                       ctx->d_stat_items, d, ctx->fused);
     kt_end(ctx, KS_STATS_DELTA);
     PCD_HIP(hipGetLastError());
     return PCD_OK;

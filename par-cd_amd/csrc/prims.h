@@ -87,6 +87,43 @@ __device__ inline double score_of_sums(long long a, long long b, long long c, in
     return (a - lambda * (double)c) / (double)(2 * m);
 }
 
+// main.cpp:241-242, -n and the iteration cap for the pass the state stands at
+__device__ inline void loop_rule(LoopState *s, double sc, int k, const LoopParams &p) {
+    if (s->frozen) return;
+    const int it = s->it;
+    if (it >= s->it_end) {
+        s->frozen = 1;
+        s->just = 1;
+        s->k_freeze = k;
+        s->step = -1;
+        return;
+    }
+    const bool known = (p.max_iter != -1 && it >= p.max_iter) || it >= p.cap;
+    const bool d = known || (p.max_iter == -1 && s->prev > 0 && sc > 0 && sc / s->prev - 1 <= p.threshold);
+    s->cur = sc;
+    s->cur_k = k;
+    if (d) {
+        s->frozen = 1;
+        s->done = 1;
+        s->just = 1;
+        s->k_freeze = k;
+        s->score_done = sc;
+        s->step = -1;
+    } else {
+        s->step = it;
+    }
+}
+
+// closes the pass
+__device__ inline void loop_next(LoopState *s) {
+    if (!s->frozen) {
+        s->prev = s->cur;
+        s->prev_k = s->cur_k;
+        s->it++;
+    }
+    s->just = 0;
+}
+
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ROUNDS = 16;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ROUNDS;

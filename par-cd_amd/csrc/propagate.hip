@@ -571,7 +571,7 @@ static int launch_propagation(pcd_ctx *ctx, const RowSet &rs, const LPArgs &a) {
     // inactive vertices keep their label: copy all, the kernels overwrite the
     // active ones (a merging round writes the partners of active communities
     // into the partner array, which keeps the others)
-    if (!MERGE)
+    if (!MERGE && !ctx->fused)  // a fused pass has made the copy and the totals below
         PCD_HIP(hipMemcpyAsync(a.new_labels, a.labels, sizeof(int32_t) * (size_t)ctx->n, hipMemcpyDeviceToDevice,
                                ctx->stream));
     const bool small_aux = a.use_aux && ctx->tune.small_aux;
@@ -586,7 +586,7 @@ static int launch_propagation(pcd_ctx *ctx, const RowSet &rs, const LPArgs &a) {
                            ctx->d_labels, ctx->d_stats, a.rule.kind, ctx->d_lv);
         kt_end(ctx, KS_LP_SELECT);
     }
-    if (a.use_aux) {  // the modularity and CPM builds read the totals
+    if (a.use_aux && !ctx->fused) {  // the modularity and CPM builds read the totals
         kt_begin(ctx, KS_LP_SELECT);
         // k is read from d_k (a deferred k is bounded by n + 1)
         const int kg = ctx->k_deferred ? ctx->n + 1 : ctx->k;

@@ -139,8 +139,9 @@ def test_small_graph_loop(ctx, name):
                                                 (O.MOD, 0.0, 1, 0.8)]):
         lab = starts[i % 2].astype(np.int32)
         got = []
-        for solo, graph in ((1, 1), (0, 1), (0, 0)):
+        for solo, fused, graph in ((1, 1, 1), (0, 1, 1), (0, 0, 1), (0, 0, 0)):
             ctx.set_tuning("solo_loop", solo)
+            ctx.set_tuning("fused_pass", fused)
             ctx.set_tuning("graph_loop", graph)
             one = []
             for job in (parcd.job(kind=kind, lam=lam, frac=frac, tie=tie, seed=5, iter_cap=40),
@@ -158,9 +159,45 @@ def test_small_graph_loop(ctx, name):
                 one += [prev, k]
             one += [ctx.iterate(job, at, prev)[0], ctx.compress(), ctx.labels()]
             got.append(one)
-        ctx.set_tuning("solo_loop", 1)
-        ctx.set_tuning("graph_loop", 1)
+        for key in ("solo_loop", "fused_pass", "graph_loop"):
+            ctx.set_tuning(key, 1)
         for other in got[1:]:
             assert len(other) == len(got[0])
             for x, y in zip(got[0], other):
                 assert np.array_equal(x, y, equal_nan=True) if isinstance(x, float) else np.array_equal(x, y), (name, i)
+
+
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 65535, 65536, 65537])
+def test_fused_pass_sizes(ctx, n):
+    """Sizes at the edges of the numbering's tiles and of the direct forms:
+    every vertex on a ring with chords (degrees 2-40 and one hub), modularity
+    and CPM with leaving vertices, equal pass by pass."""
+    rng = np.random.default_rng(n)
+    a = np.arange(n)
+    u, v = np.concatenate([a, rng.integers(0, n, 3 * n), np.zeros(min(n - 1, 6000), int)]), \
+        np.concatenate([(a + 1) % n, rng.integers(0, n, 3 * n), np.arange(1, min(n, 6001))])
+    g = GG.csr_from_edges(u, v)
+    assert g[0] == n
+    ctx.upload_graph(*g[:4])
+    lab = rng.integers(0, n, n).astype(np.int32)
+    for kind, lam, tie in ((O.MOD, 0.0, 0), (O.CPM, 0.4, 1)):
+        got = []
+        for fused, graph in ((1, 1), (0, 1), (0, 0)):
+            ctx.set_tuning("solo_loop", 0)
+            ctx.set_tuning("fused_pass", fused)
+            ctx.set_tuning("graph_loop", graph)
+            ctx.upload_labels(lab)
+            one = list(ctx.refine(parcd.job(kind=kind, lam=lam, tie=tie, seed=3, max_iter=9)))
+            one += [ctx.labels()] + list(ctx.stats(one[2]))
+            ctx.upload_labels(lab)  # the captured pass again, stopped by its range
+            at, prev = 0, 0.0
+            for count in (4, 3):
+                p, prev, k, done = ctx.iterate_many(parcd.job(kind=kind, lam=lam, tie=tie, seed=3, max_iter=90), at,
+                                                    count, prev)
+                at += p
+                one += [prev, k]
+            got.append(one + [ctx.compress(), ctx.labels()])
+        for key in ("solo_loop", "fused_pass", "graph_loop"):
+            ctx.set_tuning(key, 1)
+        for other in got[1:]:
+            assert all(np.array_equal(x, y) for x, y in zip(got[0], other)), (n, kind)
