@@ -171,7 +171,7 @@ __global__ __launch_bounds__(NUMBER_NT) void k_number_direct(int n, FirstFlag fl
     __shared__ int lds[NUMBER_NT / WAVE];
     const int tile = blockIdx.x * NUMBER_NT;
     int before = 0;
-#pragma unroll 4
+#pragma unroll 8
     for (int v = threadIdx.x; v < tile; v += NUMBER_NT) before += flag(v);
     int run;
     block_excl_scan_n<NUMBER_NT>(before, &run, lds);
