@@ -17,7 +17,7 @@
 //  * community rows (the default): as refinement.cpp:222-238 states it,
 //    each community counts the labels of its members' neighbours.  Once per
 //    step every entry's label is gathered into its community's row (rows in
-//    label order, members by a stable radix sort of the vertices by label),
+//    label order, members in any order),
 //    and each round runs the propagation kernels in their merging form over
 //    the rows, binned by length.  No sort of the entries.
 //  * sorted pairs (tunable merge_sort): the contraction above, then one pass
@@ -338,14 +338,24 @@ __global__ void k_merge_relabel(int n, const int32_t *labels, const int32_t *fou
 // k, or n + 1 while k stays on the device, when ids from *kp on are empty).
 __device__ inline int k_of(int bound, const int *kp) { return kp ? min(*kp, bound) : bound; }
 
-__global__ void k_member_keys(int n, const int32_t *labels, uint64_t *keys) {
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-        keys[v] = ((uint64_t)(uint32_t)v << 32) | (uint32_t)labels[v];
+// What a step starts from, per community id below `bound`: no partner, not
+// matched (in `found` and in the record's pad word, where the merging kernels
+// read it with a candidate's record), no links counted; the bins' counts zero.
+__global__ void k_rows_begin(int bound, const int *kp, int32_t *bp, int32_t *found, int32_t *links, CommStats *st,
+                             unsigned long long *bcount, int nbcount) {
+    const int k = k_of(bound, kp);
+    if (blockIdx.x == 0 && threadIdx.x < nbcount) bcount[threadIdx.x] = 0;
+    for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < bound; l += gridDim.x * blockDim.x) {
+        bp[l] = -1;
+        found[l] = 0;
+        links[l] = 0;
+        if (l < k) st[l].pad = 0;
+    }
 }
 
 // Community l's row starts at the volume (int_volume + ext_volume, the sum
 // of its members' degrees) of the communities below l; an empty community
-// has an empty row.
+// has an empty row.  `next` starts there too.
 struct CommVol {
     const CommStats *st;
     int bound;
@@ -355,76 +365,118 @@ struct CommVol {
     }
 };
 struct CommStart {
-    int32_t *cind;
+    int32_t *cind, *next;
     int64_t bound;
     __device__ void operator()(int64_t l, int ex, int vol) const {
         cind[l] = ex;
+        next[l] = ex;
         if (l == bound - 1) cind[bound] = ex + vol;
     }
 };
 
-// Member i of the label-sorted vertex list: an exclusive scan of the
-// members' degrees in that order puts each member's entries at its place in
-// its community's row.
-struct MemberDeg {
-    const uint64_t *members;
-    const int32_t *indices;
-    __device__ int operator()(int64_t i) const {
-        const int v = (int)(members[i] >> 32);
-        return indices[v + 1] - indices[v];
-    }
-};
-struct MemberDst {
-    const uint64_t *members;
-    int32_t *dst;
-    __device__ void operator()(int64_t i, int ex, int) const { dst[(int)(members[i] >> 32)] = ex; }
-};
-
-// every entry's label, written into the row of its vertex's community
-template <int G>
-__global__ __launch_bounds__(256) void k_member_rows_small(int p0, int p1, const int32_t *order, const int32_t *indices,
-                                                           const int32_t *adj, const int32_t *labels,
-                                                           const int32_t *dst, int32_t *ent) {
-    const int lane = __lane_id(), glane = lane & (G - 1);
-    const int per_wave = WAVE / G;
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int count = p1 - p0;
-    for (int base = wave_g * per_wave; base < count; base += nwaves * per_wave) {
-        const int gi = base + lane / G;
-        if (gi >= count) continue;
-        const int p = p0 + gi;
-        const int v = order ? order[p] : p;
-        const int start = indices[v], deg = indices[v + 1] - start, o = dst[v];
-        for (int j = glane; j < deg; j += G) ent[o + j] = labels[adj[start + j]];
+// Each vertex's place in its community's row: the next deg(v) entries of it.
+// The order of the members inside a row decides nothing (rows are counted, and
+// ties have a total order), so places are handed out as they are asked for
+// instead of sorting the vertices by label.  A workgroup sums the degrees per
+// label in LDS first, so that a large community's counter is asked once per
+// workgroup; labels beyond the table ask for themselves.  (R-MAT-20: 12 us for
+// what four radix passes and a scan of the members' degrees did in 130.)
+constexpr int MP_NT = 1024, MP_PER = 2, MP_LOG = 9;
+__global__ __launch_bounds__(MP_NT) void k_member_places(int n, const int32_t *labels, const int32_t *indices,
+                                                         int32_t *next, int32_t *dst) {
+    __shared__ int key[1 << MP_LOG], sum[1 << MP_LOG];
+    const int tile = MP_NT * MP_PER;
+    for (int64_t t0 = (int64_t)blockIdx.x * tile; t0 < n; t0 += (int64_t)gridDim.x * tile) {
+        for (int i = threadIdx.x; i < (1 << MP_LOG); i += MP_NT) {
+            key[i] = EMPTY_KEY;
+            sum[i] = 0;
+        }
+        __syncthreads();
+        int slot[MP_PER], off[MP_PER];
+#pragma unroll
+        for (int j = 0; j < MP_PER; j++) {
+            const int64_t v = t0 + j * MP_NT + threadIdx.x;
+            slot[j] = -1;
+            off[j] = 0;
+            if (v >= n) continue;
+            const int l = labels[v], deg = indices[v + 1] - indices[v];
+            const int h = (int)(((uint32_t)l * 0x9E3779B1u) >> (32 - MP_LOG));
+            int k = __hip_atomic_load(&key[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (k == EMPTY_KEY) {
+                k = atomicCAS(&key[h], EMPTY_KEY, l);
+                if (k == EMPTY_KEY) k = l;
+            }
+            if (k == l) {
+                slot[j] = h;
+                off[j] = atomicAdd(&sum[h], deg);
+            } else {
+                off[j] = atomicAdd(&next[l], deg);
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < (1 << MP_LOG); i += MP_NT)
+            if (key[i] != EMPTY_KEY) sum[i] = atomicAdd(&next[key[i]], sum[i]);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < MP_PER; j++) {
+            const int64_t v = t0 + j * MP_NT + threadIdx.x;
+            if (v < n) dst[v] = slot[j] >= 0 ? sum[slot[j]] + off[j] : off[j];
+        }
+        __syncthreads();
     }
 }
 
-__global__ __launch_bounds__(256) void k_member_rows_items(int nitems, const int4 *items, const int32_t *indices,
-                                                           const int32_t *adj, const int32_t *labels,
-                                                           const int32_t *dst, int32_t *ent) {
+// Every entry's label, written into the row of its vertex's community: the
+// long rows by items, eight neighbour-label gathers in flight per lane, then
+// the small bins, G lanes per vertex, in one launch.
+struct MemberRows {
+    int start[6];  // small bins G64..G4: positions [start[b], start[b + 1])
+    int nitems;
+    const int4 *items;
+    const int32_t *order, *indices, *adj, *labels, *dst;
+    int32_t *ent;
+};
+template <int G>
+__device__ inline void member_rows_small(const MemberRows &r, int b, int wave_g, int nwaves) {
+    const int lane = __lane_id(), glane = lane & (G - 1);
+    constexpr int per_wave = WAVE / G;
+    const int p0 = r.start[b], count = r.start[b + 1] - p0;
+    for (int base = wave_g * per_wave; base < count; base += nwaves * per_wave) {
+        const int gi = base + lane / G;
+        if (gi >= count) continue;
+        const int v = r.order ? r.order[p0 + gi] : p0 + gi;
+        const int start = r.indices[v], deg = r.indices[v + 1] - start, o = r.dst[v];
+        if (glane < deg) r.ent[o + glane] = r.labels[r.adj[start + glane]];  // at most G entries
+    }
+}
+__global__ __launch_bounds__(256) void k_member_rows(MemberRows r) {
     const int lane = __lane_id();
     const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
     const int nwaves = gridDim.x * blockDim.x / WAVE;
-    constexpr int PF = 8;  // neighbour-label gathers in flight per lane
-    for (int it = wave_g; it < nitems; it += nwaves) {
-        const int4 w = items[it];
-        const int o = dst[w.x] - indices[w.x];
+    constexpr int PF = 8;
+    for (int it = wave_g; it < r.nitems; it += nwaves) {
+        const int4 w = r.items[it];
+        const int o = r.dst[w.x] - r.indices[w.x];
         for (int j0 = w.y + lane; j0 < w.z; j0 += PF * WAVE) {
             int nb[PF];
 #pragma unroll
             for (int e = 0; e < PF; e++) {
                 const int j = j0 + e * WAVE;
-                nb[e] = j < w.z ? adj[j] : -1;
+                nb[e] = j < w.z ? r.adj[j] : -1;
             }
             int lab[PF];
 #pragma unroll
-            for (int e = 0; e < PF; e++) lab[e] = nb[e] >= 0 ? labels[nb[e]] : 0;
+            for (int e = 0; e < PF; e++) lab[e] = nb[e] >= 0 ? r.labels[nb[e]] : 0;
 #pragma unroll
             for (int e = 0; e < PF; e++)
-                if (nb[e] >= 0) ent[o + j0 + e * WAVE] = lab[e];
+                if (nb[e] >= 0) r.ent[o + j0 + e * WAVE] = lab[e];
         }
     }
+    member_rows_small<64>(r, 0, wave_g, nwaves);
+    member_rows_small<32>(r, 1, wave_g, nwaves);
+    member_rows_small<16>(r, 2, wave_g, nwaves);
+    member_rows_small<8>(r, 3, wave_g, nwaves);
+    member_rows_small<4>(r, 4, wave_g, nwaves);
 }
 
 // bin of a row of `len` entries (the vertex bins' degree bounds)
@@ -441,71 +493,105 @@ __device__ inline int row_bin(int len) {
     return BIN_G4;
 }
 
-// Per community id below `bound`: its bin as the sort key (the id above);
-// the ids from k on get bin NUM_BINS and sort after every bin.  The rows
-// and entries of each bin are counted.
-__global__ __launch_bounds__(256) void k_comm_bins(int bound, const int *kp, const int32_t *cind, uint64_t *keys,
-                                                   unsigned long long *bcount) {
-    __shared__ unsigned long long rows[NUM_BINS], ents[NUM_BINS];
-    if (threadIdx.x < NUM_BINS) {
-        rows[threadIdx.x] = 0;
-        ents[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    const int k = k_of(bound, kp);
-    for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < bound; l += gridDim.x * blockDim.x) {
-        const int len = cind[l + 1] - cind[l];
-        const int b = l < k ? row_bin(len) : NUM_BINS;
-        keys[l] = ((uint64_t)(uint32_t)l << 32) | (uint32_t)b;
-        if (b < NUM_BINS) {
-            atomicAdd(&rows[b], 1ULL);
-            atomicAdd(&ents[b], (unsigned long long)len);
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < NUM_BINS) {
-        if (rows[threadIdx.x]) atomicAdd(&bcount[threadIdx.x], rows[threadIdx.x]);
-        if (ents[threadIdx.x]) atomicAdd(&bcount[NUM_BINS + threadIdx.x], ents[threadIdx.x]);
-    }
-}
-
-__global__ void k_high_words(int k, const uint64_t *keys, int32_t *out) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < k; i += gridDim.x * blockDim.x)
-        out[i] = (int32_t)(keys[i] >> 32);
-}
-
-// One thread: the bin starts (positions in the sorted order) and the
-// fused small-row launch's split of cu16 workgroups (one per non-empty bin,
-// the rest in proportion to the bins' entries), as the host computes them
-// for the vertex bins.
-__global__ void k_row_layout(const unsigned long long *bcount, int cu16, int *layout) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Rows and entries of each bin; the workgroup that adds its counts last turns
+// them into the bin starts (positions in the bin order) and the fused
+// small-row launch's split of cu16 workgroups (one per non-empty bin, the rest
+// in proportion to the bins' entries), as the host computes them for the
+// vertex bins.  bcount: rows, entries, the bins' next positions, arrivals.
+constexpr int CB_NT = 1024, BCOUNT = 3 * NUM_BINS + 1;
+__device__ inline void row_layout(const unsigned long long *rows, const unsigned long long *ents, int cu16, int *layout) {
     long long at = 0;
     for (int b = 0; b < NUM_BINS; b++) {
         layout[b] = (int)at;
-        at += (long long)bcount[b];
+        at += (long long)rows[b];
     }
     layout[NUM_BINS] = (int)at;
     int *lo = layout + NUM_BINS + 1;
     int nonempty = 0;
     long long tot = 0;
     for (int i = 0; i < 6; i++) {
-        nonempty += bcount[BIN_W256 + i] > 0;
-        tot += (long long)bcount[NUM_BINS + BIN_W256 + i];
+        nonempty += rows[BIN_W256 + i] > 0;
+        tot += (long long)ents[BIN_W256 + i];
     }
     const long long spare = cu16 - nonempty;
     int a = 0;
     long long acc = 0;
     for (int i = 0; i < 6; i++) {
         lo[i] = a;
-        if (bcount[BIN_W256 + i] > 0) {
+        if (rows[BIN_W256 + i] > 0) {
             const int before = tot > 0 ? (int)(spare * acc / tot) : 0;
-            acc += (long long)bcount[NUM_BINS + BIN_W256 + i];
+            acc += (long long)ents[BIN_W256 + i];
             const int after = tot > 0 ? (int)(spare * acc / tot) : 0;
             a += 1 + (after - before);
         }
     }
     lo[6] = a;
+}
+__global__ __launch_bounds__(CB_NT) void k_comm_bins(int bound, const int *kp, const int32_t *cind, int cu16,
+                                                     unsigned long long *bcount, int *layout) {
+    __shared__ unsigned long long ents[NUM_BINS];
+    __shared__ unsigned rows[NUM_BINS];
+    __shared__ int last;
+    if (threadIdx.x < NUM_BINS) {
+        rows[threadIdx.x] = 0;
+        ents[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    const int k = k_of(bound, kp);
+    for (int l = blockIdx.x * CB_NT + threadIdx.x; l < k; l += gridDim.x * CB_NT) {
+        const int len = cind[l + 1] - cind[l], b = row_bin(len);
+        atomicAdd(&rows[b], 1u);
+        atomicAdd(&ents[b], (unsigned long long)len);
+    }
+    __syncthreads();
+    if (threadIdx.x < NUM_BINS) {
+        if (rows[threadIdx.x]) atomicAdd(&bcount[threadIdx.x], (unsigned long long)rows[threadIdx.x]);
+        if (ents[threadIdx.x]) atomicAdd(&bcount[NUM_BINS + threadIdx.x], ents[threadIdx.x]);
+        __threadfence();
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&bcount[3 * NUM_BINS], 1ULL) == gridDim.x - 1;
+    __syncthreads();
+    if (!last || threadIdx.x != 0) return;
+    __threadfence();
+    unsigned long long r[NUM_BINS], e[NUM_BINS];
+    for (int b = 0; b < NUM_BINS; b++) {  // as the atomics left them
+        r[b] = atomicAdd(&bcount[b], 0ULL);
+        e[b] = atomicAdd(&bcount[NUM_BINS + b], 0ULL);
+    }
+    row_layout(r, e, cu16, layout);
+}
+
+// The communities in bin order (any order inside a bin): a workgroup ranks
+// its communities per bin and asks for that many places of each bin.
+__global__ __launch_bounds__(CB_NT) void k_comm_places(int bound, const int *kp, const int32_t *cind,
+                                                       unsigned long long *bcount, const int *layout, int32_t *corder) {
+    __shared__ int cnt[NUM_BINS], base[NUM_BINS];
+    const int k = k_of(bound, kp);
+    const int lane = __lane_id();
+    for (int l0 = blockIdx.x * CB_NT; l0 < k; l0 += gridDim.x * CB_NT) {
+        if (threadIdx.x < NUM_BINS) cnt[threadIdx.x] = 0;
+        __syncthreads();
+        const int l = l0 + threadIdx.x;
+        const int b = l < k ? row_bin(cind[l + 1] - cind[l]) : -1;
+        int rank = 0;
+        for (int q = 0; q < NUM_BINS; q++) {
+            const uint64_t m = __ballot(b == q);
+            if (!m) continue;
+            const int leader = __builtin_ctzll(m);
+            int at = 0;
+            if (lane == leader) at = atomicAdd(&cnt[q], __popcll(m));
+            at = __builtin_amdgcn_readlane(at, leader);
+            if (b == q) rank = at + __popcll(m & ((1ULL << lane) - 1));
+        }
+        __syncthreads();
+        if (threadIdx.x < NUM_BINS && cnt[threadIdx.x])
+            base[threadIdx.x] = layout[threadIdx.x] +
+                                (int)atomicAdd(&bcount[2 * NUM_BINS + threadIdx.x], (unsigned long long)cnt[threadIdx.x]);
+        __syncthreads();
+        if (b >= 0) corder[base[b] + rank] = l;
+        __syncthreads();
+    }
 }
 
 // The hub layout of the rows above 4096 entries (positions [0, nh) of the
@@ -693,62 +779,49 @@ __device__ inline int pair_low(int l, const int32_t *found, const int32_t *bp) {
     return p > l ? p : -1;  // the partner when l is the lower side of a pair
 }
 
-// rows of at most 64 entries (positions [layout[b0], layout[b1])), G lanes
-// per row
-template <int G>
-__global__ __launch_bounds__(256) void k_pair_links_small(const int *layout, int b0, int b1, const int32_t *corder,
-                                                          const int32_t *cind, const int32_t *ent, const int32_t *found,
-                                                          const int32_t *bp, int32_t *links) {
-    const int lane = __lane_id(), glane = lane & (G - 1);
-    const int t = (blockIdx.x * blockDim.x + threadIdx.x) / G;
-    const int nt = gridDim.x * blockDim.x / G;
-    const int p0 = layout[b0], p1 = layout[b1];
-    for (int base = t; base < p1 - p0; base += nt) {
-        const int l = corder[p0 + base];
-        const int p = pair_low(l, found, bp);
-        int c = 0;
-        if (p >= 0)
-            for (int j = cind[l] + glane; j < cind[l + 1]; j += G) c += ent[j] == p;
+// One launch: a wave per 4096-entry chunk of a hub row (summed with atomics),
+// a wave per row of 65-4096 entries, eight lanes per shorter row; four entries
+// a lane in flight.
+template <int W>
+__device__ inline int count_links(const int32_t *ent, int b, int e, int first, int p) {
+    int c = 0;
+    for (int j = b + first; j < e; j += 4 * W) {
+        int x[4];
 #pragma unroll
-        for (int d = G / 2; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
-        if (p >= 0 && glane == 0) links[l] = c;
+        for (int q = 0; q < 4; q++) x[q] = j + q * W < e ? ent[j + q * W] : -1;
+#pragma unroll
+        for (int q = 0; q < 4; q++) c += x[q] == p;
     }
+    return c;
 }
-
-// longer rows (positions [layout[b0], layout[b1])): one wave per row (up to
-// 4096 entries), or per 4096-entry chunk of a hub row (summed with atomics)
-__global__ __launch_bounds__(256) void k_pair_links_rows(const int *layout, int b0, int b1, const int32_t *corder,
-                                                         const int32_t *cind, const int32_t *ent, const int32_t *found,
-                                                         const int32_t *bp, int32_t *links) {
+__global__ __launch_bounds__(256) void k_pair_links(const int *counts, const int4 *chunks, const int *layout,
+                                                    const int32_t *corder, const int32_t *cind, const int32_t *ent,
+                                                    const int32_t *found, const int32_t *bp, int32_t *links) {
     const int lane = __lane_id();
     const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
     const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int p1 = layout[b1];
-    for (int q = layout[b0] + wave_g; q < p1; q += nwaves) {
-        const int l = corder[q];
-        const int p = pair_low(l, found, bp);
-        if (p < 0) continue;
-        int c = 0;
-        for (int j = cind[l] + lane; j < cind[l + 1]; j += WAVE) c += ent[j] == p;
-        c = wave_sum(c);
-        if (lane == 0) links[l] = c;
-    }
-}
-
-__global__ __launch_bounds__(256) void k_pair_links_hub(const int *counts, const int4 *chunks, const int32_t *ent,
-                                                        const int32_t *found, const int32_t *bp, int32_t *links) {
-    const int lane = __lane_id();
-    const int wave_g = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int nchunks = counts[0];
+    const int nchunks = counts[0], q0 = layout[BIN_B4096], q1 = layout[BIN_G64], q2 = layout[NUM_BINS];
     for (int it = wave_g; it < nchunks; it += nwaves) {
         const int4 ck = chunks[it];  // {hub, community, begin, end}
         const int p = pair_low(ck.y, found, bp);
         if (p < 0) continue;
-        int c = 0;
-        for (int j = ck.z + lane; j < ck.w; j += WAVE) c += ent[j] == p;
-        c = wave_sum(c);
+        const int c = wave_sum(count_links<WAVE>(ent, ck.z, ck.w, lane, p));
         if (lane == 0 && c) atomicAdd(&links[ck.y], c);
+    }
+    for (int q = q0 + wave_g; q < q1; q += nwaves) {
+        const int l = corder[q];
+        const int p = pair_low(l, found, bp);
+        if (p < 0) continue;
+        const int c = wave_sum(count_links<WAVE>(ent, cind[l], cind[l + 1], lane, p));
+        if (lane == 0) links[l] = c;
+    }
+    for (int q = q1 + wave_g * 8 + lane / 8; q < q2; q += nwaves * 8) {  // the lanes of a group share q
+        const int l = corder[q];
+        const int p = pair_low(l, found, bp);
+        int c = p >= 0 ? count_links<8>(ent, cind[l], cind[l + 1], lane & 7, p) : 0;
+#pragma unroll
+        for (int d = 4; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
+        if (p >= 0 && (lane & 7) == 0) links[l] = c;
     }
 }
 
@@ -777,7 +850,9 @@ __global__ void k_clear_pads(int bound, const int *kp, CommStats *st) {
     for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < k; l += gridDim.x * blockDim.x) st[l].pad = 0;
 }
 
-// refinement.cpp:264-274 for the communities below k
+// refinement.cpp:264-274 for the communities below k.  The unmatched are
+// counted only where a caller reads the count: a counter that every wave adds
+// to cost 50 of the 57 us this took on R-MAT-20.
 __global__ void k_handshake_rec(int bound, const int *kp, int32_t *found, const int32_t *bp, int32_t *unmatched,
                                 CommStats *st) {
     const int k = k_of(bound, kp);
@@ -789,6 +864,7 @@ __global__ void k_handshake_rec(int bound, const int *kp, int32_t *found, const 
         }
         if (!found[l]) local++;
     }
+    if (!unmatched) return;
     local = wave_sum(local);
     if (__lane_id() == 0 && local) atomicAdd(unmatched, local);
 }
@@ -796,8 +872,7 @@ __global__ void k_handshake_rec(int bound, const int *kp, int32_t *found, const 
 // Device state of the community rows and the row set of the merging step
 // (every buffer sized for the largest step the graph allows).
 struct MergeRows {
-    GrowBuf<int32_t> ent, cind, corder, dst, links;
-    GrowBuf<uint64_t> mk0, mk1;
+    GrowBuf<int32_t> ent, cind, next, corder, dst, links;
     GrowBuf<unsigned long long> bcount;
     GrowBuf<int> layout, counts;
     // hub layout
@@ -833,9 +908,8 @@ static int reserve_rows(pcd_ctx *ctx, MergeRows &R) {
     PCD_TRY(R.corder.reserve(ctx, n + 2));
     PCD_TRY(R.dst.reserve(ctx, n + 2));
     PCD_TRY(R.links.reserve(ctx, n + 2));
-    PCD_TRY(R.mk0.reserve(ctx, n + 2));
-    PCD_TRY(R.mk1.reserve(ctx, n + 2));
-    PCD_TRY(R.bcount.reserve(ctx, 2 * NUM_BINS));
+    PCD_TRY(R.next.reserve(ctx, n + 3));
+    PCD_TRY(R.bcount.reserve(ctx, BCOUNT));
     PCD_TRY(R.layout.reserve(ctx, ROW_LAYOUT_INTS));
     bool grew_n = false;
     PCD_TRY(R.counts.reserve(ctx, 4, &grew_n));
@@ -908,49 +982,35 @@ static int reserve_rows(pcd_ctx *ctx, MergeRows &R) {
 // all on the stream, nothing read back.
 static int build_community_rows(pcd_ctx *ctx, MergeRows &R, int bound, const int *kp) {
     const int n = ctx->n;
-    const int half = label_bits(bound);
-    // members by label (stable: ascending vertex id inside a community)
+    // the rows' extents and the members' places in them
     kt_begin(ctx, KS_MERGE_SORT);
-    hipLaunchKernelGGL(k_member_keys, dim3(grid_for(ctx, n, 256)), dim3(256), 0, ctx->stream, n, ctx->d_labels,
-                       R.mk0.p);
-    uint64_t *members = nullptr;
-    PCD_TRY(radix_sort_u64(ctx, R.mk0.p, R.mk1.p, n, half, &members));
-    PCD_TRY(device_scan(ctx, n, MemberDeg{members, ctx->d_indices}, MemberDst{members, R.dst.p}, nullptr));
-    PCD_TRY(device_scan(ctx, bound, CommVol{ctx->d_stats, bound, kp}, CommStart{R.cind.p, bound}, nullptr));
+    PCD_TRY(device_scan(ctx, bound, CommVol{ctx->d_stats, bound, kp}, CommStart{R.cind.p, R.next.p, bound}, nullptr));
+    hipLaunchKernelGGL(k_member_places, dim3(grid_for(ctx, n, MP_NT * MP_PER, 2)), dim3(MP_NT), 0, ctx->stream, n,
+                       ctx->d_labels, ctx->d_indices, R.next.p, R.dst.p);
     kt_end(ctx, KS_MERGE_SORT);
     // the rows: every entry's label at its member's place
     kt_begin(ctx, KS_MERGE_KEYS);
-    if (ctx->num_stat_items > 0)
-        hipLaunchKernelGGL(k_member_rows_items, dim3(grid_for(ctx, ctx->num_stat_items, 4, 16)), dim3(256), 0,
-                           ctx->stream, ctx->num_stat_items, ctx->d_stat_items, ctx->d_indices, ctx->d_adj,
-                           ctx->d_labels, R.dst.p, R.ent.p);
-    const BinLayout &vb = ctx->bins;
-    auto small = [&](auto g, int bin) {
-        constexpr int G = decltype(g)::value;
-        const int p0 = vb.start[bin], p1 = vb.start[bin + 1];
-        if (p1 > p0)
-            hipLaunchKernelGGL(k_member_rows_small<G>, dim3(grid_for(ctx, p1 - p0, 256 / G, 16)), dim3(256), 0,
-                               ctx->stream, p0, p1, ctx->d_order, ctx->d_indices, ctx->d_adj, ctx->d_labels, R.dst.p,
-                               R.ent.p);
-    };
-    small(std::integral_constant<int, 64>{}, BIN_G64);
-    small(std::integral_constant<int, 32>{}, BIN_G32);
-    small(std::integral_constant<int, 16>{}, BIN_G16);
-    small(std::integral_constant<int, 8>{}, BIN_G8);
-    small(std::integral_constant<int, 4>{}, BIN_G4);
+    MemberRows mr;
+    for (int i = 0; i < 6; i++) mr.start[i] = ctx->bins.start[BIN_G64 + i];
+    mr.nitems = ctx->num_stat_items;
+    mr.items = ctx->d_stat_items;
+    mr.order = ctx->d_order;
+    mr.indices = ctx->d_indices;
+    mr.adj = ctx->d_adj;
+    mr.labels = ctx->d_labels;
+    mr.dst = R.dst.p;
+    mr.ent = R.ent.p;
+    hipLaunchKernelGGL(k_member_rows, dim3(grid_for(ctx, 2 * (int64_t)ctx->m + n, 1024, 16)), dim3(256), 0, ctx->stream,
+                       mr);
     kt_end(ctx, KS_MERGE_KEYS);
     PCD_HIP(hipGetLastError());
-    // bins of the community rows by length (one radix pass over 4-bit bin
-    // keys), the launch layout, and the hub layout
+    // the communities in bin order by row length, the launch layout, and the
+    // hub layout
     kt_begin(ctx, KS_MERGE_SORT);
-    PCD_TRY(fill_u64(ctx, (uint64_t *)R.bcount.p, 0, 2 * NUM_BINS));
-    hipLaunchKernelGGL(k_comm_bins, dim3(grid_for(ctx, bound, 256, 4)), dim3(256), 0, ctx->stream, bound, kp, R.cind.p,
-                       R.mk0.p, R.bcount.p);
-    uint64_t *cs = nullptr;
-    PCD_TRY(radix_sort_u64(ctx, R.mk0.p, R.mk1.p, bound, 4, &cs));
-    hipLaunchKernelGGL(k_high_words, dim3(grid_for(ctx, bound, 256)), dim3(256), 0, ctx->stream, bound, cs,
-                       R.corder.p);
-    hipLaunchKernelGGL(k_row_layout, dim3(1), dim3(64), 0, ctx->stream, R.bcount.p, ctx->cu_count * 16, R.layout.p);
+    hipLaunchKernelGGL(k_comm_bins, dim3(grid_for(ctx, bound, CB_NT, 1)), dim3(CB_NT), 0, ctx->stream, bound, kp,
+                       R.cind.p, ctx->cu_count * 16, R.bcount.p, R.layout.p);
+    hipLaunchKernelGGL(k_comm_places, dim3(grid_for(ctx, bound, CB_NT, 2)), dim3(CB_NT), 0, ctx->stream, bound, kp,
+                       R.cind.p, R.bcount.p, R.layout.p, R.corder.p);
     hipLaunchKernelGGL(k_hub_sizes, dim3(1), dim3(HL_NT), 0, ctx->stream, R.layout.p, R.corder.p, R.cind.p,
                        std::max(64, ctx->tune.hub_part_entries), R.hd);
     hipLaunchKernelGGL(k_hub_expand, dim3(ctx->cu_count * 2), dim3(256), 0, ctx->stream, R.cind.p, R.hd);
@@ -991,7 +1051,6 @@ int merge_rows_reserve(pcd_ctx *ctx) {
     MergeRows &R = *static_cast<MergeRows *>(ctx->mrows);
     PCD_TRY(reserve_rows(ctx, R));
     PCD_TRY(ensure_scan_parts(ctx, (int64_t)ctx->n + 2));
-    PCD_TRY(ensure_sort_space(ctx, (int64_t)ctx->n + 2));
     return PCD_OK;
 }
 
@@ -1020,11 +1079,9 @@ static int merging_rows_dev(pcd_ctx *ctx, pcd_rule rule, int rounds, uint64_t se
     if (!ctx->mrows) return fail(PCD_E_STATE, "merging rows not reserved before a capture");
     MergeRows &R = *static_cast<MergeRows *>(ctx->mrows);
     if (bound <= 0) return PCD_OK;
+    hipLaunchKernelGGL(k_rows_begin, dim3(grid_for(ctx, bound, 256)), dim3(256), 0, ctx->stream, bound, kp, ctx->d_bp,
+                       ctx->d_found, R.links.p, ctx->d_stats, R.bcount.p, BCOUNT);
     PCD_TRY(build_community_rows(ctx, R, bound, kp));
-    PCD_TRY(fill_i32(ctx, ctx->d_bp, -1, bound));
-    PCD_TRY(fill_i32(ctx, ctx->d_found, 0, bound));
-    hipLaunchKernelGGL(k_clear_pads, dim3(grid_for(ctx, bound, 256)), dim3(256), 0, ctx->stream, bound, kp,
-                       ctx->d_stats);
     LPArgs a{};
     a.indices = R.cind.p;  // community l's row: entries [cind[l], cind[l+1]) of ent
     a.adj = R.ent.p;
@@ -1041,12 +1098,13 @@ static int merging_rows_dev(pcd_ctx *ctx, pcd_rule rule, int rounds, uint64_t se
         a.seed = merge_seed(seed, rnd);
         PCD_TRY(merge_rows_launch(ctx, R.rows, a));
         kt_begin(ctx, KS_MERGE_ROUNDS);
-        PCD_TRY(fill_i32(ctx, unmatched, 0, 1));
+        const bool ask = rnd + 1 < rounds && !ctx->capturing;
+        if (ask) PCD_TRY(fill_i32(ctx, unmatched, 0, 1));
         hipLaunchKernelGGL(k_handshake_rec, dim3(grid_for(ctx, bound, 256)), dim3(256), 0, ctx->stream, bound, kp,
-                           ctx->d_found, ctx->d_bp, unmatched, ctx->d_stats);
+                           ctx->d_found, ctx->d_bp, ask ? unmatched : nullptr, ctx->d_stats);
         kt_end(ctx, KS_MERGE_ROUNDS);
         PCD_HIP(hipGetLastError());
-        if (rnd + 1 < rounds && !ctx->capturing) {
+        if (ask) {
             // refinement.cpp:220,264-274: stop once every community is matched
             // (a captured pass runs every round: once all are matched, a
             // round changes nothing)
@@ -1060,15 +1118,8 @@ static int merging_rows_dev(pcd_ctx *ctx, pcd_rule rule, int rounds, uint64_t se
         // the statistics of the merged labels, from the records and the
         // pairs' links (the next compression renumbers them)
         kt_begin(ctx, KS_MERGE_STATS);
-        PCD_TRY(fill_i32(ctx, R.links.p, 0, bound));
-        hipLaunchKernelGGL(k_pair_links_hub, dim3(ctx->cu_count * 8), dim3(256), 0, ctx->stream, R.counts.p, R.items.p,
-                           R.ent.p, ctx->d_found, ctx->d_bp, R.links.p);
-        hipLaunchKernelGGL(k_pair_links_rows, dim3(ctx->cu_count * 8), dim3(256), 0, ctx->stream, R.layout.p,
-                           (int)BIN_B4096, (int)BIN_G64, R.corder.p, R.cind.p, R.ent.p, ctx->d_found, ctx->d_bp,
-                           R.links.p);
-        hipLaunchKernelGGL(k_pair_links_small<8>, dim3(ctx->cu_count * 8), dim3(256), 0, ctx->stream, R.layout.p,
-                           (int)BIN_G64, (int)NUM_BINS, R.corder.p, R.cind.p, R.ent.p, ctx->d_found, ctx->d_bp,
-                           R.links.p);
+        hipLaunchKernelGGL(k_pair_links, dim3(ctx->cu_count * 8), dim3(256), 0, ctx->stream, R.counts.p, R.items.p,
+                           R.layout.p, R.corder.p, R.cind.p, R.ent.p, ctx->d_found, ctx->d_bp, R.links.p);
         hipLaunchKernelGGL(k_merged_stats, dim3(grid_for(ctx, bound, 256)), dim3(256), 0, ctx->stream, bound, kp,
                            ctx->d_found, ctx->d_bp, R.links.p, ctx->d_stats);
         kt_end(ctx, KS_MERGE_STATS);
