@@ -485,13 +485,15 @@ extern "C" int pcd_graph_info(pcd_ctx *ctx, int *n, int *m, int *max_degree) {
 extern "C" int pcd_labels_upload(pcd_ctx *ctx, const int32_t *labels) {
     PCD_TRY(check_graph(ctx));
     if (!labels) return fail(PCD_E_INVALID, "null labels");
-    int mx = -1;
-    bool has_new = false;
+    // least and largest label without a branch per label (vectorised: 0.44 ->
+    // 0.05 ms of the 0.5 ms that 646,000 labels took)
+    int mn = INT32_MAX, mx = -1;
     for (int v = 0; v < ctx->n; v++) {
-        if (labels[v] < -1) return fail(PCD_E_INVALID, "labels must be >= 0 or NEW_LABEL");
-        if (labels[v] == -1) has_new = true;
+        mn = std::min(mn, labels[v]);
         mx = std::max(mx, labels[v]);
     }
+    if (mn < -1) return fail(PCD_E_INVALID, "labels must be >= 0 or NEW_LABEL");
+    const bool has_new = mn == -1;
     int64_t bound = (int64_t)mx + 1;
     if (bound + 1 > ctx->first_cap) {
         dev_free(ctx, ctx->d_first);
