@@ -379,7 +379,7 @@ struct CommStart {
 // ties have a total order), so places are handed out as they are asked for
 // instead of sorting the vertices by label.  A workgroup sums the degrees per
 // label in LDS first, so that a large community's counter is asked once per
-// workgroup; labels beyond the table ask for themselves.  (R-MAT-20: 12 us for
+// workgroup; labels beyond the table ask for themselves.  (R-MAT-20: 20 us for
 // what four radix passes and a scan of the members' degrees did in 130.)
 constexpr int MP_NT = 1024, MP_PER = 2, MP_LOG = 9;
 __global__ __launch_bounds__(MP_NT) void k_member_places(int n, const int32_t *labels, const int32_t *indices,

@@ -162,27 +162,6 @@ int compress_labels_dev(pcd_ctx *ctx, bool defer_k) {
 }
 
 // ------------------------------------------------------------ the fused pass
-// The numbering of first occurrences in one launch: every workgroup counts the
-// first occurrences of all vertices before its tile itself, which for n up to
-// DIRECT_N vertices costs less than the two launches and their gaps that a scan
-// of tile sums takes (n = 10,000: 3 us instead of 9).
-constexpr int DIRECT_N = 1 << 16, NUMBER_NT = 1024;
-__global__ __launch_bounds__(NUMBER_NT) void k_number_direct(int n, FirstFlag flag, FirstStore store, int32_t *total) {
-    __shared__ int lds[NUMBER_NT / WAVE];
-    const int tile = blockIdx.x * NUMBER_NT;
-    int before = 0;
-#pragma unroll 8
-    for (int v = threadIdx.x; v < tile; v += NUMBER_NT) before += flag(v);
-    int run;
-    block_excl_scan_n<NUMBER_NT>(before, &run, lds);
-    const int v = tile + threadIdx.x;
-    const int x = v < n ? flag(v) : 0;
-    int tot;
-    const int ex = block_excl_scan_n<NUMBER_NT>(x, &tot, lds);
-    if (v < n) store(v, run + ex, x);
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = run + tot;
-}
-
 // What follows the numbering, elementwise: the new labels (into both label
 // buffers: the step's result starts as a copy), the records back in place,
 // the total each gain reads, and the metric's sums; the workgroup that adds
@@ -270,9 +249,9 @@ int fused_compress_dev(pcd_ctx *ctx, pcd_rule rule, const LoopParams &p, LoopSta
     const FirstStore store{ctx->d_labels, ctx->d_labels_alt, ctx->d_newid, ctx->d_stats,
                            ctx->d_stats_alt, ctx->d_indices, ctx->d_firstv};
     int32_t *total = ctx->d_scan_part;
-    if (n <= DIRECT_N)
-        hipLaunchKernelGGL(k_number_direct, dim3((n + NUMBER_NT - 1) / NUMBER_NT), dim3(NUMBER_NT), 0, ctx->stream, n,
-                           flag, store, total);
+    if (n <= SCAN_DIRECT_N)
+        hipLaunchKernelGGL((k_scan_direct<FirstFlag, FirstStore>), dim3((n + SCAN_DIRECT_NT - 1) / SCAN_DIRECT_NT),
+                           dim3(SCAN_DIRECT_NT), 0, ctx->stream, n, flag, store, total);
     else
         PCD_TRY(device_scan(ctx, n, flag, store, &total));
     const PassTail t{n, ctx->m, rule.kind, rule.lambda, total, ctx->d_newid, ctx->d_labels, ctx->d_labels_alt,

@@ -6,6 +6,7 @@ import pytest
 
 import oracle_lib as O
 import gpu_graphs as GG
+from test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
 
@@ -167,7 +168,7 @@ def test_small_graph_loop(ctx, name):
                 assert np.array_equal(x, y, equal_nan=True) if isinstance(x, float) else np.array_equal(x, y), (name, i)
 
 
-@pytest.mark.parametrize("n", [1023, 1024, 1025, 65535, 65536, 65537])
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 20480, 20481, 65536, 65537])
 def test_fused_pass_sizes(ctx, n):
     """Sizes at the edges of the numbering's tiles and of the direct forms:
     every vertex on a ring with chords (degrees 2-40 and one hub), modularity
@@ -201,3 +202,63 @@ def test_fused_pass_sizes(ctx, n):
             ctx.set_tuning(key, 1)
         for other in got[1:]:
             assert all(np.array_equal(x, y) for x, y in zip(got[0], other)), (n, kind)
+
+
+@pytest.mark.parametrize("kind", ["one", "half", "table", "singletons"])
+@pytest.mark.parametrize("graph", ["bin_zoo", "rmat12", "star", "no_edges"])
+def test_merging_of_crowded_partitions(ctx, graph, kind):
+    """Rows laid out by counters that many vertices ask at once: partners and
+    statistics of a merging step equal the sorted-pair form's and the oracle's
+    full count, with one round and three."""
+    g = {"bin_zoo": GG.bin_zoo, "rmat12": lambda: GG.rmat(12), "no_edges": lambda: GG.csr_direct(6, []),
+         "star": lambda: GG.csr_direct(2049, [(0, i) for i in range(1, 2049)])}[graph]()
+    n, m, ind, adj = g[:4]
+    lab = np.arange(n, dtype=np.int32) if kind == "singletons" else crowded(kind, n)
+    ctx.upload_graph(n, m, ind, adj)
+    for rule, lam, rounds, tie in ((O.MOD, 0.0, 1, 0), (O.CPM, 0.001, 3, 1)):
+        got = []
+        for sort in (0, 1):
+            ctx.set_tuning("merge_sort", sort)
+            ctx.upload_labels(lab)
+            ctx.compress()
+            ctx.statistics()
+            ctx.merge(rule, lam, rounds=rounds, seed=4, step=1, tie=tie)
+            got.append(ctx.labels())
+            k = ctx.compress()
+            ctx.statistics()
+            _, so, ivo, evo = O.collect_statistics(n, ind, adj, ctx.labels())
+            for x, y in zip(ctx.stats(k), (so, ivo, evo)):
+                assert np.array_equal(x, y), (sort, rule)
+        ctx.set_tuning("merge_sort", 0)
+        assert np.array_equal(got[0], got[1]), rule
+
+
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 1023, 1025, 4096, 4097, 8193, 12289, 20481, 28673, 36864, 36865, 262144,
+                               262145, 600001])
+def test_noalloc_compression_sizes(ctx, n):
+    """The allocation-free compression at the edges of its one-workgroup and
+    tiled forms, few and many labels, with NEW_LABEL and
+    with a label out of range (k = -1, the flag cleared for the next call)."""
+    hip = Hip()
+    rng = np.random.default_rng(n + 1)
+    d, out, k_dev = hip.alloc(4 * n), hip.alloc(4 * (n + 8)), hip.alloc(4)
+    for kinds, new, bad in ((max(1, n // 3), 0.2, False), (3, 0.0, True), (3, 0.0, False), (max(1, n), 0.0, False)):
+        lab = (rng.integers(0, kinds, n) * 7 % max(1, n)).astype(np.int32)
+        lab[rng.random(n) < new] = -1
+        if bad and n:
+            lab[n // 2] = n
+        if n:
+            hip.put(d, lab)
+        hip.put(out, np.full(n + 8, -9, np.int32))
+        parcd.compress_labels_noalloc(n, d, out, k_dev)
+        hip.ok(hip.h.hipStreamSynchronize(None))
+        got = hip.get(out, n + 8)
+        assert (got[n:] == -9).all()
+        if bad and n:
+            assert int(hip.get(k_dev, 1)[0]) == -1
+            continue
+        want, k = O.compress_labels(lab) if n else (lab, 0)
+        assert int(hip.get(k_dev, 1)[0]) == k
+        assert np.array_equal(got[:n], want)
+    for p in (d, out, k_dev):
+        hip.ok(hip.h.hipFree(p))
