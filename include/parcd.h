@@ -210,7 +210,10 @@ int pcd_bin_counters(pcd_ctx *ctx, int bin, int64_t *active, int64_t *entries, i
  * of a graph of at most 4096 vertices and 32768 entries, under modularity or
  * CPM, in one launch of one workgroup) and "fused_pass" (0/1: a
  * device-resident propagation pass under modularity or CPM shares launches
- * between compression, metric, stop rule and bookkeeping).
+ * between compression, metric, stop rule and bookkeeping) and
+ * "contract_rows_min" (pcd_contract counts pairs over community rows from this
+ * many entries on, where the communities' volumes promise few pairs; default
+ * 2^22).
  * Results do not depend on them. */
 int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value);
 /* Hub label partitions whose distinct labels overflowed their LDS table

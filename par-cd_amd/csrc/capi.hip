@@ -890,6 +890,9 @@ extern "C" int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value) {
         ctx->tune.merge_sort = value != 0;
     } else if (k == "graph_loop") {
         ctx->tune.graph_loop = value != 0;
+    } else if (k == "contract_rows_min") {
+        if (value < 0) return fail(PCD_E_INVALID, "contract_rows_min must be >= 0");
+        ctx->tune.contract_rows_min = value;
     } else if (k == "fused_pass") {
         ctx->tune.fused_pass = value != 0;
     } else if (k == "solo_loop") {

@@ -114,6 +114,7 @@ struct Tuning {
                                  // (R-MAT-22 iteration 1.120 ms at 2, 1.102 at 8, 1.131 at 32)
     int graph_loop = 1;          // modularity / CPM with -s 0: passes replayed from one captured
                                  // pass with the stop rule on the device (pcd_iterate_many)
+    int contract_rows_min = 1 << 22;  // contraction counts pairs over community rows from this many entries on
     int fused_pass = 1;          // a captured propagation pass (modularity, CPM) shares launches between its parts
     int solo_loop = 1;           // the passes of a small graph in one launch of one workgroup (solo.hip)
     int graph_loop_min_entries = 0;  // graphs with fewer CSR entries run pass by pass
@@ -342,6 +343,7 @@ int fill_i32(pcd_ctx *ctx, int32_t *p, int32_t v, int64_t count);
 int fill_u64(pcd_ctx *ctx, uint64_t *p, uint64_t v, int64_t count);
 int ensure_scan_parts(pcd_ctx *ctx, int64_t n);
 int radix_sort_u64(pcd_ctx *ctx, uint64_t *keys, uint64_t *tmp, int64_t n, int bits, uint64_t **out);
+int radix_sort_bits_u64(pcd_ctx *ctx, uint64_t *keys, uint64_t *tmp, int64_t n, int shift, int bits, uint64_t **out);
 // the tile histograms of a radix sort of n keys (a captured sort may not allocate)
 int ensure_sort_space(pcd_ctx *ctx, int64_t n);
 

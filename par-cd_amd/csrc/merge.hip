@@ -6,7 +6,9 @@
 // entry itself, the buffer is radix-sorted, and a run-length reduce-by-key
 // (scan of run heads) gives the community graph as unique (l, k, links)
 // sorted by (l, k): the table refinement.cpp:228-238 hashes per community
-// and framework-cuda.cu:744-807 sorts.
+// and framework-cuda.cu:744-807 sorts.  Where a few large communities hold
+// most entries, the entries are first gathered into community rows and counted
+// per (l, k) in LDS, tile by tile, and only the tiles' pairs are sorted.
 //
 // Merging round: each unmatched, eligible community l takes the neighbour
 // community k (unmatched) of best score_merge >= 0 (refinement.cpp:240-260;
@@ -119,9 +121,8 @@ static void launch_keys_small(pcd_ctx *ctx, int bin, int bits) {
                        p1, ctx->d_order, ctx->d_indices, ctx->d_adj, ctx->d_labels, bits, ctx->d_keys0);
 }
 
-// Builds the sorted unique (l, k) keys in ctx->d_keys1[0..U) with link
-// counts in ctx->d_pair_links.  Returns U and the key layout.
-static int build_pairs(pcd_ctx *ctx, int64_t *U_out, int *half_out) {
+// the buffers of the pairs, E entries each
+static int reserve_pairs(pcd_ctx *ctx) {
     const int64_t E = (int64_t)2 * ctx->m;
     if ((size_t)E > ctx->keys_cap) {
         if (ctx->d_keys0) dev_free(ctx, ctx->d_keys0);
@@ -137,6 +138,14 @@ static int build_pairs(pcd_ctx *ctx, int64_t *U_out, int *half_out) {
         PCD_TRY(dev_alloc_t(ctx, &ctx->d_pair_head, E + 1));
         ctx->keys_cap = (size_t)E;
     }
+    return PCD_OK;
+}
+
+// Builds the sorted unique (l, k) keys in ctx->d_keys1[0..U) with link
+// counts in ctx->d_pair_links.  Returns U and the key layout.
+static int build_pairs(pcd_ctx *ctx, int64_t *U_out, int *half_out) {
+    const int64_t E = (int64_t)2 * ctx->m;
+    PCD_TRY(reserve_pairs(ctx));
     const int half = label_bits(ctx->k);
     const int bits = 2 * half;
     kt_begin(ctx, KS_MERGE_KEYS);
@@ -977,10 +986,9 @@ static int reserve_rows(pcd_ctx *ctx, MergeRows &R) {
     return PCD_OK;
 }
 
-// Builds the community rows of the current labels (ids below `bound`, k on
-// the device when kp is set): entries, offsets, bin order and hub layout,
-// all on the stream, nothing read back.
-static int build_community_rows(pcd_ctx *ctx, MergeRows &R, int bound, const int *kp) {
+// The community rows of the current labels (ids below `bound`, k on the
+// device when kp is set): offsets and entries.
+static int fill_rows(pcd_ctx *ctx, MergeRows &R, int bound, const int *kp) {
     const int n = ctx->n;
     // the rows' extents and the members' places in them
     kt_begin(ctx, KS_MERGE_SORT);
@@ -1004,6 +1012,14 @@ static int build_community_rows(pcd_ctx *ctx, MergeRows &R, int bound, const int
                        mr);
     kt_end(ctx, KS_MERGE_KEYS);
     PCD_HIP(hipGetLastError());
+    return PCD_OK;
+}
+
+// Builds the community rows of the current labels (ids below `bound`, k on
+// the device when kp is set): entries, offsets, bin order and hub layout,
+// all on the stream, nothing read back.
+static int build_community_rows(pcd_ctx *ctx, MergeRows &R, int bound, const int *kp) {
+    PCD_TRY(fill_rows(ctx, R, bound, kp));
     // the communities in bin order by row length, the launch layout, and the
     // hub layout
     kt_begin(ctx, KS_MERGE_SORT);
@@ -1201,10 +1217,197 @@ int merging_dev(pcd_ctx *ctx, pcd_rule rule, int rounds, uint64_t seed, int step
     return merging_rows_dev(ctx, rule, rounds, seed, step, tie);
 }
 
+// ---------------------------------------------------------------- contraction by rows
+// Pairs of one tile of the community rows (rows one after another, so a tile
+// is a few rows): the (row, label) of its entries counted in LDS, and each
+// distinct one sent to `out` with its count below it.  The tile's share of
+// `out` is asked for once.
+constexpr int CT_NT = 512, CT_PER = 4, CT_TILE = CT_NT * CT_PER, CT_LOG = 12;
+constexpr int CT_CNT_BITS = 13;  // counts up to CT_TILE
+static_assert(CT_TILE < (1 << CT_CNT_BITS) && CT_TILE * 2 == (1 << CT_LOG), "tile counts and table load");
+__global__ __launch_bounds__(CT_NT) void k_row_pairs(int64_t E, int k, int half, const int32_t *cind, const int32_t *ent,
+                                                     uint64_t *out, unsigned long long *nout) {
+    constexpr uint64_t NONE = ~0ULL;  // no key: rows and labels stay below 2^half - 1
+    __shared__ unsigned long long keys[1 << CT_LOG];
+    __shared__ int cnts[1 << CT_LOG];
+    __shared__ int part[CT_NT / WAVE];
+    __shared__ unsigned long long base;
+    const int64_t ntiles = (E + CT_TILE - 1) / CT_TILE;
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const int e0 = (int)(t * CT_TILE), e1 = (int)min(E, (t + 1) * CT_TILE);
+        for (int i = threadIdx.x; i < (1 << CT_LOG); i += CT_NT) {
+            keys[i] = NONE;
+            cnts[i] = 0;
+        }
+        // rows of the tile: the last rows starting at or before its ends
+        const int r0 = last_le(cind, k, e0), r1 = last_le(cind, k, e1 - 1);
+        __syncthreads();
+        int lab[CT_PER];
+#pragma unroll
+        for (int j = 0; j < CT_PER; j++) {
+            const int e = e0 + j * CT_NT + threadIdx.x;
+            lab[j] = e < e1 ? ent[e] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < CT_PER; j++) {
+            if (lab[j] < 0) continue;
+            const int e = e0 + j * CT_NT + threadIdx.x;
+            const int r = r0 + last_le(cind + r0, r1 - r0 + 1, e);
+            if (lab[j] == r) continue;
+            const unsigned long long key = ((unsigned long long)(uint32_t)r << half) | (uint32_t)lab[j];
+            uint32_t h = (uint32_t)((key * 0x9E3779B97F4A7C15ULL) >> (64 - CT_LOG));
+            while (true) {
+                const unsigned long long old = atomicCAS(&keys[h], (unsigned long long)NONE, key);
+                if (old == NONE || old == key) break;
+                h = (h + 1) & ((1 << CT_LOG) - 1);
+            }
+            atomicAdd(&cnts[h], 1);
+        }
+        __syncthreads();
+        int mine = 0;
+        for (int i = threadIdx.x; i < (1 << CT_LOG); i += CT_NT) mine += keys[i] != NONE;
+        int tot;
+        int at = block_excl_scan_n<CT_NT>(mine, &tot, part);
+        if (threadIdx.x == 0) base = atomicAdd(nout, (unsigned long long)tot);
+        __syncthreads();
+        for (int i = threadIdx.x; i < (1 << CT_LOG); i += CT_NT)
+            if (keys[i] != NONE) out[base + at++] = (keys[i] << CT_CNT_BITS) | (unsigned long long)cnts[i];
+        __syncthreads();
+    }
+}
+
+// Runs of equal pairs among the sorted partial counts, and the counts before
+// each element: a run's links are the difference of two of those (additions to
+// a word per run queue on the long runs: 0.74 ms instead of 0.02).
+struct PairHead {
+    const uint64_t *v;
+    __device__ int operator()(int64_t i) const {
+        return (i == 0 || (v[i] >> CT_CNT_BITS) != (v[i - 1] >> CT_CNT_BITS)) ? 1 : 0;
+    }
+};
+struct PairKey {
+    const uint64_t *v;
+    uint64_t *ukeys;
+    int32_t *hpos;
+    __device__ void operator()(int64_t i, int ex, int flag) const {
+        if (!flag) return;
+        ukeys[ex] = v[i] >> CT_CNT_BITS;
+        hpos[ex] = (int)i;
+    }
+};
+struct PairCount {
+    const uint64_t *v;
+    __device__ int operator()(int64_t i) const { return (int)(v[i] & ((1 << CT_CNT_BITS) - 1)); }
+};
+struct PairBefore {
+    int32_t *before;
+    int64_t n;
+    __device__ void operator()(int64_t i, int ex, int c) const {
+        before[i] = ex;
+        if (i == n - 1) before[n] = ex + c;
+    }
+};
+__global__ void k_run_links(int U, int64_t V, const int32_t *hpos, const int32_t *before, int32_t *links) {
+    for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < U; u += gridDim.x * blockDim.x)
+        links[u] = before[u + 1 < U ? hpos[u + 1] : V] - before[hpos[u]];
+}
+
+// Distinct labels expected among a tile's entries (x 1024) if neighbours fell
+// into communities by volume: few where some communities are large.
+__global__ __launch_bounds__(256) void k_tile_labels(const CommStats *st, int k, double per_entry,
+                                                     unsigned long long *acc) {
+    __shared__ long long part[256 / WAVE];
+    long long a = 0;
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += gridDim.x * blockDim.x)
+        a += (long long)(1024.0 * (1.0 - exp(-(double)CT_TILE * per_entry * ((double)st[c].int_vol + st[c].ext_vol))));
+    a = wave_sum64(a);
+    if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = a;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(acc, (unsigned long long)(part[0] + part[1] + part[2] + part[3]));
+}
+
+// The sorted unique pairs through community rows.  The sort moves the tiles'
+// pairs instead of every entry: worth it where most entries of a tile repeat
+// a pair of it.  Partitions of hub neighbourhoods, R-MAT-18 and -20 (0.10 and
+// 0.39 M pairs of 7.6 and 31 M entries): 0.48 -> 0.33 and 1.42 -> 0.78 ms a
+// call.  Partitions at random into 1,900 to 440,000 communities would take
+// 10-25 % longer by rows; k_tile_labels tells them apart, for 0.02 ms (0.45 ->
+// 0.47 ms at R-MAT-18).  Graphs below 2^22 entries (tunable contract_rows_min)
+// gain nothing: 0.16 -> 0.19 ms at R-MAT-14.
+constexpr int CT_MAX_LABELS = CT_TILE / 4;
+static int reserve_pair_rows(pcd_ctx *ctx) {
+    const size_t E = (size_t)2 * ctx->m, n = (size_t)ctx->n;
+    if (!ctx->mrows) ctx->mrows = new MergeRows();
+    MergeRows &R = *static_cast<MergeRows *>(ctx->mrows);
+    PCD_TRY(R.ent.reserve(ctx, E + 1));
+    PCD_TRY(R.cind.reserve(ctx, n + 3));
+    PCD_TRY(R.next.reserve(ctx, n + 3));
+    PCD_TRY(R.dst.reserve(ctx, n + 2));
+    return PCD_OK;
+}
+
+static int build_pairs_by_rows(pcd_ctx *ctx, int64_t *U_out) {
+    const int64_t E = (int64_t)2 * ctx->m;
+    const int k = ctx->k, half = label_bits(k);
+    MergeRows &R = *static_cast<MergeRows *>(ctx->mrows);
+    kt_begin(ctx, KS_MERGE_KEYS);
+    PCD_TRY(fill_rows(ctx, R, k, nullptr));
+    unsigned long long *nout = (unsigned long long *)ctx->d_acc;
+    PCD_TRY(fill_u64(ctx, (uint64_t *)nout, 0, 1));
+    hipLaunchKernelGGL(k_row_pairs, dim3(grid_for(ctx, E, CT_TILE, 3)), dim3(CT_NT), 0, ctx->stream, E, k, half,
+                       R.cind.p, R.ent.p, ctx->d_keys0, nout);
+    kt_end(ctx, KS_MERGE_KEYS);
+    PCD_HIP(hipGetLastError());
+    PCD_HIP(hipMemcpyAsync(ctx->h_small64, nout, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+    PCD_HIP(hipStreamSynchronize(ctx->stream));
+    const int64_t V = ctx->h_small64[0];
+    *U_out = 0;
+    if (V == 0) return PCD_OK;
+    uint64_t *sorted = nullptr;
+    kt_begin(ctx, KS_MERGE_SORT);
+    PCD_TRY(radix_sort_bits_u64(ctx, ctx->d_keys0, ctx->d_keys1, V, CT_CNT_BITS, CT_CNT_BITS + 2 * half, &sorted));
+    kt_end(ctx, KS_MERGE_SORT);
+    uint64_t *ukeys = sorted == ctx->d_keys0 ? ctx->d_keys1 : ctx->d_keys0;
+    int32_t *total = nullptr;
+    kt_begin(ctx, KS_MERGE_RLE);
+    // the rows' entries are done with: their buffer holds the counts before
+    PCD_TRY(device_scan(ctx, V, PairCount{sorted}, PairBefore{R.ent.p, V}, nullptr));
+    PCD_TRY(device_scan(ctx, V, PairHead{sorted}, PairKey{sorted, ukeys, ctx->d_pair_head}, &total));
+    PCD_HIP(hipMemcpyAsync(ctx->h_small, total, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    PCD_HIP(hipStreamSynchronize(ctx->stream));
+    *U_out = ctx->h_small[0];
+    hipLaunchKernelGGL(k_run_links, dim3(grid_for(ctx, *U_out, 256)), dim3(256), 0, ctx->stream, (int)*U_out, V,
+                       ctx->d_pair_head, R.ent.p, ctx->d_pair_links);
+    kt_end(ctx, KS_MERGE_RLE);
+    PCD_HIP(hipGetLastError());
+    if (ukeys != ctx->d_keys1)
+        PCD_HIP(hipMemcpyAsync(ctx->d_keys1, ukeys, *U_out * sizeof(uint64_t), hipMemcpyDeviceToDevice, ctx->stream));
+    return PCD_OK;
+}
+
 int contract_dev(pcd_ctx *ctx, int64_t *num_pairs) {
     int64_t U = 0;
     int half = 0;
-    PCD_TRY(build_pairs(ctx, &U, &half));
+    PCD_TRY(reserve_pairs(ctx));
+    const int64_t E = (int64_t)2 * ctx->m;
+    // a pair and its count share a 64-bit word, and a tile's end is an int
+    bool rows = !ctx->tune.onesweep && E >= ctx->tune.contract_rows_min && E > 0 && E <= INT32_MAX - CT_TILE &&
+                ctx->k > 0 && 2 * label_bits(ctx->k) + CT_CNT_BITS <= 64;
+    if (rows) {
+        unsigned long long *acc = (unsigned long long *)ctx->d_acc;
+        PCD_TRY(fill_u64(ctx, (uint64_t *)acc, 0, 1));
+        hipLaunchKernelGGL(k_tile_labels, dim3(grid_for(ctx, ctx->k, 256, 1)), dim3(256), 0, ctx->stream, ctx->d_stats,
+                           ctx->k, 1.0 / (double)E, acc);
+        PCD_HIP(hipGetLastError());
+        PCD_HIP(hipMemcpyAsync(ctx->h_small64, acc, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+        PCD_HIP(hipStreamSynchronize(ctx->stream));
+        // the rows take 4 bytes per entry more: without that memory, the sort
+        rows = ctx->h_small64[0] / 1024 <= CT_MAX_LABELS && reserve_pair_rows(ctx) == PCD_OK;
+    }
+    if (rows)
+        PCD_TRY(build_pairs_by_rows(ctx, &U));
+    else
+        PCD_TRY(build_pairs(ctx, &U, &half));
     *num_pairs = U;
     return PCD_OK;
 }

@@ -475,4 +475,11 @@ int radix_sort_u64(pcd_ctx *ctx, uint64_t *keys, uint64_t *tmp, int64_t n, int b
     return PCD_OK;
 }
 
+// the same on the bits [shift, bits) alone, which may start anywhere
+int radix_sort_bits_u64(pcd_ctx *ctx, uint64_t *keys, uint64_t *tmp, int64_t n, int shift, int bits, uint64_t **out) {
+    *out = keys;
+    if (n <= 1) return PCD_OK;
+    return lsd_passes(ctx, keys, tmp, n, shift, bits, out);
+}
+
 }  // namespace pcd

@@ -262,3 +262,33 @@ def test_noalloc_compression_sizes(ctx, n):
         assert np.array_equal(got[:n], want)
     for p in (d, out, k_dev):
         hip.ok(hip.h.hipFree(p))
+
+
+@pytest.mark.parametrize("kind", ["one", "half", "table", "seven_new", "planted", "sparse_ids"])
+@pytest.mark.parametrize("graph", ["bin_zoo", "unsorted", "rmat12", "ring", "one_tile", "past_a_tile"])
+def test_contraction_by_rows(ctx, graph, kind):
+    """Pairs counted over community rows in tiles equal the oracle's: few large
+    rows, rows that cross tiles, empty rows (ids in use with gaps), and both
+    sides of the row length from which the rows are used."""
+    ring = lambda n: GG.csr_direct(n, [(i, (i + 1) % n) for i in range(n)])  # 2n entries
+    g = {"bin_zoo": GG.bin_zoo, "unsorted": lambda: GG.unsorted_copy(GG.bin_zoo()), "rmat12": lambda: GG.rmat(12),
+         "ring": lambda: ring(5000), "one_tile": lambda: ring(1024), "past_a_tile": lambda: ring(1025)}[graph]()
+    n, m, ind, adj = g[:4]
+    if kind == "planted":
+        lab = (np.arange(n) * 40 // n).astype(np.int32)
+    elif kind == "sparse_ids":
+        lab = (np.arange(n) % 61 * (n // 64)).astype(np.int32)  # not compressed: empty rows between
+    else:
+        lab = crowded(kind, n)
+    ctx.upload_graph(n, m, ind, adj)
+    ctx.upload_labels(lab)
+    if kind != "sparse_ids":
+        ctx.compress()
+        lab = ctx.labels()
+    k = ctx.statistics()
+    ctx.set_tuning("contract_rows_min", 0)
+    got = ctx.contract()
+    ctx.set_tuning("contract_rows_min", 1 << 22)
+    want = O.community_pairs(n, ind, adj, lab, k)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y), (graph, kind)
