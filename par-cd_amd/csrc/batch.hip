@@ -40,23 +40,11 @@ namespace pcd {
 
 constexpr int VT = 2048;  // vertices per tile item
 constexpr int ROWS_PER = 64;  // row positions per long-row item (one per lane of the update kernel)
-static_assert(ROWS_PER == WAVE, "k_b_delta_rows checks one row per lane");
+static_assert(ROWS_PER == WAVE, "delta_rows_item checks one row per lane");
 constexpr int STAT_G[5] = {64, 32, 16, 8, 4};
 constexpr int STAT_CP[5] = {8, 16, 32, 64, 64};
 
 // --------------------------------------------------------------- kernels
-__global__ __launch_bounds__(256) void k_b_fill_first(const WorkItem *tiles, const int *count, const BatchGraph *gs,
-                                                      const BatchState *st) {
-    const int nt = *count;
-    for (int u = blockIdx.x; u < nt; u += gridDim.x) {
-        const WorkItem w = tiles[u];
-        if (st[w.g].status != BG_RUNNING) continue;
-        const int hi = min(w.p1, st[w.g].label_bound);
-        int32_t *first = gs[w.g].first;
-        for (int v = w.p0 + (int)threadIdx.x; v < hi; v += blockDim.x) first[v] = INT32_MAX;
-    }
-}
-
 __global__ __launch_bounds__(256) void k_b_first_occurrence(const WorkItem *tiles, const int *count,
                                                             const BatchGraph *gs, const BatchState *st) {
     const int nt = *count;
@@ -163,6 +151,9 @@ __global__ __launch_bounds__(256) void k_b_tile_apply(const WorkItem *tiles, con
     }
 }
 
+// The labels of this round into cur and next (propagation then writes the
+// active vertices only), and the records at their ids: renumbered ones back
+// into place, or cleared for the full count of a graph's first round.
 __global__ __launch_bounds__(256) void k_b_relabel(const WorkItem *tiles, const int *count, const BatchGraph *gs,
                                                    const BatchState *st) {
     const int nt = *count;
@@ -171,104 +162,65 @@ __global__ __launch_bounds__(256) void k_b_relabel(const WorkItem *tiles, const 
         if (st[w.g].status != BG_RUNNING) continue;
         const BatchGraph &g = gs[w.g];
         for (int v = w.p0 + (int)threadIdx.x; v < w.p1; v += blockDim.x) {
-            int l = g.next[v];
-            if (l >= 0) g.cur[v] = g.newid[l];
+            const int l = g.next[v];
+            const int id = l >= 0 ? g.newid[l] : g.cur[v];
+            if (l >= 0) g.cur[v] = id;
+            g.next[v] = id;
         }
-    }
-}
-
-// renumbered statistics back into place (graphs whose statistics follow
-// the labels)
-__global__ __launch_bounds__(256) void k_b_stats_copy(const WorkItem *tiles, const int *count, const BatchGraph *gs,
-                                                      const BatchState *st) {
-    const int nt = *count;
-    for (int u = blockIdx.x; u < nt; u += gridDim.x) {
-        const WorkItem w = tiles[u];
-        if (st[w.g].status != BG_RUNNING || !st[w.g].ready) continue;
+        const bool ready = st[w.g].ready != 0;
         const int hi = min(w.p1, st[w.g].k);
-        const BatchGraph &g = gs[w.g];
-        for (int c = w.p0 + (int)threadIdx.x; c < hi; c += blockDim.x) g.stats[c] = g.stats_alt[c];
-    }
-}
-
-// The full count runs in a graph's first round only
-__global__ __launch_bounds__(256) void k_b_clear_stats(const WorkItem *tiles, const int *count, const BatchGraph *gs,
-                                                       const BatchState *st) {
-    const int nt = *count;
-    for (int u = blockIdx.x; u < nt; u += gridDim.x) {
-        const WorkItem w = tiles[u];
-        if (st[w.g].status != BG_RUNNING || st[w.g].ready) continue;
-        const int hi = min(w.p1, st[w.g].k);
-        CommStats *s = gs[w.g].stats;
-        for (int c = w.p0 + (int)threadIdx.x; c < hi; c += blockDim.x) s[c] = CommStats{0, 0, 0, 0};
+        for (int c = w.p0 + (int)threadIdx.x; c < hi; c += blockDim.x)
+            g.stats[c] = ready ? g.stats_alt[c] : CommStats{0, 0, 0, 0};
     }
 }
 
 // framework.cpp:69-143 over rows of degree <= G: G lanes per vertex
 template <int G>
-__global__ __launch_bounds__(256) void k_b_stats_small(const WorkItem *items, const int *count, const BatchGraph *gs,
-                                                       const BatchState *st) {
+__device__ inline void stats_small_item(const WorkItem &w, const BatchGraph &g) {
     const int lane = __lane_id(), glane = lane & (G - 1);
     constexpr int per_wave = WAVE / G;
-    const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int nu = *count;
-    for (int u = wave_g; u < nu; u += nwaves) {
-        const WorkItem w = items[u];
-        if (st[w.g].status != BG_RUNNING || st[w.g].ready) continue;
-        const BatchGraph &g = gs[w.g];
-        const LPArgs &a = g.lp;
-        for (int base = w.p0; base < w.p1; base += per_wave) {
-            int p = base + lane / G;
-            bool has = p < w.p1;
-            int v = 0, start = 0, deg = 0, l = 0;
-            if (has) {
-                v = a.order ? a.order[p] : p;
-                start = a.indices[v];
-                deg = a.indices[v + 1] - start;
-                l = g.cur[v];
-            }
-            int same = 0;
-            for (int j = glane; j < deg; j += G) same += (g.cur[a.adj[start + j]] == l) ? 1 : 0;
-#pragma unroll
-            for (int d = G / 2; d > 0; d >>= 1) same += __shfl_xor(same, d, WAVE);
-            if (has && glane == 0) add_stats(g.stats, l, 1, same, deg - same);
+    const LPArgs &a = g.lp;
+    for (int base = w.p0; base < w.p1; base += per_wave) {
+        int p = base + lane / G;
+        bool has = p < w.p1;
+        int v = 0, start = 0, deg = 0, l = 0;
+        if (has) {
+            v = a.order ? a.order[p] : p;
+            start = a.indices[v];
+            deg = a.indices[v + 1] - start;
+            l = g.cur[v];
         }
+        int same = 0;
+        for (int j = glane; j < deg; j += G) same += (g.cur[a.adj[start + j]] == l) ? 1 : 0;
+#pragma unroll
+        for (int d = G / 2; d > 0; d >>= 1) same += __shfl_xor(same, d, WAVE);
+        if (has && glane == 0) add_stats(g.stats, l, 1, same, deg - same);
     }
 }
 
 // rows of degree > 64 (at most 4096 entries in a batch): one wave per item
 // of up to ROWS_PER row positions, row after row
-__global__ __launch_bounds__(256) void k_b_stats_rows(const WorkItem *items, const int *count, const BatchGraph *gs,
-                                                      const BatchState *st) {
+__device__ inline void stats_rows_item(const WorkItem &w, const BatchGraph &g) {
     constexpr int PF = 8;
     const int lane = __lane_id();
-    const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int nu = *count;
-    for (int u = wave_g; u < nu; u += nwaves) {
-        const WorkItem w = items[u];
-        if (st[w.g].status != BG_RUNNING || st[w.g].ready) continue;
-        const BatchGraph &g = gs[w.g];
-        const LPArgs &a = g.lp;
-        for (int p = w.p0; p < w.p1; p++) {
-            const int v = a.order ? a.order[p] : p;
-            const int l = g.cur[v];
-            const int b = a.indices[v], e = a.indices[v + 1];
-            int same = 0;
-            for (int j0 = b + lane; j0 < e; j0 += PF * WAVE) {
-                int nb[PF];
+    const LPArgs &a = g.lp;
+    for (int p = w.p0; p < w.p1; p++) {
+        const int v = a.order ? a.order[p] : p;
+        const int l = g.cur[v];
+        const int b = a.indices[v], e = a.indices[v + 1];
+        int same = 0;
+        for (int j0 = b + lane; j0 < e; j0 += PF * WAVE) {
+            int nb[PF];
 #pragma unroll
-                for (int k = 0; k < PF; k++) {
-                    const int j = j0 + k * WAVE;
-                    nb[k] = j < e ? a.adj[j] : -1;
-                }
-#pragma unroll
-                for (int k = 0; k < PF; k++) same += (nb[k] >= 0 && g.cur[nb[k]] == l) ? 1 : 0;
+            for (int k = 0; k < PF; k++) {
+                const int j = j0 + k * WAVE;
+                nb[k] = j < e ? a.adj[j] : -1;
             }
-            same = wave_sum(same);
-            if (lane == 0) add_stats(g.stats, l, 1, same, (e - b) - same);
+#pragma unroll
+            for (int k = 0; k < PF; k++) same += (nb[k] >= 0 && g.cur[nb[k]] == l) ? 1 : 0;
         }
+        same = wave_sum(same);
+        if (lane == 0) add_stats(g.stats, l, 1, same, (e - b) - same);
     }
 }
 
@@ -280,115 +232,164 @@ __global__ __launch_bounds__(256) void k_b_stats_rows(const WorkItem *items, con
 
 // rows of degree <= G: G lanes per vertex; unmoved vertices read no row
 template <int G>
-__global__ __launch_bounds__(256) void k_b_delta_small(const WorkItem *items, const int *count, const BatchGraph *gs,
-                                                       const BatchState *st) {
+__device__ inline void delta_small_item(const WorkItem &w, const BatchGraph &g) {
     const int lane = __lane_id(), glane = lane & (G - 1);
     constexpr int per_wave = WAVE / G;
-    const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int nu = *count;
-    for (int u = wave_g; u < nu; u += nwaves) {
-        const WorkItem w = items[u];
-        if (st[w.g].status != BG_RUNNING || !st[w.g].ready) continue;
-        const BatchGraph &g = gs[w.g];
-        const LPArgs &a = g.lp;
-        for (int base = w.p0; base < w.p1; base += per_wave) {
-            const int p = base + lane / G;
-            int start = 0, deg = 0, lo = 0, ln = 0;
-            bool moved = false;
-            if (p < w.p1) {
-                const int v = a.order ? a.order[p] : p;
-                lo = g.cur[v];
-                ln = g.next[v];
-                moved = lo != ln;
-                if (moved) {
-                    start = a.indices[v];
-                    deg = a.indices[v + 1] - start;
-                }
+    const LPArgs &a = g.lp;
+    for (int base = w.p0; base < w.p1; base += per_wave) {
+        const int p = base + lane / G;
+        int start = 0, deg = 0, lo = 0, ln = 0;
+        bool moved = false;
+        if (p < w.p1) {
+            const int v = a.order ? a.order[p] : p;
+            lo = g.cur[v];
+            ln = g.next[v];
+            moved = lo != ln;
+            if (moved) {
+                start = a.indices[v];
+                deg = a.indices[v + 1] - start;
             }
-            if (!__ballot(moved)) continue;
-            int sa = 0, sb = 0;
-            for (int j = glane; j < deg; j += G) {
-                const int x = a.adj[start + j];
-                const int lx = g.cur[x], nx = g.next[x];
-                const int f = lx != nx ? 1 : 2;
-                sa += lx == lo ? f : 0;
-                sb += nx == ln ? f : 0;
-            }
+        }
+        if (!__ballot(moved)) continue;
+        int sa = 0, sb = 0;
+        for (int j = glane; j < deg; j += G) {
+            const int x = a.adj[start + j];
+            const int lx = g.cur[x], nx = g.next[x];
+            const int f = lx != nx ? 1 : 2;
+            sa += lx == lo ? f : 0;
+            sb += nx == ln ? f : 0;
+        }
 #pragma unroll
-            for (int d = G / 2; d > 0; d >>= 1) {
-                sa += __shfl_xor(sa, d, WAVE);
-                sb += __shfl_xor(sb, d, WAVE);
-            }
-            if (moved && glane == 0) {
-                add_stats(g.stats, lo, -1, -sa, sa - deg);
-                if (ln >= 0) add_stats(g.stats, ln, 1, sb, deg - sb);
-            }
+        for (int d = G / 2; d > 0; d >>= 1) {
+            sa += __shfl_xor(sa, d, WAVE);
+            sb += __shfl_xor(sb, d, WAVE);
+        }
+        if (moved && glane == 0) {
+            add_stats(g.stats, lo, -1, -sa, sa - deg);
+            if (ln >= 0) add_stats(g.stats, ln, 1, sb, deg - sb);
         }
     }
 }
 
 // rows of degree > 64: one wave per item of up to ROWS_PER (= 64) row
 // positions; lane j checks row p0 + j, then the wave runs the moved rows
-__global__ __launch_bounds__(256) void k_b_delta_rows(const WorkItem *items, const int *count, const BatchGraph *gs,
-                                                      const BatchState *st) {
+__device__ inline void delta_rows_item(const WorkItem &w, const BatchGraph &g) {
     constexpr int PF = 4;
     const int lane = __lane_id();
-    const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
-    const int nwaves = gridDim.x * blockDim.x / WAVE;
-    const int nu = *count;
-    for (int u = wave_g; u < nu; u += nwaves) {
-        const WorkItem w = items[u];
-        if (st[w.g].status != BG_RUNNING || !st[w.g].ready) continue;
-        const BatchGraph &g = gs[w.g];
-        const LPArgs &a = g.lp;
-        int v = 0, lo = 0, ln = 0;
-        bool moved = false;
-        if (w.p0 + lane < w.p1) {
-            const int p = w.p0 + lane;
-            v = a.order ? a.order[p] : p;
-            lo = g.cur[v];
-            ln = g.next[v];
-            moved = lo != ln;
+    const LPArgs &a = g.lp;
+    int v = 0, lo = 0, ln = 0;
+    bool moved = false;
+    if (w.p0 + lane < w.p1) {
+        const int p = w.p0 + lane;
+        v = a.order ? a.order[p] : p;
+        lo = g.cur[v];
+        ln = g.next[v];
+        moved = lo != ln;
+    }
+    uint64_t mv = __ballot(moved);
+    while (mv) {
+        const int src = __builtin_ctzll(mv);
+        mv &= mv - 1;
+        const int xv = __builtin_amdgcn_readlane(v, src);
+        const int xlo = __builtin_amdgcn_readlane(lo, src), xln = __builtin_amdgcn_readlane(ln, src);
+        const int xb = a.indices[xv], xe = a.indices[xv + 1];
+        int sa = 0, sb = 0;
+        for (int j0 = xb + lane; j0 < xe; j0 += PF * WAVE) {
+            int nb[PF];
+#pragma unroll
+            for (int k = 0; k < PF; k++) {
+                const int j = j0 + k * WAVE;
+                nb[k] = j < xe ? a.adj[j] : -1;
+            }
+            int lx[PF], nx[PF];
+#pragma unroll
+            for (int k = 0; k < PF; k++) {
+                lx[k] = nb[k] < 0 ? -2 : g.cur[nb[k]];
+                nx[k] = nb[k] < 0 ? -2 : g.next[nb[k]];
+            }
+#pragma unroll
+            for (int k = 0; k < PF; k++) {
+                if (nb[k] < 0) continue;
+                const int f = lx[k] != nx[k] ? 1 : 2;
+                sa += lx[k] == xlo ? f : 0;
+                sb += nx[k] == xln ? f : 0;
+            }
         }
-        uint64_t mv = __ballot(moved);
-        while (mv) {
-            const int src = __builtin_ctzll(mv);
-            mv &= mv - 1;
-            const int xv = __builtin_amdgcn_readlane(v, src);
-            const int xlo = __builtin_amdgcn_readlane(lo, src), xln = __builtin_amdgcn_readlane(ln, src);
-            const int xb = a.indices[xv], xe = a.indices[xv + 1];
-            int sa = 0, sb = 0;
-            for (int j0 = xb + lane; j0 < xe; j0 += PF * WAVE) {
-                int nb[PF];
-#pragma unroll
-                for (int k = 0; k < PF; k++) {
-                    const int j = j0 + k * WAVE;
-                    nb[k] = j < xe ? a.adj[j] : -1;
-                }
-                int lx[PF], nx[PF];
-#pragma unroll
-                for (int k = 0; k < PF; k++) {
-                    lx[k] = nb[k] < 0 ? -2 : g.cur[nb[k]];
-                    nx[k] = nb[k] < 0 ? -2 : g.next[nb[k]];
-                }
-#pragma unroll
-                for (int k = 0; k < PF; k++) {
-                    if (nb[k] < 0) continue;
-                    const int f = lx[k] != nx[k] ? 1 : 2;
-                    sa += lx[k] == xlo ? f : 0;
-                    sb += nx[k] == xln ? f : 0;
-                }
-            }
-            sa = wave_sum(sa);
-            sb = wave_sum(sb);
-            if (lane == 0) {
-                const int len = xe - xb;
-                add_stats(g.stats, xlo, -1, -sa, sa - len);
-                if (xln >= 0) add_stats(g.stats, xln, 1, sb, len - sb);
-            }
+        sa = wave_sum(sa);
+        sb = wave_sum(sb);
+        if (lane == 0) {
+            const int len = xe - xb;
+            add_stats(g.stats, xlo, -1, -sa, sa - len);
+            if (xln >= 0) add_stats(g.stats, xln, 1, sb, len - sb);
         }
     }
+}
+
+// One launch over the five short-row lists and the long rows: f(i, item) for
+// every item of list i, one wave each.  The lists follow one another over the
+// waves, so that short lists do not all fall to the first ones.  A round of
+// small graphs is bound by its launches: six row lists in one launch twice, the
+// four passes over the vertices after the scan in one, and the first-occurrence
+// fill beside the update take 14 of 32 away.  256 block-model graphs of 50 to
+// 20,000 vertices, admission and results included: 63.4 -> 57.4 ms.
+struct RowLists {
+    const WorkItem *items[6];
+    const int *counts;
+};
+template <class F>
+__device__ inline void for_row_items(const RowLists &l, F f) {
+    const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
+    const int nwaves = gridDim.x * blockDim.x / WAVE;
+    int at = 0;  // the wave that takes the list's first item
+#pragma unroll
+    for (int i = 5; i >= 0; i--) {  // long rows first
+        const int nu = l.counts[i];
+        const WorkItem *items = l.items[i];
+        for (int u = wave_g >= at ? wave_g - at : wave_g - at + nwaves; u < nu; u += nwaves) f(i, items[u]);
+        at = (int)(((int64_t)at + nu) % nwaves);
+    }
+}
+
+// Update of the statistics after the last round's propagation step, and the
+// first-occurrence table made ready for this round's labels.
+__global__ __launch_bounds__(256) void k_b_delta(RowLists l, const WorkItem *tiles, const int *ntile,
+                                                 const BatchGraph *gs, const BatchState *st) {
+    const int nt = *ntile;
+    for (int u = blockIdx.x; u < nt; u += gridDim.x) {
+        const WorkItem w = tiles[u];
+        if (st[w.g].status != BG_RUNNING) continue;
+        const int hi = min(w.p1, st[w.g].label_bound);
+        int32_t *first = gs[w.g].first;
+        for (int v = w.p0 + (int)threadIdx.x; v < hi; v += blockDim.x) first[v] = INT32_MAX;
+    }
+    for_row_items(l, [&](int i, const WorkItem &w) {
+        if (st[w.g].status != BG_RUNNING || !st[w.g].ready) return;
+        const BatchGraph &g = gs[w.g];
+        switch (i) {
+        case 0: delta_small_item<64>(w, g); break;
+        case 1: delta_small_item<32>(w, g); break;
+        case 2: delta_small_item<16>(w, g); break;
+        case 3: delta_small_item<8>(w, g); break;
+        case 4: delta_small_item<4>(w, g); break;
+        default: delta_rows_item(w, g);
+        }
+    });
+}
+
+// The full count, of the graphs in their first round.
+__global__ __launch_bounds__(256) void k_b_stats(RowLists l, const BatchGraph *gs, const BatchState *st) {
+    for_row_items(l, [&](int i, const WorkItem &w) {
+        if (st[w.g].status != BG_RUNNING || st[w.g].ready) return;
+        const BatchGraph &g = gs[w.g];
+        switch (i) {
+        case 0: stats_small_item<64>(w, g); break;
+        case 1: stats_small_item<32>(w, g); break;
+        case 2: stats_small_item<16>(w, g); break;
+        case 3: stats_small_item<8>(w, g); break;
+        case 4: stats_small_item<4>(w, g); break;
+        default: stats_rows_item(w, g);
+        }
+    });
 }
 
 // exact int64 sums of int_volume, volume^2 and size*(size-1) per graph
@@ -422,19 +423,6 @@ __global__ __launch_bounds__(256) void k_b_metric(const WorkItem *tiles, const i
             atomicAdd(&st[w.g].acc[threadIdx.x], (unsigned long long)t);
         }
         __syncthreads();
-    }
-}
-
-// next = cur for the graphs still running: propagation then writes the
-// active vertices only
-__global__ __launch_bounds__(256) void k_b_copy_next(const WorkItem *tiles, const int *count, const BatchGraph *gs,
-                                                     const BatchState *st) {
-    const int nt = *count;
-    for (int u = blockIdx.x; u < nt; u += gridDim.x) {
-        const WorkItem w = tiles[u];
-        if (st[w.g].status != BG_RUNNING) continue;
-        const BatchGraph &g = gs[w.g];
-        for (int v = w.p0 + (int)threadIdx.x; v < w.p1; v += blockDim.x) g.next[v] = g.cur[v];
     }
 }
 
@@ -1919,46 +1907,25 @@ static int launch_round(pcd_batch *b) {
     const int *ntile = b->d_counts + L_TILES;
     const BatchGraph *gs = b->d_graphs;
     BatchState *st = b->d_state;
+    RowLists rows;
+    for (int i = 0; i < 6; i++) rows.items[i] = list_ptr<WorkItem>(b, L_SMALL0 + i);
+    rows.counts = b->d_counts + L_SMALL0;
     // statistics of the last round's propagation step (graphs past their
     // first round)
-    hipLaunchKernelGGL(k_b_delta_rows, dim3(cu * 8), dim3(256), 0, s, list_ptr<WorkItem>(b, L_ROWS),
-                       b->d_counts + L_ROWS, gs, st);
-#define PCD_BDELTA(I, G)                                                                                    \
-    hipLaunchKernelGGL(k_b_delta_small<G>, dim3(cu * 8), dim3(256), 0, s, list_ptr<WorkItem>(b, L_SMALL0 + I), \
-                       b->d_counts + L_SMALL0 + I, gs, st);
-    PCD_BDELTA(0, 64)
-    PCD_BDELTA(1, 32)
-    PCD_BDELTA(2, 16)
-    PCD_BDELTA(3, 8)
-    PCD_BDELTA(4, 4)
-#undef PCD_BDELTA
+    hipLaunchKernelGGL(k_b_delta, dim3(cu * 8), dim3(256), 0, s, rows, tiles, ntile, gs, st);
     // compress_labels (framework.cpp:146-170)
-    hipLaunchKernelGGL(k_b_fill_first, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
     hipLaunchKernelGGL(k_b_first_occurrence, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
     hipLaunchKernelGGL(k_b_tile_count, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st, b->d_tile_sum);
     hipLaunchKernelGGL(k_b_tile_scan, dim3(1), dim3(1024), 0, s, ntile, b->d_tile_sum, b->d_tile_pre);
     hipLaunchKernelGGL(k_b_tile_apply, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, b->d_gtiles, gs, st,
                        b->d_tile_sum, b->d_tile_pre);
     hipLaunchKernelGGL(k_b_relabel, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
-    hipLaunchKernelGGL(k_b_stats_copy, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
     // collect_statistics (framework.cpp:69-143) in a graph's first round
-    hipLaunchKernelGGL(k_b_clear_stats, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
-    hipLaunchKernelGGL(k_b_stats_rows, dim3(cu * 8), dim3(256), 0, s, list_ptr<WorkItem>(b, L_ROWS),
-                       b->d_counts + L_ROWS, gs, st);
-#define PCD_BSTATS(I, G)                                                                                    \
-    hipLaunchKernelGGL(k_b_stats_small<G>, dim3(cu * 8), dim3(256), 0, s, list_ptr<WorkItem>(b, L_SMALL0 + I), \
-                       b->d_counts + L_SMALL0 + I, gs, st);
-    PCD_BSTATS(0, 64)
-    PCD_BSTATS(1, 32)
-    PCD_BSTATS(2, 16)
-    PCD_BSTATS(3, 8)
-    PCD_BSTATS(4, 4)
-#undef PCD_BSTATS
+    hipLaunchKernelGGL(k_b_stats, dim3(cu * 8), dim3(256), 0, s, rows, gs, st);
     // Rule::calculate and the stop rule
     hipLaunchKernelGGL(k_b_metric, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
     hipLaunchKernelGGL(k_b_finalize, dim3((b->cap + 255) / 256), dim3(256), 0, s, gs, st, b->cap);
     // PropagationRefinement::refine for the graphs still running
-    hipLaunchKernelGGL(k_b_copy_next, dim3(cu * 4), dim3(256), 0, s, tiles, ntile, gs, st);
     PCD_TRY(batch_propagation_launch(s, lp_launch(b)));
     PCD_HIP(hipGetLastError());
     return PCD_OK;

@@ -292,3 +292,30 @@ def test_contraction_by_rows(ctx, graph, kind):
     want = O.community_pairs(n, ind, adj, lab, k)
     for x, y in zip(got, want):
         assert np.array_equal(x, y), (graph, kind)
+
+
+@pytest.mark.parametrize("cut", [1, 2, 3])
+def test_batch_rows_of_every_width(cut):
+    # one graph per row width at the edges of the short-row classes
+    graphs, jobs = [], []
+    for i, deg in enumerate([2, 4, 6, 8, 10, 16, 18, 32, 34, 64, 66, 130]):
+        n = 2 * deg + 3 + 97 * i
+        v = np.arange(n)
+        nb = np.sort(np.stack([(v + s * d) % n for d in range(1, deg // 2 + 1) for s in (1, -1)], 1), axis=1)
+        graphs.append((n, n * deg // 2, (np.arange(n + 1) * deg).astype(np.int32), nb.ravel().astype(np.int32)))
+        # graphs end in different rounds, so the lists hold finished ones too
+        jobs.append(parcd.job(kind=O.MOD, seed=i, max_iter=1 + (i + cut) % 4))
+    graphs.append(GG.rmat(10, seed=5)[:4])  # rows of up to a few hundred
+    jobs.append(parcd.job(kind=O.CPM, lam=0.01, seed=5, max_iter=5))
+    labels = [np.arange(x[0], dtype=np.int32) for x in graphs]
+    if cut == 3:
+        labels = [np.where(np.arange(x[0]) % 5 == 0, -1, np.arange(x[0]) % 11).astype(np.int32) for x in graphs]
+    with parcd.Batch(0, max_graphs=16, arena_bytes=256 << 20) as b:
+        slots = [b.add(*x, lab, jb) for x, lab, jb in zip(graphs, labels, jobs)]
+        while b.step(cut):
+            pass
+        got = [(b.labels(s),) + b.status(s)[1:] for s in slots]
+    for x, lab, jb, (bl, it, k, score) in zip(graphs, labels, jobs, got):
+        with parcd.Context(0) as c:
+            pl, ps, pit, pk = c.run(*x, lab, jb)
+        assert np.array_equal(bl, pl) and (it, k, score) == (pit, pk, ps)
