@@ -134,11 +134,11 @@ __device__ inline void tri_flush(const TriArgs &a, const int *hot) {
         if (hot[i]) atomicAdd(&a.tri[i], hot[i]);
 }
 
-// A wave looks at eight vertices at once, eight lanes each, and takes those
-// with at least two (same-label) neighbours below them one by one.  Rows
+// A wave looks at `per` vertices at once (eight, fewer where the graph has too
+// few vertices for all waves), eight lanes each, and takes those with at least two (same-label) neighbours below them one by one.  Rows
 // u are read 64 lanes wide, or four at a time 16 lanes wide where they are
 // short on average (Chung-Lu rows hold 30-60 entries, R-MAT rows 150-190).
-__global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a) {
+__global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a, int per) {
     __shared__ int s_keys[256 / WAVE][1 << TRI_WAVE_LOG], s_cnts[256 / WAVE][1 << TRI_WAVE_LOG];
     __shared__ int s_row[256 / WAVE][3][TRI_WAVE];
     __shared__ int hot[TRI_HOT];
@@ -150,9 +150,9 @@ __global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a) {
     int *rsu = s_row[w][0], *rlen = s_row[w][1], *rcnt = s_row[w][2];
     const int wave_g = (blockIdx.x * 256 + threadIdx.x) / WAVE;
     const int nwaves = gridDim.x * (256 / WAVE);
-    for (int64_t base = (int64_t)wave_g * 8; base < a.n; base += (int64_t)nwaves * 8) {
+    for (int64_t base = (int64_t)wave_g * per; base < a.n; base += (int64_t)nwaves * per) {
         const int vo = (int)min((int64_t)a.n - 1, base + lane / 8);
-        int plen = base + lane / 8 < a.n ? a.lowpos[vo] : 0;
+        int plen = lane / 8 < per && base + lane / 8 < a.n ? a.lowpos[vo] : 0;
         if (plen > TRI_WAVE) plen = 0;
         const int pstart = a.indices[vo], plab = a.labels ? a.labels[vo] : 0;
         int mine = plen;
@@ -230,7 +230,12 @@ __global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a) {
 
 // One workgroup per listed vertex: its prefix goes into the table in chunks,
 // and for each chunk the waves take the rows behind the chunk's first entry
-// (64 rows' extents loaded at once, one lane each).
+// (64 rows' extents loaded at once, one lane each).  Where the list is short,
+// up to TRI_PARTS workgroups share a vertex, each with its own table and a part
+// of the rows: the rows of one wave are a serial chain.  That and the smaller
+// units of k_triangles_wave, whole call: R-MAT-11 237 -> 97 us, R-MAT-13 332 ->
+// 166, R-MAT-15 435 -> 304, R-MAT-18 unchanged.
+constexpr int TRI_PARTS = 16;
 __global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
     constexpr int NT = 256, NW = NT / WAVE;
     __shared__ int keys[1 << TRI_BLOCK_LOG], cnts[1 << TRI_BLOCK_LOG];
@@ -238,8 +243,11 @@ __global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
     for (int i = threadIdx.x; i < TRI_HOT; i += NT) hot[i] = 0;
     const int lane = __lane_id(), w = threadIdx.x / WAVE;
     const int nlist = *a.listed;
-    for (int it = blockIdx.x; it < nlist; it += gridDim.x) {
-        const int v = a.list[it];
+    const int parts = nlist > 0 ? max(1, min(TRI_PARTS, (int)gridDim.x / nlist)) : 1;
+    const int64_t items = (int64_t)nlist * parts;
+    for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+        const int v = a.list[it / parts];
+        const int first = (int)(it % parts) * NW + w, step = parts * NW;  // this wave's rows
         const int sv = a.indices[v], len = a.lowpos[v], lab = a.labels ? a.labels[v] : 0;
         int tv = 0;
         for (int c0 = 0; c0 < len; c0 += TRI_CHUNK) {
@@ -255,9 +263,8 @@ __global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
                 if (!a.labels || a.labels[u] == lab) tri_insert(keys, log, u);
             }
             __syncthreads();
-            // wave w takes rows c0 + 1 + w, + NW, ...
-            for (int r0 = c0 + 1 + w; r0 < len; r0 += NW * WAVE) {
-                const int r = r0 + NW * lane;
+            for (int r0 = c0 + 1 + first; r0 < len; r0 += step * WAVE) {
+                const int r = r0 + step * lane;
                 int u = -1, su = 0, lu = 0;
                 if (r < len) {
                     u = a.adj[sv + r];
@@ -445,8 +452,11 @@ static int count_pass(pcd_ctx *ctx, const int32_t *labels, int32_t *t, int32_t *
     hipLaunchKernelGGL(k_tri_clear, dim3(grid_for(ctx, std::max<int64_t>(words, n), 256 * 4)), dim3(256), 0,
                        ctx->stream, words, (uint32_t *)ctx->d_tri_flag, n, t, td);
     // several rounds of workgroups: vertices differ a hundredfold in work
-    hipLaunchKernelGGL(k_triangles_block, dim3(ctx->cu_count * 24), dim3(256), 0, ctx->stream, a);
-    hipLaunchKernelGGL(k_triangles_wave, dim3(grid_for(ctx, n, 4 * 8, 24)), dim3(256), 0, ctx->stream, a);
+    const int64_t listed = std::min<int64_t>(n, E / (TRI_WAVE + 1)) + 1;  // at most
+    hipLaunchKernelGGL(k_triangles_block, dim3((int)std::min<int64_t>(ctx->cu_count * 24, listed * TRI_PARTS)), dim3(256),
+                       0, ctx->stream, a);
+    const int per = std::min(8, (n + ctx->cu_count * 32 - 1) / (ctx->cu_count * 32));
+    hipLaunchKernelGGL(k_triangles_wave, dim3(grid_for(ctx, n, 4 * per, 24)), dim3(256), 0, ctx->stream, a, per);
     hipLaunchKernelGGL(k_tri_degrees, dim3(grid_for(ctx, n, TDEG_NT / 8, 2)), dim3(TDEG_NT), 0, ctx->stream, a, td);
     kt_end(ctx, KS_TRIANGLES);
     PCD_HIP(hipGetLastError());
