@@ -904,7 +904,34 @@ int propagation_commit(pcd_ctx *ctx) {
 }
 
 // ------------------------------------------------------------- batches
-// One persistent launch per variant in use: a fixed grid whose waves or
+// The short-row lists of a batch in one launch: a wave takes its items of one
+// list after another, the lists laid one behind the other over the waves.
+// Rounds of small graphs are bound by their launches (256 block-model graphs of
+// 50 to 20,000 vertices: 57.9 -> 56.5 ms with four fewer a round).
+struct SmallItems {
+    ItemSrc src[5];  // LPV_S4 .. LPV_S64
+    bool used[5];
+};
+template <unsigned KM>
+__global__ __launch_bounds__(256) void k_lp_small_items(SmallItems si) {
+    __shared__ int s_list[256 / WAVE][WAVE];
+    const int nwaves = gridDim.x * blockDim.x / WAVE;
+    const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
+    int *list = s_list[threadIdx.x / WAVE];
+    int at = 0;  // the wave that takes the list's first item
+    auto next = [&](int i) {
+        const int w = wave_g >= at ? wave_g - at : wave_g - at + nwaves;
+        at = (int)(((int64_t)at + si.src[i].units()) % nwaves);
+        return w;
+    };
+    if (si.used[4]) lp_small<64, 8, false, KM>(si.src[4], next(4), nwaves, list);
+    if (si.used[3]) lp_small<32, 16, false, KM>(si.src[3], next(3), nwaves, list);
+    if (si.used[2]) lp_small<16, 32, false, KM>(si.src[2], next(2), nwaves, list);
+    if (si.used[1]) lp_small<8, 64, false, KM>(si.src[1], next(1), nwaves, list);
+    if (si.used[0]) lp_small<4, 64, false, KM>(si.src[0], next(0), nwaves, list);
+}
+
+// One persistent launch per variant in use, one for all short rows: a fixed grid whose waves or
 // workgroups stride over the variant's work items (the item count is read
 // on the device, so the launches can be captured once and replayed while
 // the lists change).  Small bins read labels and statistics (no records).
@@ -925,16 +952,15 @@ int batch_propagation_launch(hipStream_t stream, const BatchLPLaunch &l) {
                            src(LPV_W1024));
     if (l.used[LPV_W512])
         hipLaunchKernelGGL((k_lp_wave<512, RK_BATCH, ItemSrc>), dim3(cu * 8), dim3(256), 0, stream, src(LPV_W512));
-    if (l.used[LPV_S64])
-        hipLaunchKernelGGL((k_lp_small<64, 8, false, RK_BATCH, ItemSrc>), dim3(cu * 8), dim3(256), 0, stream, src(LPV_S64));
-    if (l.used[LPV_S32])
-        hipLaunchKernelGGL((k_lp_small<32, 16, false, RK_BATCH, ItemSrc>), dim3(cu * 8), dim3(256), 0, stream, src(LPV_S32));
-    if (l.used[LPV_S16])
-        hipLaunchKernelGGL((k_lp_small<16, 32, false, RK_BATCH, ItemSrc>), dim3(cu * 8), dim3(256), 0, stream, src(LPV_S16));
-    if (l.used[LPV_S8])
-        hipLaunchKernelGGL((k_lp_small<8, 64, false, RK_BATCH, ItemSrc>), dim3(cu * 8), dim3(256), 0, stream, src(LPV_S8));
-    if (l.used[LPV_S4])
-        hipLaunchKernelGGL((k_lp_small<4, 64, false, RK_BATCH, ItemSrc>), dim3(cu * 8), dim3(256), 0, stream, src(LPV_S4));
+    SmallItems si;
+    bool any = false;
+    for (int i = 0; i < 5; i++) {
+        si.src[i] = src(LPV_S4 + i);
+        si.used[i] = l.used[LPV_S4 + i];
+        any |= si.used[i];
+    }
+    if (any)
+        hipLaunchKernelGGL((k_lp_small_items<RK_BATCH>), dim3(cu * 8), dim3(256), 0, stream, si);
     PCD_HIP(hipGetLastError());
     return PCD_OK;
 }
