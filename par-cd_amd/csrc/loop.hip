@@ -30,6 +30,13 @@
 
 namespace pcd {
 
+// Edges from which the WCC metric is a branch of its own in the captured pass.
+// A pass with two branches costs more to capture and replay: whole runs on
+// Chung-Lu graphs of 3,000 vertices 2.19 ms with the branch and 1.40 without,
+// 20,000 vertices 2.28 and 1.95, 60,000 vertices (above the line) 2.84 and
+// 2.83-2.98, 200,000 vertices 3.89 and 4.30.
+constexpr int WCC_BESIDE_M = 1 << 18;
+
 __global__ void k_loop_rule(LoopState *s, const double *score, const int32_t *dk, LoopParams p) {
     loop_rule(s, *score, *dk, p);
 }
@@ -154,7 +161,7 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
         // as the propagation and neither reads the other: it runs beside it
         // on the metric stream, and a pass that turns out to be the last
         // drops its step (Chung-Lu, 1 M vertices: 0.27 of a pass's 0.72 ms).
-        const bool beside = kind == PASS_PROPAGATE && rule.kind == PCD_RULE_WCC && ctx->mstream && ctx->ev_mfork &&
+        const bool beside = kind == PASS_PROPAGATE && rule.kind == PCD_RULE_WCC && ctx->m >= WCC_BESIDE_M && ctx->mstream && ctx->ev_mfork &&
                             ctx->ev_metric;
         hipStream_t main_stream = ctx->stream;
         if (rc == PCD_OK && beside) {

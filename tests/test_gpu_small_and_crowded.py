@@ -319,3 +319,22 @@ def test_batch_rows_of_every_width(cut):
         with parcd.Context(0) as c:
             pl, ps, pit, pk = c.run(*x, lab, jb)
         assert np.array_equal(bl, pl) and (it, k, score) == (pit, pk, ps)
+
+
+@pytest.mark.parametrize("n", [200, 1025, 3001])
+def test_wcc_loop_of_a_small_graph(n):
+    # below 2^18 edges the captured pass holds the metric in line
+    rng = np.random.default_rng(n)
+    deg = 12
+    a = np.repeat(np.arange(n), deg)
+    g = GG.csr_from_edges(a, (a + rng.integers(1, 24, n * deg)) % n)
+    lab = (np.arange(g[0]) // 9).astype(np.int32)
+    res = []
+    for loop in (1, 0):
+        with parcd.Context(0) as c:
+            c.set_tuning("graph_loop", loop)
+            c.upload_graph(*g[:4])
+            c.triangles()
+            c.upload_labels(lab)
+            res.append(c.refine(parcd.job(kind=O.WCC, seed=3, max_iter=6)) + (c.labels(),))
+    assert np.array_equal(res[0][-1], res[1][-1]) and res[0][:-1] == res[1][:-1]
