@@ -67,21 +67,35 @@ static int pass_kind(int strategy, int it) {
     return it % 2 == 0 ? PASS_PROPAGATE : PASS_MERGE;
 }
 
-// The captured passes, their state and the buffers they were captured with.
+// What a captured pass depends on: the buffers, the tuning and the job.
+struct PassKey {
+    const void *ptrs[4] = {nullptr, nullptr, nullptr, nullptr};
+    int64_t alloc_gen = -1, tune_gen = -1;
+    pcd_rule rule{};
+    double cc = 0;  // clustering coefficient, which WCC's gains hold
+    double frac = 0, threshold = 0;
+    uint64_t seed = 0;
+    int tie = 0, max_iter = 0, cap = 0;
+    int rounds = 0;      // of a merging pass; 0 for a propagation pass
+    bool fused = false;  // a propagation pass in its fused form: no copy is kept
+
+    bool operator==(const PassKey &o) const {
+        return std::equal(ptrs, ptrs + 4, o.ptrs) && alloc_gen == o.alloc_gen && tune_gen == o.tune_gen &&
+               rule.kind == o.rule.kind && rule.lambda == o.rule.lambda && cc == o.cc && frac == o.frac &&
+               threshold == o.threshold && seed == o.seed && tie == o.tie && max_iter == o.max_iter && cap == o.cap && rounds == o.rounds &&
+               fused == o.fused;
+    }
+};
+
+// The captured passes, each with its own key (schedules -s 0, 1 and 2 share
+// the two slots, and a call recaptures only the kinds it replays), and their
+// state.
 struct Loop {
     hipGraphExec_t exec[2] = {nullptr, nullptr};  // by PassKind
+    PassKey key[2];
     LoopState *d_state = nullptr, *h_state = nullptr;
     int32_t *snap_labels = nullptr;
     CommStats *snap_stats = nullptr;
-    // what the capture depends on
-    const void *ptrs[4] = {nullptr, nullptr, nullptr, nullptr};
-    int64_t alloc_gen = -1;
-    int64_t tune_gen = -1;
-    pcd_rule rule{};
-    double frac = 0, threshold = 0;
-    uint64_t seed = 0;
-    int tie = 0, max_iter = 0, cap = 0, rounds = 0;
-    bool fused = false;   // the propagation pass is in its fused form: no copy is kept
     bool broken = false;  // capture failed once: this context runs pass by pass
 };
 
@@ -98,19 +112,40 @@ void loop_release(pcd_ctx *ctx) {
     ctx->loop = nullptr;
 }
 
-// whether the captured passes of `kinds` (bit per PassKind) were captured
-// for these buffers, tuning, job and merging rounds
-static bool same_key(const Loop *L, pcd_ctx *ctx, const pcd_job *job, int cap, int rounds, unsigned kinds, bool fused) {
-    if (L->fused != fused) return false;
+static PassKey pass_key(pcd_ctx *ctx, const pcd_job *job, int cap, int kind, int rounds, bool fused) {
+    PassKey k;
     const void *p[4] = {ctx->d_labels, ctx->d_labels_alt, ctx->d_stats, ctx->d_stats_alt};
-    for (int i = 0; i < 4; i++)
-        if (p[i] != L->ptrs[i]) return false;
-    for (int k = 0; k < 2; k++)
-        if (((kinds >> k) & 1) && !L->exec[k]) return false;
-    return L->alloc_gen == ctx->alloc_gen && L->tune_gen == ctx->tune_gen && L->rule.kind == job->rule.kind &&
-           L->rule.lambda == job->rule.lambda && L->frac == job->frac && L->threshold == job->threshold &&
-           L->seed == job->seed && L->tie == job->tie && L->max_iter == job->max_iter && L->cap == cap &&
-           (!((kinds >> PASS_MERGE) & 1) || L->rounds == rounds);
+    std::copy(p, p + 4, k.ptrs);
+    k.alloc_gen = ctx->alloc_gen;
+    k.tune_gen = ctx->tune_gen;
+    k.rule = job->rule;
+    k.cc = ctx->cc;
+    k.frac = job->frac;
+    k.threshold = job->threshold;
+    k.seed = job->seed;
+    k.tie = job->tie;
+    k.max_iter = job->max_iter;
+    k.cap = cap;
+    k.rounds = kind == PASS_MERGE ? rounds : 0;
+    k.fused = fused;
+    return k;
+}
+
+// Everything the passes of `kinds` (bit per PassKind) may otherwise allocate
+// lazily: no allocation may happen while the stream captures, nor between two
+// captures (it would make the first one's key stale).
+static int reserve_passes(pcd_ctx *ctx, Loop *L, unsigned kinds, bool fused) {
+    PCD_TRY(ensure_scan_parts(ctx, (int64_t)ctx->n + ctx->num_stat_items + 64));
+    if ((kinds >> PASS_MERGE) & 1) PCD_TRY(merge_rows_reserve(ctx));
+    if (!L->d_state) PCD_TRY(dev_alloc_t(ctx, &L->d_state, 1));
+    if (!L->h_state && hipHostMalloc((void **)&L->h_state, sizeof(LoopState), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        L->h_state = nullptr;
+        return fail(PCD_E_NOMEM, "pinned loop state");
+    }
+    if (!fused && !L->snap_labels) PCD_TRY(dev_alloc_t(ctx, &L->snap_labels, ctx->n + 1));
+    if (!fused && !L->snap_stats) PCD_TRY(dev_alloc_t(ctx, &L->snap_stats, ctx->n + 1));
+    return PCD_OK;
 }
 
 // Captures one pass of step kind `kind`.  Nothing runs: the host
@@ -122,18 +157,6 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
         (void)hipGraphExecDestroy(exec);
         exec = nullptr;
     }
-    // buffers the pass may grow lazily are sized first (no allocation may
-    // happen while the stream captures)
-    PCD_TRY(ensure_scan_parts(ctx, (int64_t)ctx->n + ctx->num_stat_items + 64));
-    if (kind == PASS_MERGE) PCD_TRY(merge_rows_reserve(ctx));
-    if (!L->d_state) PCD_TRY(dev_alloc_t(ctx, &L->d_state, 1));
-    if (!L->h_state && hipHostMalloc((void **)&L->h_state, sizeof(LoopState), hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        L->h_state = nullptr;
-        return fail(PCD_E_NOMEM, "pinned loop state");
-    }
-    if (!fused && !L->snap_labels) PCD_TRY(dev_alloc_t(ctx, &L->snap_labels, ctx->n + 1));
-    if (!fused && !L->snap_stats) PCD_TRY(dev_alloc_t(ctx, &L->snap_stats, ctx->n + 1));
     // host bookkeeping as it stands (a pass changes it while capturing)
     const bool s_timing = ctx->timing, s_counters = ctx->counters, s_comp = ctx->labels_compressed,
                s_has = ctx->has_stats, s_pend = ctx->stats_pending, s_new = ctx->labels_have_new,
@@ -219,24 +242,13 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
     }
     if (g) (void)hipGraphDestroy(g);
     if (rc != PCD_OK) return rc;
-    for (int i = 0; i < 4; i++) L->ptrs[i] = p0[i];
-    L->alloc_gen = ctx->alloc_gen;
-    L->tune_gen = ctx->tune_gen;
-    L->rule = rule;
-    L->frac = job->frac;
-    L->threshold = job->threshold;
-    L->seed = job->seed;
-    L->tie = job->tie;
-    L->max_iter = job->max_iter;
-    L->cap = cap;
-    L->fused = fused;
-    if (kind == PASS_MERGE) L->rounds = rounds;
+    L->key[kind] = pass_key(ctx, job, cap, kind, rounds, fused);
     return PCD_OK;
 }
 
 // Passes [it, it + count) on the device; see pcd_iterate_many.
-static int device_passes(pcd_ctx *ctx, Loop *L, const pcd_job *job, int strategy, int cap, int it, int count,
-                         double prev_score, int *passes, double *score, int *num_labels, int *done) {
+static int device_passes(pcd_ctx *ctx, Loop *L, int strategy, bool fused, int it, int count, double prev_score,
+                         int *passes, double *score, int *num_labels, int *done) {
     LoopState &h = *L->h_state;
     std::memset(&h, 0, sizeof(h));
     h.it = it;
@@ -245,7 +257,7 @@ static int device_passes(pcd_ctx *ctx, Loop *L, const pcd_job *job, int strategy
     h.prev = prev_score;
     h.prev_k = ctx->k;
     PCD_HIP(hipMemcpyAsync(L->d_state, &h, sizeof(LoopState), hipMemcpyHostToDevice, ctx->stream));
-    if (L->fused) PCD_TRY(fused_prepare(ctx));
+    if (fused) PCD_TRY(fused_prepare(ctx));
     // replays per read of the record: about half a millisecond of passes
     // (one pass at a time for large graphs), never beyond the first pass
     // that can freeze
@@ -266,12 +278,13 @@ static int device_passes(pcd_ctx *ctx, Loop *L, const pcd_job *job, int strategy
         per = std::max(1, std::min(32, (int)(0.5 / std::max(pass_ms, 1e-3))));
     }
     // the labels and statistics of the frozen pass back in place
-    if (!L->fused)
-      PCD_HIP(hipMemcpyAsync(ctx->d_labels, L->snap_labels, sizeof(int32_t) * (size_t)ctx->n, hipMemcpyDeviceToDevice,
-                           ctx->stream));
-    if (!L->fused && h.k_freeze > 0)
-        PCD_HIP(hipMemcpyAsync(ctx->d_stats, L->snap_stats, sizeof(CommStats) * (size_t)h.k_freeze,
+    if (!fused) {
+        PCD_HIP(hipMemcpyAsync(ctx->d_labels, L->snap_labels, sizeof(int32_t) * (size_t)ctx->n,
                                hipMemcpyDeviceToDevice, ctx->stream));
+        if (h.k_freeze > 0)
+            PCD_HIP(hipMemcpyAsync(ctx->d_stats, L->snap_stats, sizeof(CommStats) * (size_t)h.k_freeze,
+                                   hipMemcpyDeviceToDevice, ctx->stream));
+    }
     PCD_HIP(hipStreamSynchronize(ctx->stream));
     ctx->k = h.k_freeze;
     ctx->label_bound = h.k_freeze;
@@ -368,28 +381,27 @@ extern "C" int pcd_iterate_many(pcd_ctx *ctx, const pcd_job *job, int strategy, 
     Loop *L = loop_of(ctx);
     const bool fused = strategy == 0 && ctx->tune.fused_pass &&
                        (job->rule.kind == PCD_RULE_MODULARITY || job->rule.kind == PCD_RULE_CPM);
-    if (!same_key(L, ctx, job, cap, rounds, kinds, fused)) {
-        // everything a captured merging step uses is allocated first, so
-        // that neither capture allocates
-        int rc = (kinds & 2u) ? merge_rows_reserve(ctx) : PCD_OK;
-        for (int kd = 0; kd < 2 && rc == PCD_OK; kd++)
-            if ((kinds >> kd) & 1u) rc = capture_pass(ctx, L, job, cap, kd, rounds, fused);
-        if (rc != PCD_OK) {
-            // this context runs pass by pass from now on
-            L->broken = true;
-            int p2 = 0, d2 = 0, k2 = 0;
-            double s2 = 0.0;
-            PCD_TRY(pcd_iterate_many(ctx, job, strategy, rounds, it + run, count - run, prev, &p2, &s2, &k2, &d2));
-            *passes = run + p2;
-            *score = p2 ? s2 : *score;
-            *num_labels = p2 ? k2 : *num_labels;
-            *done = d2;
-            return PCD_OK;
-        }
+    int rc = reserve_passes(ctx, L, kinds, fused);
+    for (int kd = 0; kd < 2 && rc == PCD_OK; kd++) {
+        if (!((kinds >> kd) & 1u)) continue;
+        if (!L->exec[kd] || !(L->key[kd] == pass_key(ctx, job, cap, kd, rounds, fused)))
+            rc = capture_pass(ctx, L, job, cap, kd, rounds, fused);
+    }
+    if (rc != PCD_OK) {
+        // this context runs pass by pass from now on
+        L->broken = true;
+        int p2 = 0, d2 = 0, k2 = 0;
+        double s2 = 0.0;
+        PCD_TRY(pcd_iterate_many(ctx, job, strategy, rounds, it + run, count - run, prev, &p2, &s2, &k2, &d2));
+        *passes = run + p2;
+        *score = p2 ? s2 : *score;
+        *num_labels = p2 ? k2 : *num_labels;
+        *done = d2;
+        return PCD_OK;
     }
     int p2 = 0, d2 = 0, k2 = 0;
     double s2 = 0.0;
-    PCD_TRY(device_passes(ctx, L, job, strategy, cap, it + run, count - run, prev, &p2, &s2, &k2, &d2));
+    PCD_TRY(device_passes(ctx, L, strategy, fused, it + run, count - run, prev, &p2, &s2, &k2, &d2));
     if (kinds & 2u) PCD_TRY(merge_rows_check(ctx));
     *passes = run + p2;
     if (p2) {

@@ -247,3 +247,76 @@ def test_merging_pass_ranges_then_single_passes():
             prev = sa
             if da:
                 break
+
+
+def outcome(ctx, lab, jb, strategy, rounds):
+    ctx.upload_labels(lab)
+    score, it, k = ctx.refine(jb, strategy=strategy, rounds=rounds)
+    return [score, it, k, ctx.labels()] + list(ctx.stats(k))
+
+
+# Runs that follow one another on one context: each recaptures the kinds of
+# pass whose job, rounds or form differ from what the context holds, and no
+# others.  A job is an index into `jobs` below.
+SEQUENCES = {"schedules": [(0, 0, 1), (1, 0, 1), (2, 0, 1), (0, 0, 1), (2, 0, 1), (1, 0, 1), (0, 0, 1)],
+             "jobs": [(2, 0, 1), (1, 1, 1), (2, 1, 1), (0, 0, 1), (2, 0, 1)],
+             "rounds": [(2, 0, 1), (1, 0, 3), (2, 0, 3), (0, 1, 1), (2, 0, 1)],
+             "rules": [(0, 2, 1), (1, 0, 1), (2, 2, 1), (0, 0, 1), (2, 0, 1), (0, 2, 1), (0, 3, 1), (2, 3, 1)]}
+
+
+@pytest.mark.parametrize("stop", [6, 7, -1])  # on a propagation pass, on a merging pass, by the score
+@pytest.mark.parametrize("sequence", sorted(SEQUENCES))
+@pytest.mark.parametrize("name", ["bin_zoo", "unsorted"])
+def test_schedules_one_after_another(name, sequence, stop):
+    """Schedules, jobs, merging rounds and rules alternate on one context:
+    every run equals the run of a fresh context."""
+    g = graphs()[name]
+    n, m, ind, adj, _ = g
+    jobs = [parcd.job(kind=O.MOD, seed=3, max_iter=stop, iter_cap=40),
+            parcd.job(kind=O.MOD, seed=8, max_iter=stop, iter_cap=40),
+            parcd.job(kind=O.CPM, lam=0.01, seed=3, max_iter=stop, iter_cap=40, tie=O.TIE_LOWEST),
+            parcd.job(kind=O.COND, seed=3, max_iter=stop, iter_cap=40)]
+    lab = GG.singleton_labels(n)
+
+    def context():
+        c = parcd.Context(0)
+        c.set_tuning("solo_loop", 0)
+        c.upload_graph(n, m, ind, adj)
+        return c
+
+    fresh = {}
+    with context() as held:
+        for i, run in enumerate(SEQUENCES[sequence]):
+            strategy, j, rounds = run
+            got = outcome(held, lab, jobs[j], strategy, rounds)
+            if run not in fresh:
+                with context() as c:
+                    fresh[run] = outcome(c, lab, jobs[j], strategy, rounds)
+            for x, y in zip(got, fresh[run]):
+                assert np.array_equal(x, y, equal_nan=True) if isinstance(x, float) else np.array_equal(x, y), (i, run)
+
+
+def test_clustering_coefficient_set_between_runs():
+    """WCC's gains hold the clustering coefficient: a run after a new one is
+    set equals that of a fresh context."""
+    n, m, ind, adj, _ = GG.sbm(8, 120, 0.12, 0.004, seed=31)
+    lab = (np.arange(n) // 11).astype(np.int32)
+    jb = parcd.job(kind=O.WCC, seed=3, max_iter=6)
+
+    def context():
+        c = parcd.Context(0)
+        c.upload_graph(n, m, ind, adj)
+        c.triangles()
+        return c
+
+    seen = []
+    with context() as held:
+        for cc in (0.9, 0.001, 0.9):
+            held.set_cc(cc)
+            got = outcome(held, lab, jb, 0, 1)
+            with context() as c:
+                c.set_cc(cc)
+                want = outcome(c, lab, jb, 0, 1)
+            assert got[:3] == want[:3] and all(np.array_equal(x, y) for x, y in zip(got[3:], want[3:]))
+            seen.append(got[3])
+    assert not np.array_equal(seen[0], seen[1])
