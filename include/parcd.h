@@ -206,9 +206,10 @@ int pcd_bin_counters(pcd_ctx *ctx, int bin, int64_t *active, int64_t *entries, i
  * default 2^20; 0 makes the second pass of every sort of more than one tile
  * give up, for tests of that fallback) and "scan_tiles_per_cu" (scans use
  * shorter tiles until there are this many per CU; default 8, in [1, 64]) and
- * "solo_loop" (0/1: pcd_iterate_many and pcd_refine run the propagation passes
- * of a graph of at most 4096 vertices and 32768 entries, under modularity or
- * CPM, in one launch of one workgroup) and "fused_pass" (0/1: a
+ * "solo_loop" (pcd_iterate_many and pcd_refine run the propagation passes of a
+ * graph of at most 4096 vertices and 32768 entries, under modularity or CPM, in
+ * one launch of one workgroup: 0 never, 1, the default, where its entries, long
+ * rows and passes make that the faster way, 2 always) and "fused_pass" (0/1: a
  * device-resident propagation pass under modularity or CPM shares launches
  * between compression, metric, stop rule and bookkeeping) and
  * "contract_rows_min" (pcd_contract counts pairs over community rows from this

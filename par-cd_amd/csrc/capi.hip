@@ -896,7 +896,7 @@ extern "C" int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value) {
     } else if (k == "fused_pass") {
         ctx->tune.fused_pass = value != 0;
     } else if (k == "solo_loop") {
-        ctx->tune.solo_loop = value != 0;
+        ctx->tune.solo_loop = value == 2 ? 2 : value != 0;
     } else if (k == "graph_loop_min_entries") {
         if (value < 0) return fail(PCD_E_INVALID, "graph_loop_min_entries must be >= 0");
         ctx->tune.graph_loop_min_entries = value;

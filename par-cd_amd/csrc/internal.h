@@ -116,7 +116,8 @@ struct Tuning {
                                  // pass with the stop rule on the device (pcd_iterate_many)
     int contract_rows_min = 1 << 22;  // contraction counts pairs over community rows from this many entries on
     int fused_pass = 1;          // a captured propagation pass (modularity, CPM) shares launches between its parts
-    int solo_loop = 1;           // the passes of a small graph in one launch of one workgroup (solo.hip)
+    int solo_loop = 1;           // the passes of a small graph in one launch of one workgroup (solo.hip):
+                                 // 0 never, 1 where it is the faster way, 2 wherever it fits
     int graph_loop_min_entries = 0;  // graphs with fewer CSR entries run pass by pass
     int merge_sort = 0;          // merging picks partners from the sorted unique community pairs
                                  // (1) or counts over community rows, no sort of the entries (0)
@@ -389,7 +390,7 @@ int wcc_metric_dev(pcd_ctx *ctx, double *out);
 
 // the loop of a small graph on one workgroup (solo.hip)
 constexpr int SOLO_MAX_N = 4096, SOLO_MAX_E = 32768, SOLO_MAX_PASSES = 4096;
-bool solo_fits(const pcd_ctx *ctx, const pcd_job *job, int strategy);
+bool solo_fits(const pcd_ctx *ctx, const pcd_job *job, int strategy, int passes);
 int solo_passes(pcd_ctx *ctx, const pcd_job *job, int cap, int it, int count, double prev, SoloResult *res);
 
 RuleParams make_rule(pcd_ctx *ctx, pcd_rule rule);

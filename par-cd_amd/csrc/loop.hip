@@ -311,6 +311,13 @@ static int device_passes(pcd_ctx *ctx, Loop *L, int strategy, bool fused, int it
 
 using namespace pcd;
 
+// passes of [it, it + count) that -n and the iteration cap leave, at least one
+static int last_passes(const pcd_job *job, int cap, int it, int count) {
+    int64_t end = std::min<int64_t>((int64_t)it + count, (int64_t)cap + 1);
+    if (job->max_iter != -1) end = std::min<int64_t>(end, (int64_t)job->max_iter + 1);
+    return (int)std::max<int64_t>(1, end - it);
+}
+
 extern "C" int pcd_iterate_many(pcd_ctx *ctx, const pcd_job *job, int strategy, int rounds, int it, int count,
                                 double prev_score, int *passes, double *score, int *num_labels, int *done) {
     if (!ctx || !job || !passes || !score || !num_labels || !done) return fail(PCD_E_INVALID, "null argument");
@@ -333,7 +340,7 @@ extern "C" int pcd_iterate_many(pcd_ctx *ctx, const pcd_job *job, int strategy, 
     int run = 0;
     if (ctx->tune.graph_loop && ctx->tune.solo_loop && ctx->tune.inc_stats &&
         2 * (int64_t)ctx->m >= ctx->tune.graph_loop_min_entries && !ctx->counters && !ctx->timing &&
-        solo_fits(ctx, job, strategy)) {
+        solo_fits(ctx, job, strategy, last_passes(job, cap, it, count))) {
         // a small graph: the passes in one launch, up to SOLO_MAX_PASSES at a time
         PCD_HIP(hipSetDevice(ctx->device));
         while (run < count && !*done) {

@@ -8,8 +8,9 @@
 // community records and the totals in LDS, and the host reads one record at
 // the end.  What bounds it is the chain of dependent reads and barriers of a
 // pass and, with growing rows, the instruction rate of one CU, so it serves
-// graphs of at most SOLO_N vertices and SOLO_E entries; larger ones run their
-// passes over the whole chip (loop.hip).  Every label, statistic and score is
+// graphs of at most SOLO_MAX_N vertices and SOLO_MAX_E entries, and of those the jobs
+// that solo_pays picks; the others run their passes over the whole chip
+// (loop.hip).  Every label, statistic and score is
 // the one those passes give: the sums are integers, and ties have a total
 // order.
 #include <algorithm>
@@ -275,9 +276,28 @@ __global__ __launch_bounds__(SOLO_NT) void k_solo_loop(SoloArgs a) {
     for (int c = tid; c < k; c += SOLO_NT) a.stats[c] = CommStats{s.size[c], s.iv[c], s.ev[c], 0};
 }
 
-bool solo_fits(const pcd_ctx *ctx, const pcd_job *job, int strategy) {
+// Whether the passes of a job (at most `passes` of them) are faster on one
+// workgroup than replayed over the whole chip.  A pass here takes about 11 us
+// and, per 1,000, 1.2 us for entries, 1.6 us for entries of active rows and
+// 3.2 us for active vertices, and 3.2 us for each active row above 256 entries,
+// which the whole workgroup takes by itself (least squares over 250 to 4,000
+// vertices, 4,000 to 32,000 entries, 0 to 24 such rows, half of the vertices
+// and all of them active; the largest error up to 16,000 entries is 7 us).  A replayed
+// pass takes 45-48 us at all these sizes, after some 120 us for a first pass of
+// single launches and the capture.  Runs of 20 passes, one workgroup / replayed:
+// 1,000 vertices of 8,000 entries 0.53 / 0.95 ms, of 16,000 0.96 / 0.97, of
+// 24,000 1.30 / 0.94; 60 rows of 265 entries 3.6 / 0.98.
+static bool solo_pays(const pcd_ctx *ctx, const pcd_job *job, int passes) {
+    const double f = std::min(job->frac, 1.0), e = 2e-3 * ctx->m, n = 1e-3 * ctx->n;
+    const int long_rows = ctx->bins.start[BIN_W256] - ctx->bins.start[BIN_HUB];
+    const double pass = 11.0 + e * (1.2 + 1.6 * f) + 3.2 * f * (n + long_rows);
+    return pass <= 46.0 + 120.0 / passes;
+}
+
+bool solo_fits(const pcd_ctx *ctx, const pcd_job *job, int strategy, int passes) {
     return strategy == 0 && (job->rule.kind == PCD_RULE_MODULARITY || job->rule.kind == PCD_RULE_CPM) &&
-           ctx->n <= SOLO_N && 2 * (int64_t)ctx->m <= SOLO_MAX_E && ctx->label_bound <= ctx->n;
+           ctx->n <= SOLO_N && 2 * (int64_t)ctx->m <= SOLO_MAX_E && ctx->label_bound <= ctx->n &&
+           (ctx->tune.solo_loop == 2 || solo_pays(ctx, job, passes));
 }
 
 int solo_passes(pcd_ctx *ctx, const pcd_job *job, int cap, int it, int count, double prev, SoloResult *res) {

@@ -1,6 +1,8 @@
 """GPU parity where kernels share an address or a workgroup: partitions with
 a few large communities (every member's update falls on the same records),
 and sizes at the edges of tiles, tables and launch forms."""
+import time
+
 import numpy as np
 import pytest
 
@@ -140,7 +142,7 @@ def test_small_graph_loop(ctx, name):
                                                 (O.MOD, 0.0, 1, 0.8)]):
         lab = starts[i % 2].astype(np.int32)
         got = []
-        for solo, fused, graph in ((1, 1, 1), (0, 1, 1), (0, 0, 1), (0, 0, 0)):
+        for solo, fused, graph in ((2, 1, 1), (1, 1, 1), (0, 1, 1), (0, 0, 1), (0, 0, 0)):
             ctx.set_tuning("solo_loop", solo)
             ctx.set_tuning("fused_pass", fused)
             ctx.set_tuning("graph_loop", graph)
@@ -166,6 +168,34 @@ def test_small_graph_loop(ctx, name):
             assert len(other) == len(got[0])
             for x, y in zip(got[0], other):
                 assert np.array_equal(x, y, equal_nan=True) if isinstance(x, float) else np.array_equal(x, y), (name, i)
+
+
+@pytest.mark.parametrize("hubs,degree", [(60, 265), (30, 530), (0, 0)])
+def test_small_graph_loop_is_not_the_slower_way(hubs, degree):
+    """Small graphs whose passes one workgroup runs two to four times slower
+    than the whole chip (many rows that it takes one by one; 32,000 entries)
+    take the whole chip."""
+    rng = np.random.default_rng(hubs)
+    a, b = [rng.integers(hubs, 4000, 300 if hubs else 16300)], [rng.integers(hubs, 4000, 300 if hubs else 16300)]
+    for h in range(hubs):
+        a.append(np.full(degree, h))
+        b.append(hubs + rng.choice(4000 - hubs, degree, replace=False))
+    g = GG.csr_from_edges(np.concatenate(a), np.concatenate(b))
+    lab = rng.permutation(g[0]).astype(np.int32)
+    with parcd.Context(0) as c:
+        c.upload_graph(*g[:4])
+
+        def best(solo):
+            c.set_tuning("solo_loop", solo)
+            times = []
+            for _ in range(8):
+                c.upload_labels(lab)
+                t = time.perf_counter()
+                c.refine(parcd.job(kind=O.CPM, lam=0.005, seed=3, max_iter=20))
+                times.append(time.perf_counter() - t)
+            return min(times)
+
+        assert best(1) < 1.4 * best(0)
 
 
 @pytest.mark.parametrize("n", [1023, 1024, 1025, 20480, 20481, 65536, 65537])
