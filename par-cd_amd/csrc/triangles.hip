@@ -228,9 +228,39 @@ __global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a, int per) {
     tri_flush<256>(a, hot);
 }
 
+// [first entry >= lo, first entry > hi) of the ascending entries [s, s + len):
+// what of a row can be in a table of the ids lo..hi.  Rows shorter than one
+// step of a wave are kept or left out as a whole.
+__device__ inline void tri_clip(const TriArgs &a, int lo, int hi, int &s, int &len) {
+    if (a.adj[s + len - 1] < lo || a.adj[s] > hi) {
+        len = 0;
+        return;
+    }
+    if (len <= TRI_PF * WAVE) return;
+    const int e = s + len;
+    int b = s, t = e;
+    while (b < t) {
+        const int mid = b + (t - b) / 2;
+        if (a.adj[mid] < lo) b = mid + 1;
+        else t = mid;
+    }
+    s = b;
+    t = e;
+    while (b < t) {
+        const int mid = b + (t - b) / 2;
+        if (a.adj[mid] <= hi) b = mid + 1;
+        else t = mid;
+    }
+    len = b - s;
+}
+
 // One workgroup per listed vertex: its prefix goes into the table in chunks,
 // and for each chunk the waves take the rows behind the chunk's first entry
-// (64 rows' extents loaded at once, one lane each).  Where the list is short,
+// (64 rows' extents loaded at once, one lane each), of which only the entries
+// within the chunk's ids: prefixes of several chunks, the hubs of graphs whose
+// ids do not descend by degree, would look every entry up once per chunk
+// (R-MAT-19 with shuffled ids 180 -> 57 ms; a hub after the 200,000 vertices of
+// its wheel 179 -> 8 ms).  Where the list is short,
 // up to TRI_PARTS workgroups share a vertex, each with its own table and a part
 // of the rows: the rows of one wave are a serial chain.  That and the smaller
 // units of k_triangles_wave, whole call: R-MAT-11 237 -> 97 us, R-MAT-13 332 ->
@@ -271,6 +301,7 @@ __global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
                     if (!a.labels || a.labels[u] == lab) {
                         su = a.indices[u];
                         lu = a.lowpos[u];
+                        if (lu > 0 && len > TRI_CHUNK) tri_clip(a, a.adj[sv + c0], a.adj[sv + c1 - 1], su, lu);
                     }
                 }
                 int found = 0;

@@ -102,6 +102,79 @@ def test_internal_triangles(ctx, graph, labels):
         assert ctx.metric(O.WCC) == pytest.approx(want, rel=1e-9, abs=1e-12)
 
 
+def renamed(g, name):
+    """The graph with vertex v as name[v]."""
+    n, _, ind, adj = g[:4]
+    v = np.repeat(np.arange(n), np.diff(ind))
+    low = adj < v
+    return GG.csr_direct(n, list(zip(name[v[low]].tolist(), name[adj[low]].tolist())))
+
+
+def late_hubs(kind):
+    """Graphs whose hubs come after their neighbours: prefixes of several
+    table chunks, met by rows below and above one step of a wave, with gaps."""
+    rng = np.random.default_rng(17)
+    if kind == "reversed":
+        g = GG.rmat(12, factor=24)
+        return renamed(g, np.arange(g[0])[::-1])
+    if kind == "shuffled":
+        g = GG.rmat(13)
+        return renamed(g, rng.permutation(g[0]))
+    n = 4200  # three hubs over a random graph whose rows reach 60 or 500 entries
+    a, b = np.triu_indices(n - 3, 1)
+    pick = rng.random(a.size) < np.where(a % 2 == 1, 0.014, np.where(b < 2400, 0.2, 0.001))
+    e = [np.stack([a[pick], b[pick]], 1)]
+    for h in (n - 3, n - 2, n - 1):
+        v = np.flatnonzero(rng.random(h) < 0.9)
+        e.append(np.stack([v, np.full(v.size, h)], 1))
+    return GG.csr_direct(n, np.concatenate(e).tolist())
+
+
+@pytest.mark.parametrize("kind", ["reversed", "shuffled", "random"])
+def test_triangles_of_late_hubs(ctx, kind):
+    n, m, ind, adj = late_hubs(kind)[:4]
+    low = np.array([np.searchsorted(adj[ind[v]:ind[v + 1]], v) for v in range(n)])
+    assert low.max() > 1024  # several chunks
+    ctx.upload_graph(n, m, ind, adj)
+    tri, tdeg, _ = ctx.triangles()
+    _, t_o, td_o, _ = O.count_triangles(n, ind, adj)
+    assert np.array_equal(tri, t_o) and np.array_equal(tdeg, td_o)
+    lab, _ = O.compress_labels(np.random.default_rng(2).integers(0, 3, n).astype(np.int32))
+    ctx.upload_labels(lab)
+    ctx.compress()
+    ctx.statistics()
+    s, _, _ = O.collect_statistics(n, ind, adj, lab)[1:]
+    want = O.wcc_calculate(n, ind, adj, lab, s, t_o, td_o)[0]
+    assert ctx.metric(O.WCC) == pytest.approx(want, rel=1e-9, abs=1e-12)
+
+
+def test_a_late_hub_costs_what_its_rows_hold(ctx):
+    """A hub after its 200,000 neighbours: their rows are looked up in the
+    chunks of the hub's prefix that they can meet (in all 196, the wheel took
+    57 times what the star takes, whose rows hold nothing to look up)."""
+    n = 200001
+    v = np.arange(n - 1)
+
+    def best(u, w):
+        key = np.sort(np.concatenate([u * n + w, w * n + u]))
+        ind = np.zeros(n + 1, np.int32)
+        ind[1:] = np.cumsum(np.bincount(key // n, minlength=n))
+        ctx.upload_graph(n, key.size // 2, ind, (key % n).astype(np.int32))
+        times = []
+        for _ in range(4):
+            t = time.perf_counter()
+            tri = ctx.triangles()[0]
+            times.append(time.perf_counter() - t)
+        return min(times), tri
+
+    hub = np.full(n - 1, n - 1)
+    star, tri = best(v, hub)
+    assert not tri.any()
+    wheel, tri = best(np.concatenate([v, v]), np.concatenate([hub, (v + 1) % (n - 1)]))
+    assert tri[n - 1] == 2 * (n - 1) and (tri[:n - 1] == 4).all()
+    assert wheel < 15 * star
+
+
 def small_graphs():
     """Sizes at the edges of the one-workgroup loop: degrees in every table
     class, isolated vertices, unsorted ids, the largest vertex and entry
