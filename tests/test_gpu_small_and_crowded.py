@@ -148,6 +148,24 @@ def test_triangles_of_late_hubs(ctx, kind):
     assert ctx.metric(O.WCC) == pytest.approx(want, rel=1e-9, abs=1e-12)
 
 
+@pytest.mark.parametrize("n", [1023, 1025, 20480, 20481])
+def test_triangles_of_listed_vertices(ctx, n):
+    """The list of long prefixes at the edges of its scans' tiles: wheels whose
+    hubs lie there, and at the last id."""
+    v = np.arange(100, 200)  # the rim, below every hub
+    e = [np.stack([v, np.where(v == 199, 100, v + 1)], 1)]
+    hubs = [h for h in (200, 1022, 1023, 1024, 4095, 4096, 20479, n - 1) if h < n]
+    for i, h in enumerate(hubs):
+        k = (64, 65, 100)[i % 3]  # a wave's prefix, and two longer ones
+        e.append(np.stack([v[:k], np.full(k, h)], 1))
+    n, m, ind, adj = GG.csr_direct(n, np.concatenate(e).tolist())[:4]
+    ctx.upload_graph(n, m, ind, adj)
+    tri, tdeg, cc = ctx.triangles()
+    _, t_o, td_o, cc_o = O.count_triangles(n, ind, adj)
+    assert np.array_equal(tri, t_o) and np.array_equal(tdeg, td_o)
+    assert cc == pytest.approx(cc_o, rel=1e-9)
+
+
 def test_a_late_hub_costs_what_its_rows_hold(ctx):
     """A hub after its 200,000 neighbours: their rows are looked up in the
     chunks of the hub's prefix that they can meet (in all 196, the wheel took
