@@ -88,7 +88,9 @@ __global__ void k_order_of(int n, const uint64_t *sorted, int32_t *order, uint8_
 // vertices a round meets are decided already, and most rows are short: with a
 // wave per vertex a round of the 1 M vertex Chung-Lu graph took 63 us when
 // hardly any vertex was left, 99 us on average; eight to a wave 8 and 35 us.
-constexpr int OCT_ROW = 128;
+// Above 32 entries the wave is the faster reader (random graph of 1 M vertices
+// and mean degree 40, whole clustering: 3.27 ms with 128 here, 2.84 with 32).
+constexpr int OCT_ROW = 32;
 
 // any lane of the aligned group of eight / of the wave
 __device__ inline bool oct_any(bool x) { return ((__ballot(x) >> (__lane_id() & ~7)) & 0xff) != 0; }
@@ -108,17 +110,25 @@ __device__ inline void center_scan(int b, int e, int first, uint64_t kv, const i
     }
 }
 
-// One round over the vertices in order.  *open is set when a vertex stays
-// undecided.
-__global__ __launch_bounds__(256) void k_center_round(int n, const int32_t *order, const int32_t *indices,
+// One round over the vertices in order, a wave's eight `step` apart (1, or the
+// number of waves where `spread`).  *open is set when a vertex stays
+// undecided.  Neighbours in the order have like coefficients, so hubs stand
+// together; where the longest row is long for the graph, a wave with eight of
+// them would be what the round waits for (whole clustering, consecutive /
+// spread: R-MAT-18 1.44 / 1.19 ms, R-MAT-22 7.9 / 6.9).  Otherwise consecutive ones share the cache lines of the order (the 1 M vertex
+// Chung-Lu graph, longest row 8,415: 1.74 / 1.84; of 200,000, longest 5,966:
+// 1.08 / 1.07).
+constexpr int SPREAD_SHARE = 64;  // spread from a longest row of n / 64 entries on
+__global__ __launch_bounds__(256) void k_center_round(int n, bool spread, const int32_t *order, const int32_t *indices,
                                                       const int32_t *adj, const uint64_t *key, uint8_t *state,
                                                       int32_t *open) {
     const int lane = __lane_id(), oct = lane & 7;
     const int wave_g = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
     const int nwaves = gridDim.x * blockDim.x / WAVE;
     bool left = false;
-    for (int64_t base = (int64_t)wave_g * 8; base < n; base += (int64_t)nwaves * 8) {
-        const int64_t t = base + lane / 8;
+    const int step = spread ? nwaves : 1;
+    for (int64_t base = spread ? wave_g : (int64_t)wave_g * 8; base < n; base += (int64_t)nwaves * 8) {
+        const int64_t t = base + (int64_t)(lane / 8) * step;
         const int v = t < n ? order[t] : 0;
         const bool mine = t < n && state[v] == ST_OPEN;
         if (!__ballot(mine)) continue;
@@ -272,8 +282,9 @@ int clustering_labels_dev(pcd_ctx *ctx, int *num_communities) {
     bool done = false;
     for (int r = 0; r < ctx->tune.cluster_rounds; r++) {
         PCD_CL(fill_i32(ctx, open, 0, 1));
-        hipLaunchKernelGGL(k_center_round, dim3(grid_for(ctx, n, 4 * 8, 8)), dim3(256), 0, ctx->stream, n, order,
-                           ctx->d_indices, ctx->d_adj, fkey, state, open);
+        hipLaunchKernelGGL(k_center_round, dim3(grid_for(ctx, n, 4 * 8, 8)), dim3(256), 0, ctx->stream, n,
+                           (int64_t)ctx->max_degree * SPREAD_SHARE >= n, order, ctx->d_indices, ctx->d_adj, fkey, state,
+                           open);
         if (hipGetLastError() != hipSuccess) PCD_CL(fail(PCD_E_HIP, "k_center_round launch"));
         if (hipMemcpyAsync(ctx->h_small, open, 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess)

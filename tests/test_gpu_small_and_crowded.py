@@ -193,6 +193,35 @@ def test_a_late_hub_costs_what_its_rows_hold(ctx):
     assert wheel < 15 * star
 
 
+@pytest.mark.parametrize("hub", [0, 200])
+@pytest.mark.parametrize("n", [2047, 2048, 6000])
+def test_clustering_of_rows_of_every_length(ctx, n, hub):
+    """Rows at the edges of the eight-lane and the whole-wave reader (8, 32, 33,
+    64, 65 entries), the rounds' vertices consecutive (no row of n / 64
+    entries) and spread over the waves (one hub)."""
+    rng = np.random.default_rng(n)
+    v = np.arange(n)
+    e = [np.stack([v, (v + 1) % n], 1)]
+    for size in (7, 8, 9, 31, 32, 33) + ((63, 64, 65) if n == 6000 else ()):
+        for _ in range(4 if hub or n == 6000 else 0):
+            m = rng.choice(n, size, replace=False)
+            e.append(np.stack([np.repeat(m[:1], size - 1), m[1:]], 1))
+            i, j = np.triu_indices(min(size, 9), 1)
+            e.append(np.stack([m[i], m[j]], 1))
+    if hub:
+        e.append(np.stack([np.full(hub, 5), rng.choice(np.arange(6, n), hub, replace=False)], 1))
+    n, m, ind, adj = GG.csr_direct(n, np.concatenate(e).tolist())[:4]
+    assert (64 * int(np.diff(ind).max()) >= n) == bool(hub)
+    ctx.upload_graph(n, m, ind, adj)
+    tri = ctx.triangles()[0]
+    want = O.clustering_partition(n, ind, adj, tri)
+    for rounds in (1, 128):
+        ctx.set_tuning("cluster_rounds", rounds)
+        ctx.clustering()
+        ctx.set_tuning("cluster_rounds", 128)
+        assert np.array_equal(ctx.labels(), want), rounds
+
+
 def small_graphs():
     """Sizes at the edges of the one-workgroup loop: degrees in every table
     class, isolated vertices, unsorted ids, the largest vertex and entry
