@@ -213,8 +213,9 @@ int pcd_bin_counters(pcd_ctx *ctx, int bin, int64_t *active, int64_t *entries, i
  * device-resident propagation pass under modularity or CPM shares launches
  * between compression, metric, stop rule and bookkeeping) and
  * "contract_rows_min" (pcd_contract counts pairs over community rows from this
- * many entries on, where the communities' volumes promise few pairs; default
- * 2^22).
+ * many entries on; default 2^22) and "contract_rows_labels" (... and where the
+ * communities' volumes promise at most this many labels among 2,048 entries;
+ * default 512).
  * Results do not depend on them. */
 int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value);
 /* Hub label partitions whose distinct labels overflowed their LDS table

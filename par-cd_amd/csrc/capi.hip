@@ -156,7 +156,7 @@ extern "C" int pcd_ctx_create(int device, pcd_ctx **out) {
     }
     if (hipHostMalloc((void **)&ctx->h_result, 64, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&ctx->h_small, 256, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&ctx->h_small64, 256, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void **)&ctx->h_small64, sizeof(int64_t) * SMALL64, hipHostMallocDefault) != hipSuccess) {
         pcd_ctx_destroy(ctx);
         return fail(PCD_E_NOMEM, "pinned host allocation failed");
     }
@@ -893,6 +893,9 @@ extern "C" int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value) {
     } else if (k == "contract_rows_min") {
         if (value < 0) return fail(PCD_E_INVALID, "contract_rows_min must be >= 0");
         ctx->tune.contract_rows_min = value;
+    } else if (k == "contract_rows_labels") {
+        if (value < 0) return fail(PCD_E_INVALID, "contract_rows_labels must be >= 0");
+        ctx->tune.contract_rows_labels = value;
     } else if (k == "fused_pass") {
         ctx->tune.fused_pass = value != 0;
     } else if (k == "solo_loop") {

@@ -115,6 +115,7 @@ struct Tuning {
     int graph_loop = 1;          // modularity / CPM with -s 0: passes replayed from one captured
                                  // pass with the stop rule on the device (pcd_iterate_many)
     int contract_rows_min = 1 << 22;  // contraction counts pairs over community rows from this many entries on
+    int contract_rows_labels = 512;   // ... and up to this many labels expected in a tile of 2,048 entries
     int fused_pass = 1;          // a captured propagation pass (modularity, CPM) shares launches between its parts
     int solo_loop = 1;           // the passes of a small graph in one launch of one workgroup (solo.hip):
                                  // 0 never, 1 where it is the faster way, 2 wherever it fits
@@ -128,6 +129,7 @@ constexpr int HUB_TB = 4096;          // LDS table capacity of a hub partition
 static_assert(Tuning{}.hub_table_slots <= HUB_TB && Tuning{}.hub_table_slots % 64 == 0,
               "default hub table must fit the LDS table");
 constexpr int HUB_CHUNK = 4096;      // entries per hub chunk item (pass 1 holds 512 x 8)
+constexpr int SMALL64 = 64;           // page-locked int64 words of a context
 constexpr int HUB_PARTIAL_BYTES = 32; // storage per (hub, partition) partial result
 
 // Kernel timer slots (HIP events around each launch when timing is on).
@@ -270,7 +272,7 @@ struct pcd_ctx {
     bool k_deferred = false;         // k is on the device; h_small[K_SLOT] receives it
     hipEvent_t ev_metric = nullptr;  // recorded after the score's read-back
     int32_t *h_small = nullptr;      // pinned scratch ints
-    int64_t *h_small64 = nullptr;    // pinned scratch int64
+    int64_t *h_small64 = nullptr;    // pinned scratch int64, pcd::SMALL64 of them
 
     // triangles
     bool has_triangles = false;

@@ -98,12 +98,52 @@ __global__ void k_run_lengths(const int32_t *Up, const int32_t *hpos, int P, int
         links[u] = (u + 1 < U ? hpos[u + 1] : P) - hpos[u];
 }
 
-__global__ void k_sum_int_vol(const CommStats *st, const int32_t *kp, unsigned long long *acc) {
-    const int k = *kp;
-    long long a = 0;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += gridDim.x * blockDim.x) a += st[c].int_vol;
+// What a contraction is planned from: the entries inside communities, and the
+// distinct labels expected among `tile` entries (x 1024) if neighbours fell
+// into communities by volume, few where some communities are large.  Each
+// workgroup leaves its two shares in page-locked host memory (R-MAT-18, refined:
+// 474 us a contraction with a counter to clear, add to, copy and wait for, for
+// each sum; 441 so).
+constexpr int PS_NT = 1024, PS_GRID = 32;
+__global__ __launch_bounds__(PS_NT) void k_pair_sums(const CommStats *st, int k, float tile_share, int64_t *out) {
+    __shared__ long long inside[PS_NT / WAVE], labels[PS_NT / WAVE];
+    long long a = 0, b = 0;
+    for (int c = blockIdx.x * PS_NT + threadIdx.x; c < k; c += gridDim.x * PS_NT) {
+        const CommStats s = st[c];
+        a += s.int_vol;
+        b += (long long)(-1024.0f * expm1f(-tile_share * ((float)s.int_vol + (float)s.ext_vol)));
+    }
     a = wave_sum64(a);
-    if (__lane_id() == 0) atomicAdd(acc, (unsigned long long)a);
+    b = wave_sum64(b);
+    if (threadIdx.x % WAVE == 0) {
+        inside[threadIdx.x / WAVE] = a;
+        labels[threadIdx.x / WAVE] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int i = 1; i < PS_NT / WAVE; i++) {
+        a += inside[i];
+        b += labels[i];
+    }
+    out[2 * blockIdx.x] = a;
+    out[2 * blockIdx.x + 1] = b;
+}
+static int pair_sums_grid(const pcd_ctx *ctx) { return std::max(1, std::min(PS_GRID, (ctx->k + PS_NT - 1) / PS_NT)); }
+static int pair_sums_enqueue(pcd_ctx *ctx, int tile) {
+    static_assert(2 * PS_GRID <= SMALL64, "the shares' place in host memory");
+    hipLaunchKernelGGL(k_pair_sums, dim3(pair_sums_grid(ctx)), dim3(PS_NT), 0, ctx->stream, ctx->d_stats, ctx->k,
+                       (float)tile / std::max(1.0f, 2.0f * (float)ctx->m), ctx->h_small64);
+    PCD_HIP(hipGetLastError());
+    return PCD_OK;
+}
+// the sums, once the stream has passed the kernel
+static void pair_sums(const pcd_ctx *ctx, int64_t *inside, int64_t *tile_labels) {
+    *inside = *tile_labels = 0;
+    for (int i = 0; i < pair_sums_grid(ctx); i++) {
+        *inside += ctx->h_small64[2 * i];
+        *tile_labels += ctx->h_small64[2 * i + 1];
+    }
+    *tile_labels /= 1024;
 }
 
 static int label_bits(int k) {
@@ -142,8 +182,9 @@ static int reserve_pairs(pcd_ctx *ctx) {
 }
 
 // Builds the sorted unique (l, k) keys in ctx->d_keys1[0..U) with link
-// counts in ctx->d_pair_links.  Returns U and the key layout.
-static int build_pairs(pcd_ctx *ctx, int64_t *U_out, int *half_out) {
+// counts in ctx->d_pair_links.  Returns U and the key layout.  `inside`: the
+// entries inside communities, or -1 to sum them here.
+static int build_pairs(pcd_ctx *ctx, int64_t inside, int64_t *U_out, int *half_out) {
     const int64_t E = (int64_t)2 * ctx->m;
     PCD_TRY(reserve_pairs(ctx));
     const int half = label_bits(ctx->k);
@@ -158,20 +199,19 @@ static int build_pairs(pcd_ctx *ctx, int64_t *U_out, int *half_out) {
     launch_keys_small<16>(ctx, BIN_G16, bits);
     launch_keys_small<8>(ctx, BIN_G8, bits);
     launch_keys_small<4>(ctx, BIN_G4, bits);
-    // P = E - sum(int_volume): entries between different communities
-    unsigned long long *acc = (unsigned long long *)ctx->d_acc;
-    PCD_TRY(fill_u64(ctx, (uint64_t *)acc, 0, 1));
-    hipLaunchKernelGGL(k_sum_int_vol, dim3(grid_for(ctx, ctx->k, 256, 4)), dim3(256), 0, ctx->stream, ctx->d_stats,
-                       ctx->d_k, acc);
+    if (inside < 0) PCD_TRY(pair_sums_enqueue(ctx, 0));
     kt_end(ctx, KS_MERGE_KEYS);
     PCD_HIP(hipGetLastError());
     uint64_t *sorted = nullptr;
     kt_begin(ctx, KS_MERGE_SORT);
     PCD_TRY(radix_sort_u64(ctx, ctx->d_keys0, ctx->d_keys1, E, bits, &sorted));
     kt_end(ctx, KS_MERGE_SORT);
-    PCD_HIP(hipMemcpyAsync(ctx->h_small64, acc, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
-    PCD_HIP(hipStreamSynchronize(ctx->stream));
-    const int64_t P = E - ctx->h_small64[0];
+    if (inside < 0) {
+        int64_t tile_labels;
+        PCD_HIP(hipStreamSynchronize(ctx->stream));
+        pair_sums(ctx, &inside, &tile_labels);
+    }
+    const int64_t P = E - inside;  // entries between different communities
     uint64_t *ukeys = sorted == ctx->d_keys0 ? ctx->d_keys1 : ctx->d_keys0;
     int32_t *total = nullptr;
     kt_begin(ctx, KS_MERGE_RLE);
@@ -1156,7 +1196,7 @@ static int merging_pairs_dev(pcd_ctx *ctx, pcd_rule rule, int rounds, uint64_t s
     const int k = ctx->k;
     int64_t U = 0;
     int half = 0;
-    PCD_TRY(build_pairs(ctx, &U, &half));
+    PCD_TRY(build_pairs(ctx, -1, &U, &half));
     PCD_TRY(ensure_merge_state(ctx));
     // candidate slots: two per 64 pairs (the runs that may cross a wave boundary)
     const size_t ncap = (size_t)(2 * ((U + WAVE - 1) / WAVE) + 2);
@@ -1312,29 +1352,18 @@ __global__ void k_run_links(int U, int64_t V, const int32_t *hpos, const int32_t
         links[u] = before[u + 1 < U ? hpos[u + 1] : V] - before[hpos[u]];
 }
 
-// Distinct labels expected among a tile's entries (x 1024) if neighbours fell
-// into communities by volume: few where some communities are large.
-__global__ __launch_bounds__(256) void k_tile_labels(const CommStats *st, int k, double per_entry,
-                                                     unsigned long long *acc) {
-    __shared__ long long part[256 / WAVE];
-    long long a = 0;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += gridDim.x * blockDim.x)
-        a += (long long)(1024.0 * (1.0 - exp(-(double)CT_TILE * per_entry * ((double)st[c].int_vol + st[c].ext_vol))));
-    a = wave_sum64(a);
-    if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = a;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(acc, (unsigned long long)(part[0] + part[1] + part[2] + part[3]));
-}
-
 // The sorted unique pairs through community rows.  The sort moves the tiles'
 // pairs instead of every entry: worth it where most entries of a tile repeat
 // a pair of it.  Partitions of hub neighbourhoods, R-MAT-18 and -20 (0.10 and
 // 0.39 M pairs of 7.6 and 31 M entries): 0.48 -> 0.33 and 1.42 -> 0.78 ms a
 // call.  Partitions at random into 1,900 to 440,000 communities would take
-// 10-25 % longer by rows; k_tile_labels tells them apart, for 0.02 ms (0.45 ->
-// 0.47 ms at R-MAT-18).  Graphs below 2^22 entries (tunable contract_rows_min)
-// gain nothing: 0.16 -> 0.19 ms at R-MAT-14.
-constexpr int CT_MAX_LABELS = CT_TILE / 4;
+// 10-25 % longer by rows; k_pair_sums tells them apart (up to a quarter of a
+// tile's entries, tunable contract_rows_labels), and the sort would have
+// summed and waited for the entries inside communities anyway.  The line of
+// 2^22 entries (tunable contract_rows_min): both ways, two contractions and
+// their download, 0.43 / 0.37 ms at 0.2 M entries, 0.55 / 0.55 and 0.54 / 0.49
+// (300 communities at random) at 1.8 M, 0.61 / 0.72 and 0.59 / 0.59 at 3.7 M,
+// 0.78 / 1.05 and 0.73 / 0.82 at 7.6 M.
 static int reserve_pair_rows(pcd_ctx *ctx) {
     const size_t E = (size_t)2 * ctx->m, n = (size_t)ctx->n;
     if (!ctx->mrows) ctx->mrows = new MergeRows();
@@ -1393,21 +1422,19 @@ int contract_dev(pcd_ctx *ctx, int64_t *num_pairs) {
     // a pair and its count share a 64-bit word, and a tile's end is an int
     bool rows = !ctx->tune.onesweep && E >= ctx->tune.contract_rows_min && E > 0 && E <= INT32_MAX - CT_TILE &&
                 ctx->k > 0 && 2 * label_bits(ctx->k) + CT_CNT_BITS <= 64;
+    int64_t inside = -1;
     if (rows) {
-        unsigned long long *acc = (unsigned long long *)ctx->d_acc;
-        PCD_TRY(fill_u64(ctx, (uint64_t *)acc, 0, 1));
-        hipLaunchKernelGGL(k_tile_labels, dim3(grid_for(ctx, ctx->k, 256, 1)), dim3(256), 0, ctx->stream, ctx->d_stats,
-                           ctx->k, 1.0 / (double)E, acc);
-        PCD_HIP(hipGetLastError());
-        PCD_HIP(hipMemcpyAsync(ctx->h_small64, acc, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+        int64_t tile_labels;
+        PCD_TRY(pair_sums_enqueue(ctx, CT_TILE));
         PCD_HIP(hipStreamSynchronize(ctx->stream));
+        pair_sums(ctx, &inside, &tile_labels);
         // the rows take 4 bytes per entry more: without that memory, the sort
-        rows = ctx->h_small64[0] / 1024 <= CT_MAX_LABELS && reserve_pair_rows(ctx) == PCD_OK;
+        rows = tile_labels <= ctx->tune.contract_rows_labels && reserve_pair_rows(ctx) == PCD_OK;
     }
     if (rows)
         PCD_TRY(build_pairs_by_rows(ctx, &U));
     else
-        PCD_TRY(build_pairs(ctx, &U, &half));
+        PCD_TRY(build_pairs(ctx, inside, &U, &half));
     *num_pairs = U;
     return PCD_OK;
 }

@@ -414,20 +414,28 @@ def test_noalloc_compression_sizes(ctx, n):
         hip.ok(hip.h.hipFree(p))
 
 
-@pytest.mark.parametrize("kind", ["one", "half", "table", "seven_new", "planted", "sparse_ids"])
-@pytest.mark.parametrize("graph", ["bin_zoo", "unsorted", "rmat12", "ring", "one_tile", "past_a_tile"])
-def test_contraction_by_rows(ctx, graph, kind):
-    """Pairs counted over community rows in tiles equal the oracle's: few large
-    rows, rows that cross tiles, empty rows (ids in use with gaps), and both
-    sides of the row length from which the rows are used."""
-    ring = lambda n: GG.csr_direct(n, [(i, (i + 1) % n) for i in range(n)])  # 2n entries
+def ring(n):  # 2n entries
+    return GG.csr_direct(n, [(i, (i + 1) % n) for i in range(n)])
+
+
+@pytest.mark.parametrize("kind", ["one", "half", "table", "seven_new", "planted", "sparse_ids", "singletons"])
+@pytest.mark.parametrize("graph", ["bin_zoo", "unsorted", "rmat12", "ring", "one_tile", "past_a_tile", "wide"])
+def test_contraction_by_rows_and_by_sort(ctx, graph, kind):
+    """Pairs counted over community rows in tiles, and sorted entry by entry,
+    equal the oracle's: few large rows, rows that cross tiles, empty rows (ids
+    in use with gaps), both sides of the row length from which the rows are
+    used, and tiles of 2,048 different pairs (half of a tile's table).  The
+    limits on entries and labels force each way."""
     g = {"bin_zoo": GG.bin_zoo, "unsorted": lambda: GG.unsorted_copy(GG.bin_zoo()), "rmat12": lambda: GG.rmat(12),
-         "ring": lambda: ring(5000), "one_tile": lambda: ring(1024), "past_a_tile": lambda: ring(1025)}[graph]()
+         "ring": lambda: ring(5000), "one_tile": lambda: ring(1024), "past_a_tile": lambda: ring(1025),
+         "wide": lambda: ring(33000)}[graph]()  # more communities than one pass of the sums takes
     n, m, ind, adj = g[:4]
     if kind == "planted":
         lab = (np.arange(n) * 40 // n).astype(np.int32)
     elif kind == "sparse_ids":
         lab = (np.arange(n) % 61 * (n // 64)).astype(np.int32)  # not compressed: empty rows between
+    elif kind == "singletons":
+        lab = np.random.default_rng(5).permutation(n).astype(np.int32)
     else:
         lab = crowded(kind, n)
     ctx.upload_graph(n, m, ind, adj)
@@ -436,12 +444,17 @@ def test_contraction_by_rows(ctx, graph, kind):
         ctx.compress()
         lab = ctx.labels()
     k = ctx.statistics()
-    ctx.set_tuning("contract_rows_min", 0)
-    got = ctx.contract()
-    ctx.set_tuning("contract_rows_min", 1 << 22)
     want = O.community_pairs(n, ind, adj, lab, k)
-    for x, y in zip(got, want):
-        assert np.array_equal(x, y), (graph, kind)
+    try:
+        for least, labels in ((0, 1 << 30), (0, 0), (0, 512), (1 << 30, 512)):  # rows, sort, by the volumes, sort
+            ctx.set_tuning("contract_rows_min", least)
+            ctx.set_tuning("contract_rows_labels", labels)
+            got = ctx.contract()
+            for x, y in zip(got, want):
+                assert np.array_equal(x, y), (graph, kind, least, labels)
+    finally:
+        ctx.set_tuning("contract_rows_min", 1 << 22)
+        ctx.set_tuning("contract_rows_labels", 512)
 
 
 @pytest.mark.parametrize("cut", [1, 2, 3])
