@@ -805,14 +805,17 @@ struct GrowBuf {
     int reserve(pcd_ctx *ctx, size_t need, bool *grew = nullptr) {
         if (grew) *grew = false;
         if (p && cap >= need) return PCD_OK;
-        if (p) dev_free(ctx, p);
-        p = nullptr;
-        cap = 0;
+        release(ctx);
         const size_t c = need + need / 8 + 16;
         PCD_TRY(dev_alloc_t(ctx, &p, c));
         cap = c;
         if (grew) *grew = true;
         return PCD_OK;
+    }
+    void release(pcd_ctx *ctx) {
+        if (p) dev_free(ctx, p);
+        p = nullptr;
+        cap = 0;
     }
 };
 
@@ -1368,11 +1371,18 @@ static int reserve_pair_rows(pcd_ctx *ctx) {
     const size_t E = (size_t)2 * ctx->m, n = (size_t)ctx->n;
     if (!ctx->mrows) ctx->mrows = new MergeRows();
     MergeRows &R = *static_cast<MergeRows *>(ctx->mrows);
-    PCD_TRY(R.ent.reserve(ctx, E + 1));
-    PCD_TRY(R.cind.reserve(ctx, n + 3));
-    PCD_TRY(R.next.reserve(ctx, n + 3));
-    PCD_TRY(R.dst.reserve(ctx, n + 2));
-    return PCD_OK;
+    int rc = R.ent.reserve(ctx, E + 1);
+    if (rc == PCD_OK) rc = R.cind.reserve(ctx, n + 3);
+    if (rc == PCD_OK) rc = R.next.reserve(ctx, n + 3);
+    if (rc == PCD_OK) rc = R.dst.reserve(ctx, n + 2);
+    if (rc != PCD_OK) {
+        // the sort takes over: what it needs must not be held here
+        R.ent.release(ctx);
+        R.cind.release(ctx);
+        R.next.release(ctx);
+        R.dst.release(ctx);
+    }
+    return rc;
 }
 
 static int build_pairs_by_rows(pcd_ctx *ctx, int64_t *U_out) {
