@@ -209,7 +209,7 @@ static void free_graph_state(pcd_ctx *ctx) {
     ctx->d_firstv = nullptr;
     ctx->d_scan_part = nullptr;
     ctx->scan_part_cap = 0;
-    ctx->d_tri = ctx->d_tri_deg = ctx->d_tri_list = nullptr;
+    ctx->d_tri = ctx->d_tri_deg = ctx->d_tri_list = ctx->d_tri_chunked = nullptr;
     ctx->d_lowpos = ctx->d_it = ctx->d_itd = nullptr;
     ctx->d_tri_flag = nullptr;
     ctx->d_solo = nullptr;

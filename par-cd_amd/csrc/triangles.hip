@@ -23,19 +23,6 @@
 
 namespace pcd {
 
-// lowpos[v] = number of neighbours of v with a smaller id
-__global__ void k_lowpos(int n, const int32_t *indices, const int32_t *adj, int32_t *lowpos) {
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-        int lo = indices[v], hi = indices[v + 1];
-        while (lo < hi) {
-            int mid = (lo + hi) >> 1;
-            if (adj[mid] < v) lo = mid + 1;
-            else hi = mid;
-        }
-        lowpos[v] = lo - indices[v];
-    }
-}
-
 // prefixes of at most TRI_WAVE entries: one wave per vertex; longer ones,
 // listed once per graph: one workgroup per vertex
 constexpr int TRI_WAVE = 64, TRI_WAVE_LOG = 9;
@@ -44,6 +31,24 @@ constexpr int TRI_BLOCK_LOG = 11, TRI_CHUNK = 1 << (TRI_BLOCK_LOG - 1);
 // highest degrees, and their words are what the additions queue on
 constexpr int TRI_HOT = 1024;
 constexpr int TRI_PF = 3;  // row entries a lane looks up at once
+
+// lowpos[v] = number of neighbours of v with a smaller id, and, where `list` is
+// given, the vertices whose prefix exceeds one table, in any order (there are
+// few: *listed starts at 0)
+__global__ void k_lowpos(int n, const int32_t *indices, const int32_t *adj, int32_t *lowpos, int32_t *list,
+                         int32_t *listed) {
+    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
+        int lo = indices[v], hi = indices[v + 1];
+        while (lo < hi) {
+            int mid = (lo + hi) >> 1;
+            if (adj[mid] < v) lo = mid + 1;
+            else hi = mid;
+        }
+        lo -= indices[v];
+        lowpos[v] = lo;
+        if (list && lo > TRI_CHUNK) list[atomicAdd(listed, 1)] = v;
+    }
+}
 
 struct TriArgs {
     int n;
@@ -135,10 +140,19 @@ __device__ inline void tri_flush(const TriArgs &a, const int *hot) {
 }
 
 // A wave looks at `per` vertices at once (eight, fewer where the graph has too
-// few vertices for all waves), eight lanes each, and takes those with at least two (same-label) neighbours below them one by one.  Rows
+// few vertices for all waves), eight lanes each, and takes those with at least
+// two (same-label) neighbours below them one by one.  Rows
 // u are read 64 lanes wide, or four at a time 16 lanes wide where they are
 // short on average (Chung-Lu rows hold 30-60 entries, R-MAT rows 150-190).
-__global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a, int per) {
+// A wave's vertices follow one another, or with `spread` lie the number of
+// waves apart: ids descend by degree, so the dear ones stand together, and up
+// to TRI_SPREAD_N vertices there are too few waves to even that out
+// (consecutive / spread: Chung-Lu graphs of 60,000 vertices 334 / 168 us, of
+// 200,000 568 / 491, of 400,000 872 / 869; where only the internal triangles
+// of small communities count, reading the extents is most of it: 44 / 45 us,
+// 75 / 81, 101 / 108).
+constexpr int TRI_SPREAD_N = 1 << 18;
+__global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a, int per, bool spread) {
     __shared__ int s_keys[256 / WAVE][1 << TRI_WAVE_LOG], s_cnts[256 / WAVE][1 << TRI_WAVE_LOG];
     __shared__ int s_row[256 / WAVE][3][TRI_WAVE];
     __shared__ int hot[TRI_HOT];
@@ -150,9 +164,11 @@ __global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a, int per) {
     int *rsu = s_row[w][0], *rlen = s_row[w][1], *rcnt = s_row[w][2];
     const int wave_g = (blockIdx.x * 256 + threadIdx.x) / WAVE;
     const int nwaves = gridDim.x * (256 / WAVE);
-    for (int64_t base = (int64_t)wave_g * per; base < a.n; base += (int64_t)nwaves * per) {
-        const int vo = (int)min((int64_t)a.n - 1, base + lane / 8);
-        int plen = lane / 8 < per && base + lane / 8 < a.n ? a.lowpos[vo] : 0;
+    const int step = spread ? nwaves : 1;
+    for (int64_t base = spread ? wave_g : (int64_t)wave_g * per; base < a.n; base += (int64_t)nwaves * per) {
+        const int64_t vl = base + (int64_t)(lane / 8) * step;
+        const int vo = (int)min((int64_t)a.n - 1, vl);
+        int plen = lane / 8 < per && vl < a.n ? a.lowpos[vo] : 0;
         if (plen > TRI_WAVE) plen = 0;
         const int pstart = a.indices[vo], plab = a.labels ? a.labels[vo] : 0;
         int mine = plen;
@@ -166,7 +182,7 @@ __global__ __launch_bounds__(256) void k_triangles_wave(TriArgs a, int per) {
         while (todo) {
             const int src = __builtin_ctzll(todo);
             todo &= todo - 1;
-            const int v = (int)base + src / 8;
+            const int v = (int)(base + (int64_t)(src / 8) * step);
             const int len = __builtin_amdgcn_readlane(plen, src), sv = __builtin_amdgcn_readlane(pstart, src);
             const int lab = __builtin_amdgcn_readlane(plab, src);
             const int log = tri_log(len);
@@ -254,31 +270,38 @@ __device__ inline void tri_clip(const TriArgs &a, int lo, int hi, int &s, int &l
     len = b - s;
 }
 
-// One workgroup per listed vertex: its prefix goes into the table in chunks,
-// and for each chunk the waves take the rows behind the chunk's first entry
-// (64 rows' extents loaded at once, one lane each), of which only the entries
-// within the chunk's ids: prefixes of several chunks, the hubs of graphs whose
-// ids do not descend by degree, would look every entry up once per chunk
-// (R-MAT-19 with shuffled ids 180 -> 57 ms; a hub after the 200,000 vertices of
-// its wheel 179 -> 8 ms).  Where the list is short,
+// One workgroup per listed vertex: its prefix goes into the table, and the
+// waves take the rows behind its first entry (64 rows' extents loaded at once,
+// one lane each).  Prefixes of more than TRI_CHUNK entries, the hubs of graphs
+// whose ids do not descend by degree, go in by chunks, and of a row only the
+// entries within the chunk's ids are looked up in it, not every entry once per
+// chunk (a hub after the 200,000 vertices of its wheel 179 -> 8 ms).  They have
+// a list and a launch of their own: the parts below are then counted over them
+// alone (R-MAT-19 with shuffled ids, clipped, 57 -> 18 ms), and the clipping in
+// one kernel with the others cost these 10 % (R-MAT-20 3.5 -> 3.9 ms).  Where
+// the list is short,
 // up to TRI_PARTS workgroups share a vertex, each with its own table and a part
 // of the rows: the rows of one wave are a serial chain.  That and the smaller
 // units of k_triangles_wave, whole call: R-MAT-11 237 -> 97 us, R-MAT-13 332 ->
 // 166, R-MAT-15 435 -> 304, R-MAT-18 unchanged.
-constexpr int TRI_PARTS = 16;
-__global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
-    constexpr int NT = 256, NW = NT / WAVE;
+constexpr int TRI_PARTS = 16, TRI_BLOCK_NT = 256;
+template <bool CHUNKS>
+__global__ __launch_bounds__(TRI_BLOCK_NT) void k_triangles_block(TriArgs a, const int32_t *list,
+                                                                  const int32_t *listed) {
+    constexpr int NT = TRI_BLOCK_NT, NW = NT / WAVE;
     __shared__ int keys[1 << TRI_BLOCK_LOG], cnts[1 << TRI_BLOCK_LOG];
     __shared__ int hot[TRI_HOT];
+    const int nlist = *listed;
+    if (nlist == 0) return;
     for (int i = threadIdx.x; i < TRI_HOT; i += NT) hot[i] = 0;
     const int lane = __lane_id(), w = threadIdx.x / WAVE;
-    const int nlist = *a.listed;
-    const int parts = nlist > 0 ? max(1, min(TRI_PARTS, (int)gridDim.x / nlist)) : 1;
+    const int parts = max(1, min(TRI_PARTS, (int)gridDim.x / nlist));
     const int64_t items = (int64_t)nlist * parts;
     for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
-        const int v = a.list[it / parts];
+        const int v = list[it / parts];
         const int first = (int)(it % parts) * NW + w, step = parts * NW;  // this wave's rows
         const int sv = a.indices[v], len = a.lowpos[v], lab = a.labels ? a.labels[v] : 0;
+        if (!CHUNKS && len > TRI_CHUNK) continue;
         int tv = 0;
         for (int c0 = 0; c0 < len; c0 += TRI_CHUNK) {
             const int c1 = min(len, c0 + TRI_CHUNK);
@@ -301,7 +324,7 @@ __global__ __launch_bounds__(256) void k_triangles_block(TriArgs a) {
                     if (!a.labels || a.labels[u] == lab) {
                         su = a.indices[u];
                         lu = a.lowpos[u];
-                        if (lu > 0 && len > TRI_CHUNK) tri_clip(a, a.adj[sv + c0], a.adj[sv + c1 - 1], su, lu);
+                        if (CHUNKS && lu > 0) tri_clip(a, a.adj[sv + c0], a.adj[sv + c1 - 1], su, lu);
                     }
                 }
                 int found = 0;
@@ -457,10 +480,12 @@ static int ensure_tri_buffers(pcd_ctx *ctx) {
     const int64_t E = (int64_t)2 * ctx->m;
     // prefixes above 64 entries: at most E / 65 vertices, and their number
     const int64_t cap = std::min<int64_t>(ctx->n, E / (TRI_WAVE + 1)) + 1;
+    // and those above one table's
+    const int64_t chunked = ctx->max_degree > TRI_CHUNK ? std::min<int64_t>(ctx->n, E / (TRI_CHUNK + 1)) + 1 : 0;
     auto words = [](int64_t w) { return (w + 63) & ~(int64_t)63; };
     const int64_t per_vertex = words((int64_t)ctx->n + 1), flags = words(E / 4 + 1);
     int32_t *p = nullptr;
-    PCD_TRY(dev_alloc_t(ctx, &p, 5 * per_vertex + flags + words(cap + 1)));
+    PCD_TRY(dev_alloc_t(ctx, &p, 5 * per_vertex + flags + words(cap + 1) + words(chunked + 1)));
     int32_t *at = p + per_vertex;
     auto take = [&](int64_t w) {
         int32_t *x = at;
@@ -473,8 +498,10 @@ static int ensure_tri_buffers(pcd_ctx *ctx) {
     ctx->d_itd = take(per_vertex);
     ctx->d_tri_flag = (uint8_t *)take(flags);
     ctx->d_tri_list = take(words(cap + 1));
+    ctx->d_tri_chunked = chunked ? take(words(chunked + 1)) : nullptr;
+    if (chunked) PCD_TRY(fill_i32(ctx, ctx->d_tri_chunked, 0, 1));
     hipLaunchKernelGGL(k_lowpos, dim3(grid_for(ctx, ctx->n, 256)), dim3(256), 0, ctx->stream, ctx->n, ctx->d_indices,
-                       ctx->d_adj, ctx->d_lowpos);
+                       ctx->d_adj, ctx->d_lowpos, chunked ? ctx->d_tri_chunked + 1 : nullptr, ctx->d_tri_chunked);
     // in the order of the ids, which descend by degree: the listed vertices'
     // work then falls off along the list (R-MAT-16 0.49 ms, in any order 0.51)
     const LongPrefix is_long{ctx->d_lowpos};
@@ -502,10 +529,14 @@ static int count_pass(pcd_ctx *ctx, const int32_t *labels, int32_t *t, int32_t *
                        ctx->stream, words, (uint32_t *)ctx->d_tri_flag, n, t, td);
     // several rounds of workgroups: vertices differ a hundredfold in work
     const int64_t listed = std::min<int64_t>(n, E / (TRI_WAVE + 1)) + 1;  // at most
-    hipLaunchKernelGGL(k_triangles_block, dim3((int)std::min<int64_t>(ctx->cu_count * 24, listed * TRI_PARTS)), dim3(256),
-                       0, ctx->stream, a);
+    const dim3 grid((unsigned)std::min<int64_t>(ctx->cu_count * 24, listed * TRI_PARTS)), block(TRI_BLOCK_NT);
+    if (ctx->d_tri_chunked)
+        hipLaunchKernelGGL(k_triangles_block<true>, grid, block, 0, ctx->stream, a, ctx->d_tri_chunked + 1,
+                           ctx->d_tri_chunked);
+    hipLaunchKernelGGL(k_triangles_block<false>, grid, block, 0, ctx->stream, a, a.list, a.listed);
     const int per = std::min(8, (n + ctx->cu_count * 32 - 1) / (ctx->cu_count * 32));
-    hipLaunchKernelGGL(k_triangles_wave, dim3(grid_for(ctx, n, 4 * per, 24)), dim3(256), 0, ctx->stream, a, per);
+    hipLaunchKernelGGL(k_triangles_wave, dim3(grid_for(ctx, n, 4 * per, 24)), dim3(256), 0, ctx->stream, a, per,
+                       n <= TRI_SPREAD_N);
     hipLaunchKernelGGL(k_tri_degrees, dim3(grid_for(ctx, n, TDEG_NT / 8, 2)), dim3(TDEG_NT), 0, ctx->stream, a, td);
     kt_end(ctx, KS_TRIANGLES);
     PCD_HIP(hipGetLastError());
