@@ -212,6 +212,8 @@ int pcd_bin_counters(pcd_ctx *ctx, int bin, int64_t *active, int64_t *entries, i
  * rows and passes make that the faster way, 2 always) and "fused_pass" (0/1: a
  * device-resident propagation pass under modularity or CPM shares launches
  * between compression, metric, stop rule and bookkeeping) and
+ * "wcc_beside_min_edges" (in a device-resident pass under WCC the metric runs
+ * beside the propagation from this many edges on; default 2^19) and
  * "contract_rows_min" (pcd_contract counts pairs over community rows from this
  * many entries on; default 2^22) and "contract_rows_labels" (... and where the
  * communities' volumes promise at most this many labels among 2,048 entries;

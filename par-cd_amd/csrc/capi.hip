@@ -896,6 +896,9 @@ extern "C" int pcd_set_tuning(pcd_ctx *ctx, const char *key, int value) {
     } else if (k == "contract_rows_labels") {
         if (value < 0) return fail(PCD_E_INVALID, "contract_rows_labels must be >= 0");
         ctx->tune.contract_rows_labels = value;
+    } else if (k == "wcc_beside_min_edges") {
+        if (value < 0) return fail(PCD_E_INVALID, "wcc_beside_min_edges must be >= 0");
+        ctx->tune.wcc_beside_min_edges = value;
     } else if (k == "fused_pass") {
         ctx->tune.fused_pass = value != 0;
     } else if (k == "solo_loop") {

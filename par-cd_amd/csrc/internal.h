@@ -114,6 +114,8 @@ struct Tuning {
                                  // (R-MAT-22 iteration 1.120 ms at 2, 1.102 at 8, 1.131 at 32)
     int graph_loop = 1;          // modularity / CPM with -s 0: passes replayed from one captured
                                  // pass with the stop rule on the device (pcd_iterate_many)
+    int wcc_beside_min_edges = 1 << 19;  // WCC's metric is a branch of its own in the captured pass from this many
+                                 // edges on (loop.hip)
     int contract_rows_min = 1 << 22;  // contraction counts pairs over community rows from this many entries on
     int contract_rows_labels = 512;   // ... and up to this many labels expected in a tile of 2,048 entries
     int fused_pass = 1;          // a captured propagation pass (modularity, CPM) shares launches between its parts

@@ -30,13 +30,6 @@
 
 namespace pcd {
 
-// Edges from which the WCC metric is a branch of its own in the captured pass.
-// A pass with two branches costs more to capture and replay: whole runs on
-// Chung-Lu graphs of 3,000 vertices 2.19 ms with the branch and 1.40 without,
-// 20,000 vertices 2.28 and 1.95, 60,000 vertices (above the line) 2.84 and
-// 2.83-2.98, 200,000 vertices 3.89 and 4.30.
-constexpr int WCC_BESIDE_M = 1 << 18;
-
 __global__ void k_loop_rule(LoopState *s, const double *score, const int32_t *dk, LoopParams p) {
     loop_rule(s, *score, *dk, p);
 }
@@ -184,8 +177,14 @@ static int capture_pass(pcd_ctx *ctx, Loop *L, const pcd_job *job, int cap, int 
         // as the propagation and neither reads the other: it runs beside it
         // on the metric stream, and a pass that turns out to be the last
         // drops its step (Chung-Lu, 1 M vertices: 0.27 of a pass's 0.72 ms).
-        const bool beside = kind == PASS_PROPAGATE && rule.kind == PCD_RULE_WCC && ctx->m >= WCC_BESIDE_M && ctx->mstream && ctx->ev_mfork &&
-                            ctx->ev_metric;
+        // A pass with two branches costs more to capture and replay, so graphs
+        // below wcc_beside_min_edges keep the metric in line (8 passes and the
+        // clustering before them, which makes them captured anew, on Chung-Lu
+        // graphs, beside / in line: 0.17 M edges 2.75 / 2.32 ms, 0.32 M 2.71 /
+        // 2.49, 0.47 M 2.91 / 2.69, 0.64 M 3.39 / 3.73, 1.7 M 4.08 / 4.46, 7.4 M
+        // 7.41 / 8.42; replayed only: 0.47 M 1.78 / 1.75, 0.64 M 1.94 / 2.27).
+        const bool beside = kind == PASS_PROPAGATE && rule.kind == PCD_RULE_WCC &&
+                            ctx->m >= ctx->tune.wcc_beside_min_edges && ctx->mstream && ctx->ev_mfork && ctx->ev_metric;
         hipStream_t main_stream = ctx->stream;
         if (rc == PCD_OK && beside) {
             if (hipEventRecord(ctx->ev_mfork, ctx->stream) != hipSuccess ||

@@ -249,6 +249,46 @@ def test_merging_pass_ranges_then_single_passes():
                 break
 
 
+@pytest.mark.parametrize("streams", [0, 1])
+@pytest.mark.parametrize("strategy", [0, 2])
+@pytest.mark.parametrize("name", ["sbm", "bin_zoo", "unsorted"])
+def test_wcc_metric_beside_the_propagation(name, strategy, streams):
+    """WCC passes whose metric is a branch of the captured graph beside the
+    propagation (every size, by its tunable), and in line: both equal the
+    per-pass loop, stopped by the score, by -n on either kind of pass, by the
+    iteration cap and by the end of a range of passes; with the hub rows on
+    side streams too."""
+    n, m, ind, adj, _ = graphs()[name]
+    lab = (np.arange(n) // 23).astype(np.int32)
+    got = []
+    for loop, least in ((0, 0), (1, 0), (1, 1 << 30)):
+        with parcd.Context(0) as c:
+            c.set_tuning("graph_loop", loop)
+            c.set_tuning("wcc_beside_min_edges", least)
+            c.set_tuning("bin_streams", streams)
+            c.set_tuning("bin_streams_min_edges", 0)
+            c.upload_graph(n, m, ind, adj)
+            c.triangles()
+            one = []
+            for jb in (parcd.job(kind=O.WCC, seed=3, iter_cap=30), parcd.job(kind=O.WCC, seed=4, max_iter=5),
+                       parcd.job(kind=O.WCC, seed=4, max_iter=6), parcd.job(kind=O.WCC, seed=5, iter_cap=4, threshold=-1.0)):
+                one.append(outcome(c, lab, jb, strategy, 1))
+            jb = parcd.job(kind=O.WCC, seed=6, max_iter=50)
+            c.upload_labels(lab)
+            it, prev = 0, 0.0
+            for count in (1, 4, 3):
+                ran, prev, k, done = (c.iterate_many(jb, it, count, prev, strategy=strategy) if loop else
+                                      per_pass(c, jb, it, count, prev, strategy=strategy))
+                assert ran == count and not done
+                it += ran
+                one.append([prev, k, O.compress_labels(c.labels())[0]])
+            one.append(list(c.iterate(jb, it, prev, strategy=strategy)) + [O.compress_labels(c.labels())[0]])
+            got.append(one)
+    for other in got[1:]:
+        for x, y in zip(got[0], other):
+            assert len(x) == len(y) and all(np.array_equal(a, b) for a, b in zip(x, y))
+
+
 def outcome(ctx, lab, jb, strategy, rounds):
     ctx.upload_labels(lab)
     score, it, k = ctx.refine(jb, strategy=strategy, rounds=rounds)

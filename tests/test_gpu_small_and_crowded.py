@@ -486,7 +486,6 @@ def test_batch_rows_of_every_width(cut):
 
 @pytest.mark.parametrize("n", [200, 1025, 3001])
 def test_wcc_loop_of_a_small_graph(n):
-    # below 2^18 edges the captured pass holds the metric in line
     rng = np.random.default_rng(n)
     deg = 12
     a = np.repeat(np.arange(n), deg)
