@@ -416,7 +416,8 @@ int collect_statistics_dev(pcd_ctx *ctx) {
 // t - nsmall (its entry is the item index), and a last index with flag 0
 // closes the list.  The scan keeps position order, so the small bins'
 // moved vertices come out grouped by bin; bounds[b] (b < 5) is where bin b
-// starts, bounds[5] where the items start and bounds[6] the total.
+// starts, bounds[5] where the items start and bounds[6] the total; bounds[7]
+// starts k_moved_bits' count at 0.
 struct MovedArgs {
     int s[6];  // small bins G64..G4: positions [s[b], s[b+1])
     int nitems;
@@ -451,7 +452,10 @@ struct MovedStore {
         for (int b = 0; b < 5; b++)
             if (t == a.s[b] - a.s[0]) bounds[b] = ex;
         if (t == nsmall) bounds[5] = ex;
-        if (t == nsmall + a.nitems) bounds[6] = ex;
+        if (t == nsmall + a.nitems) {
+            bounds[6] = ex;
+            bounds[7] = 0;
+        }
         if (!flag) return;
         if (t < nsmall) {
             const int p = a.s[0] + (int)t;
@@ -465,9 +469,16 @@ struct MovedStore {
 // Moved bitmap: bit v of M is set when vertex v's label changed in the step
 // (L[v] != N[v]).  One wave writes one 64-bit word.
 // With dk set (a captured pass) it also starts the next compression's
-// first-occurrence table, as k_first_init does.
+// first-occurrence table, as k_first_init does.  Every CROWD_SAMPLE-th
+// workgroup counts the moved vertices that share the old or the new community
+// of another of their wave: *crowd tells crowded steps (see
+// k_delta_crowded).
+constexpr int CROWD_SAMPLE = 16;
 __global__ __launch_bounds__(256) void k_moved_bits(int n, const int32_t *L, const int32_t *N, uint64_t *M,
-                                                    const int32_t *dk, const int32_t *firstv, int32_t *first) {
+                                                    const int32_t *dk, const int32_t *firstv, int32_t *first,
+                                                    int32_t *crowd) {
+    const bool sample = blockIdx.x % CROWD_SAMPLE == 0;
+    int shared = 0;
     if (dk) {
         const int k = *dk;
         for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += gridDim.x * blockDim.x) {
@@ -481,9 +492,17 @@ __global__ __launch_bounds__(256) void k_moved_bits(int n, const int32_t *L, con
     const int nwaves = gridDim.x * blockDim.x / WAVE;
     for (int wd = wave_g; wd < nwords; wd += nwaves) {
         const int v = wd * WAVE + lane;
-        const uint64_t bits = __ballot(v < n && L[v] != N[v]);
+        const int lo = v < n ? L[v] : 0, ln = v < n ? N[v] : 0;
+        const uint64_t bits = __ballot(lo != ln);
         if (lane == 0) M[wd] = bits;
+        if (sample && bits) {
+            const int one = __builtin_ctzll(bits);
+            shared += __popcll(__ballot(lo != ln && lo == __builtin_amdgcn_readlane(lo, one))) - 1;
+            if (__builtin_amdgcn_readlane(ln, one) >= 0)  // leaving vertices join nothing
+                shared += __popcll(__ballot(lo != ln && ln == __builtin_amdgcn_readlane(ln, one))) - 1;
+        }
     }
+    if (sample && lane == 0 && shared) atomicAdd(crowd, shared);
 }
 
 // A neighbour's label before the step is its label after the step (already
@@ -503,9 +522,15 @@ struct DeltaArgs {
 __device__ inline int label_before(const DeltaArgs &a, int w, int after) {
     return !a.M || ((a.M[w >> 6] >> (w & 63)) & 1) ? a.L[w] : after;
 }
-template <int G>
-__device__ inline void delta_batch(const DeltaArgs &d, int left, int v, const HotLabels &after,
-                                   StatsAcc<DELTA_LOG> &acc) {
+struct DirectSums {  // no accumulators between a row and the records
+    __device__ void add(CommStats *st, int l, int size, int same, int e) { add_stats(st, l, size, same, e); }
+};
+struct PlainLabels {
+    const int32_t *labels;
+    __device__ int operator()(int v) const { return labels[v]; }
+};
+template <int G, class After, class Sums>
+__device__ inline void delta_batch(const DeltaArgs &d, int left, int v, const After &after, Sums &acc) {
     const int lane = __lane_id(), glane = lane & (G - 1);
     constexpr int per_wave = WAVE / G;
     int bstart = 0, bdeg = 0, blo = 0, bln = 0;
@@ -550,9 +575,9 @@ __device__ inline void delta_batch(const DeltaArgs &d, int left, int v, const Ho
     }
 }
 // a wave takes up to DELTA_BATCH entries of the bin's list at once
-template <int G>
+template <int G, class After, class Sums>
 __device__ inline void delta_small(const DeltaArgs &d, int wave_g, int nwaves, const int32_t *list, int cnt,
-                                   const HotLabels &after, StatsAcc<DELTA_LOG> &acc) {
+                                   const After &after, Sums &acc) {
     constexpr int per_wave = WAVE / G;
     const int lane = __lane_id();
     // entries per batch: a multiple of per_wave that leaves no wave idle
@@ -565,8 +590,8 @@ __device__ inline void delta_small(const DeltaArgs &d, int wave_g, int nwaves, c
 }
 
 // One long-row item {v, begin, end, first} of a moved vertex, the whole wave
-__device__ inline void delta_item(const DeltaArgs &d, const int4 &w, int lo, int ln, const HotLabels &after,
-                                  StatsAcc<DELTA_LOG> &acc) {
+template <class After, class Sums>
+__device__ inline void delta_item(const DeltaArgs &d, const int4 &w, int lo, int ln, const After &after, Sums &acc) {
     constexpr int PF = 8;
     const int lane = __lane_id();
     int a = 0, b = 0;
@@ -602,8 +627,9 @@ __device__ inline void delta_item(const DeltaArgs &d, const int4 &w, int lo, int
 // Moved items, one wave each: workgroup wg of nwg takes list entries wg,
 // wg + nwg, ..., its waves whichever comes next (rows differ 30-fold in
 // length), and the next item's records are on their way while one is counted.
+template <class After, class Sums>
 __device__ inline void delta_items(const DeltaArgs &d, int wg, int nwg, int *next, const int32_t *list, int cnt,
-                                   const int4 *items, const HotLabels &after, StatsAcc<DELTA_LOG> &acc) {
+                                   const int4 *items, const After &after, Sums &acc) {
     const int lane = __lane_id();
     int4 wn = make_int4(0, 0, 0, 0);
     int lon = 0, lnn = 0;
@@ -627,35 +653,94 @@ __device__ inline void delta_items(const DeltaArgs &d, int wg, int nwg, int *nex
     }
 }
 
-// All six moved lists in one launch: every wave takes its share of each list
-// in turn, from a place in the list that differs by list, so that short
-// lists fall to different waves and the lists' dependent-load chains overlap.
-// The sums go through the workgroup's accumulators: in a step that moves many
-// vertices into few communities the atomics on their records were the bound
-// (first step of CPM 0.01 on R-MAT-20, 15.7 M entries: 1.28 ms, now 0.22).
-// One resident round of workgroups: more of them measured slower once few
-// vertices move (24 us at twice as many, 12 us here), because every
-// workgroup pays the accumulators' start and flush.
-constexpr int DELTA_NT = 1024, DELTA_HOT_ITEMS = 2;
-__global__ __launch_bounds__(DELTA_NT) void k_delta_all(int n, const int32_t *list, const int32_t *bounds,
-                                                        const int4 *items, DeltaArgs d, LoopState *state) {
-    if (state && blockIdx.x == 0 && threadIdx.x == 0) loop_next(state);  // a captured pass ends here
-    int bd[7];  // read at once: a read per list would lengthen every wave's chain
+// All six moved lists in one launch, so that the lists' short chains of
+// dependent loads overlap.  Every workgroup reads the list bounds and computes
+// the same split of the grid into ranges, one per list, in proportion to the
+// lists' entries (a long-row item as DELTA_ITEM_COST), at least one workgroup
+// for a list that is not empty.  The sums go to the records directly, and small
+// workgroups finish unevenly and leave room to the next (modularity from
+// singletons, steps 1 to 6: R-MAT-18 38 24 18 15 13 12 us, R-MAT-22 670 330 177
+// 103 64 46; as k_delta_crowded 66 43 34 25 21 18 and 642 354 200 132 100 77).
+// Crowded steps are left to k_delta_crowded.
+constexpr int DELTA_NT = 256, DELTA_ITEM_COST = 512, DELTA_PER_CU = 24;
+// moved vertices that share a community with another of their wave, among the
+// sampled: about as many atomics on one record as take 5 us
+constexpr int CROWDED = 512 / CROWD_SAMPLE;
+__global__ __launch_bounds__(DELTA_NT) void k_delta_all(const int32_t *list, const int32_t *bounds, const int4 *items,
+                                                        DeltaArgs d) {
+    int bd[8];
 #pragma unroll
-    for (int i = 0; i < 7; i++) bd[i] = bounds[i];
-    if (bd[0] == bd[6]) return;  // nothing moved
+    for (int i = 0; i < 8; i++) bd[i] = bounds[i];
+    if (bd[0] == bd[6] || bd[7] > CROWDED) return;
+    // this workgroup's list, and its place among the list's workgroups
+    constexpr int cost[6] = {64, 32, 16, 8, 4, DELTA_ITEM_COST};
+    float total = 0.0f, before = 0.0f;
+    int nonempty = 0, at = 0, mine = -1, wg = 0, nwg = 1;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        total += (float)(bd[i + 1] - bd[i]) * cost[i];
+        nonempty += bd[i + 1] > bd[i];
+    }
+    const float per = (float)((int)gridDim.x - nonempty) / total;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        if (bd[i + 1] == bd[i]) continue;
+        const float upto = before + (float)(bd[i + 1] - bd[i]) * cost[i];
+        const int count = 1 + ((int)(upto * per) - (int)(before * per));
+        if ((int)blockIdx.x >= at && (int)blockIdx.x < at + count) {
+            mine = i;
+            wg = (int)blockIdx.x - at;
+            nwg = count;
+        }
+        at += count;
+        before = upto;
+    }
+    if (mine < 0) return;  // beyond the last range
+    __shared__ int next;
+    if (threadIdx.x == 0) next = 0;
+    __syncthreads();
+    const int wave_g = wg * (DELTA_NT / WAVE) + (int)threadIdx.x / WAVE, nwaves = nwg * (DELTA_NT / WAVE);
+    const PlainLabels after{d.N};
+    DirectSums sums;
+    switch (mine) {
+    case 0: delta_small<64>(d, wave_g, nwaves, list + bd[0], bd[1] - bd[0], after, sums); break;
+    case 1: delta_small<32>(d, wave_g, nwaves, list + bd[1], bd[2] - bd[1], after, sums); break;
+    case 2: delta_small<16>(d, wave_g, nwaves, list + bd[2], bd[3] - bd[2], after, sums); break;
+    case 3: delta_small<8>(d, wave_g, nwaves, list + bd[3], bd[4] - bd[3], after, sums); break;
+    case 4: delta_small<4>(d, wave_g, nwaves, list + bd[4], bd[5] - bd[4], after, sums); break;
+    default: delta_items(d, wg, nwg, &next, list + bd[5], bd[6] - bd[5], items, after, sums); break;
+    }
+}
+
+// The same for a crowded step, one that moves many vertices into or out of few
+// communities: the atomics on those communities' records are the bound, so the
+// sums go through the workgroup's accumulators (first step of CPM 0.01 on
+// R-MAT-20, 15.7 M entries: 1.28 ms without, 0.22 with).  Every wave takes its
+// share of each list in turn, from a place in the list that differs by list.
+// One resident round of workgroups: every workgroup pays the accumulators'
+// start and flush (0.34 ms with 2,048 workgroups of 256 threads).
+constexpr int CROWD_NT = 1024, DELTA_HOT_ITEMS = 2;
+constexpr int64_t DELTA_ONE = 1 << 18;
+__global__ __launch_bounds__(CROWD_NT) void k_delta_crowded(int n, int least, const int32_t *list,
+                                                            const int32_t *bounds, const int4 *items, DeltaArgs d,
+                                                            LoopState *state) {
+    if (state && blockIdx.x == 0 && threadIdx.x == 0) loop_next(state);  // a captured pass ends here
+    int bd[8];  // read at once: a read per list would lengthen every wave's chain
+#pragma unroll
+    for (int i = 0; i < 8; i++) bd[i] = bounds[i];
+    if (bd[0] == bd[6] || bd[7] <= least) return;
     __shared__ int32_t hot[STATS_CACHE];
     __shared__ StatsAcc<DELTA_LOG> acc;
     __shared__ int next;
-    const int nwaves = gridDim.x * DELTA_NT / WAVE;
+    const int nwaves = gridDim.x * CROWD_NT / WAVE;
     // with several long-row items a wave, the labels of the most frequent
     // neighbours are staged in LDS (as in k_stats_rows)
     const HotLabels after{hot, d.N, bd[6] - bd[5] >= DELTA_HOT_ITEMS * nwaves ? min(n, STATS_CACHE) : 0};
-    for (int i = threadIdx.x; i < after.n; i += DELTA_NT) hot[i] = d.N[i];
+    for (int i = threadIdx.x; i < after.n; i += CROWD_NT) hot[i] = d.N[i];
     if (threadIdx.x == 0) next = 0;
     acc.init();
     __syncthreads();
-    const int wave_g = (blockIdx.x * DELTA_NT + threadIdx.x) / WAVE;
+    const int wave_g = (blockIdx.x * CROWD_NT + threadIdx.x) / WAVE;
     auto place = [&](int i) {
         const int w = wave_g + i * (nwaves / 6);
         return w < nwaves ? w : w - nwaves;
@@ -677,8 +762,8 @@ __global__ __launch_bounds__(DELTA_NT) void k_delta_all(int n, const int32_t *li
 // closes a captured pass.
 constexpr int DIRECT_MAX_N = 1 << 16, DIRECT_NT = 512;
 template <int G>
-__device__ inline void delta_positions(const DeltaArgs &d, const MovedArgs &m, int b, int wave_g, int nwaves,
-                                       const HotLabels &after, int *list, StatsAcc<DELTA_LOG> &acc) {
+__device__ inline void delta_positions(const DeltaArgs &d, const MovedArgs &m, int b, int wave_g, int nwaves, int *list,
+                                       StatsAcc<DELTA_LOG> &acc) {
     const int lane = __lane_id();
     // no wider than the bin leaves every wave busy
     const int count = m.s[b + 1] - m.s[b];
@@ -695,7 +780,7 @@ __device__ inline void delta_positions(const DeltaArgs &d, const MovedArgs &m, i
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const int left = __popcll(mm);
-        delta_batch<G>(d, left, lane < left ? list[lane] : 0, after, acc);
+        delta_batch<G>(d, left, lane < left ? list[lane] : 0, PlainLabels{d.N}, acc);
         __builtin_amdgcn_wave_barrier();
     }
 }
@@ -711,21 +796,19 @@ __global__ __launch_bounds__(DIRECT_NT) void k_delta_direct(MovedArgs m, DeltaAr
     }
     acc.init();
     __syncthreads();
-    const int lane = __lane_id(), w = threadIdx.x / WAVE;
+    const int w = threadIdx.x / WAVE;
     const int nwaves = gridDim.x * DIRECT_NT / WAVE, wave_g = blockIdx.x * DIRECT_NT / WAVE + w;
     auto place = [&](int i) { return (wave_g + i * (nwaves / 6)) % nwaves; };
-    const HotLabels after{s_list[w], d.N, 0};
     for (int i = wave_g; i < m.nitems; i += nwaves) {
         const int4 it = m.items[i];
         const int lo = d.L[it.x], ln = d.N[it.x];
-        if (lo != ln) delta_item(d, it, lo, ln, after, acc);
+        if (lo != ln) delta_item(d, it, lo, ln, PlainLabels{d.N}, acc);
     }
-    delta_positions<64>(d, m, 0, place(1), nwaves, after, s_list[w], acc);
-    delta_positions<32>(d, m, 1, place(2), nwaves, after, s_list[w], acc);
-    delta_positions<16>(d, m, 2, place(3), nwaves, after, s_list[w], acc);
-    delta_positions<8>(d, m, 3, place(4), nwaves, after, s_list[w], acc);
-    delta_positions<4>(d, m, 4, place(5), nwaves, after, s_list[w], acc);
-    (void)lane;
+    delta_positions<64>(d, m, 0, place(1), nwaves, s_list[w], acc);
+    delta_positions<32>(d, m, 1, place(2), nwaves, s_list[w], acc);
+    delta_positions<16>(d, m, 2, place(3), nwaves, s_list[w], acc);
+    delta_positions<8>(d, m, 3, place(4), nwaves, s_list[w], acc);
+    delta_positions<4>(d, m, 4, place(5), nwaves, s_list[w], acc);
     __syncthreads();
     acc.flush(d.st);
 }
@@ -757,11 +840,18 @@ int statistics_delta_dev(pcd_ctx *ctx, const int32_t *before, const int32_t *aft
     PCD_TRY(device_scan(ctx, len, MovedFlag{m}, MovedStore{m, bounds, list}, nullptr));
     hipLaunchKernelGGL(k_moved_bits, dim3(grid_for(ctx, (ctx->n + WAVE - 1) / WAVE, 4, 8)), dim3(256), 0, ctx->stream,
                        ctx->n, before, after, ctx->d_moved_bits, ctx->fused ? ctx->d_k : nullptr, ctx->d_firstv,
-                       ctx->d_first);
-    // two workgroups per CU, fewer for a small graph
-    const int delta_grid = std::max(8, grid_for(ctx, 2 * (int64_t)ctx->m, 2048, 2));
-    hipLaunchKernelGGL(k_delta_all, dim3(delta_grid), dim3(DELTA_NT), 0, ctx->stream, ctx->n, list, bounds,
-                       ctx->d_stat_items, d, ctx->fused);
+                       ctx->d_first, bounds + 7);
+    // one of the two has work; fewer workgroups for small graphs, and of graphs
+    // below DELTA_ONE entries the second takes every step: a launch more is
+    // what they would notice (R-MAT-12, 97,000 entries: 27 to 22 us a step
+    // either way)
+    const int64_t E = 2 * (int64_t)ctx->m;
+    const bool one = E < DELTA_ONE;
+    if (!one)
+        hipLaunchKernelGGL(k_delta_all, dim3(std::max(8, grid_for(ctx, E, 1024, DELTA_PER_CU))), dim3(DELTA_NT), 0,
+                           ctx->stream, list, bounds, ctx->d_stat_items, d);
+    hipLaunchKernelGGL(k_delta_crowded, dim3(std::max(8, grid_for(ctx, E, 2048, 2))), dim3(CROWD_NT), 0, ctx->stream,
+                       ctx->n, one ? -1 : CROWDED, list, bounds, ctx->d_stat_items, d, ctx->fused);
     kt_end(ctx, KS_STATS_DELTA);
     PCD_HIP(hipGetLastError());
     return PCD_OK;

@@ -30,6 +30,8 @@ def crowded(kind, n):
     v = np.arange(n)
     if kind == "one":
         return np.full(n, n - 1, np.int32)
+    if kind == "singletons":  # hardly two members of a wave share one
+        return rng.permutation(n).astype(np.int32)
     if kind == "half":  # one community of half the vertices among singletons
         return np.where(rng.random(n) < 0.5, n // 2, v).astype(np.int32)
     if kind == "table":  # more communities than a workgroup's accumulators, some of them large
@@ -37,13 +39,15 @@ def crowded(kind, n):
     return np.where(rng.random(n) < 0.1, -1, v % 7).astype(np.int32)  # seven communities and NEW_LABEL vertices
 
 
-@pytest.mark.parametrize("kind", ["one", "half", "table", "seven_new"])
-@pytest.mark.parametrize("graph", ["bin_zoo", "unsorted", "rmat12", "star"])
+@pytest.mark.parametrize("kind", ["one", "half", "table", "seven_new", "singletons"])
+@pytest.mark.parametrize("graph", ["bin_zoo", "unsorted", "rmat12", "rmat14", "star"])
 def test_statistics_of_crowded_partitions(ctx, graph, kind):
     """Compression, the full count, and the statistics updated from the moved
-    rows over four steps (crowded communities lose and gain many members at
-    once) equal the oracle's full count, for both tie orders."""
-    g = {"bin_zoo": GG.bin_zoo, "unsorted": lambda: GG.unsorted_copy(GG.bin_zoo()), "rmat12": lambda: GG.rmat(12),
+    rows over four steps equal the oracle's full count, for both tie orders:
+    crowded communities lose and gain many members at once, or none does, on
+    graphs on both sides of the entries from which the two kinds of step have
+    a kernel each."""
+    g = {"bin_zoo": GG.bin_zoo, "rmat14": lambda: GG.rmat(14), "unsorted": lambda: GG.unsorted_copy(GG.bin_zoo()), "rmat12": lambda: GG.rmat(12),
          "star": lambda: GG.csr_direct(700, [(0, i) for i in range(1, 700)])}[graph]()
     n, m, ind, adj = g[:4]
     ctx.upload_graph(n, m, ind, adj)
@@ -363,7 +367,7 @@ def test_merging_of_crowded_partitions(ctx, graph, kind):
     g = {"bin_zoo": GG.bin_zoo, "rmat12": lambda: GG.rmat(12), "no_edges": lambda: GG.csr_direct(6, []),
          "star": lambda: GG.csr_direct(2049, [(0, i) for i in range(1, 2049)])}[graph]()
     n, m, ind, adj = g[:4]
-    lab = np.arange(n, dtype=np.int32) if kind == "singletons" else crowded(kind, n)
+    lab = crowded(kind, n)
     ctx.upload_graph(n, m, ind, adj)
     for rule, lam, rounds, tie in ((O.MOD, 0.0, 1, 0), (O.CPM, 0.001, 3, 1)):
         got = []
@@ -434,8 +438,6 @@ def test_contraction_by_rows_and_by_sort(ctx, graph, kind):
         lab = (np.arange(n) * 40 // n).astype(np.int32)
     elif kind == "sparse_ids":
         lab = (np.arange(n) % 61 * (n // 64)).astype(np.int32)  # not compressed: empty rows between
-    elif kind == "singletons":
-        lab = np.random.default_rng(5).permutation(n).astype(np.int32)
     else:
         lab = crowded(kind, n)
     ctx.upload_graph(n, m, ind, adj)
