@@ -879,10 +879,10 @@ def main():
     lp_phase = {"ms_per_step": lp_ms / args.steps, "gbs": lp_bytes / (lp_ms / 1000.0) / 1e9 if lp_ms else None,
                 "gteps_EA": tot_e / (lp_ms / 1000.0) / 1e9 if lp_ms else None,
                 "E_A_per_step": tot_e / args.steps, "D_per_step": tot_d / args.steps}
-    # statistics: a full recount (stats_items + stats_small) when the labels
-    # came from outside the loop, else the update from the moved vertices'
+    # statistics: a full recount (stats_items) when the labels came from
+    # outside the loop, else the update from the moved vertices'
     # rows (stats_delta) that each propagation step runs
-    recount_ms = timers.get("stats_items", (0, 0))[0] + timers.get("stats_small", (0, 0))[0]
+    recount_ms = timers.get("stats_items", (0, 0))[0]
     delta_ms = timers.get("stats_delta", (0, 0))[0]
     stats_ms = recount_ms + delta_ms
     stats_bytes = (8 * E + 8 * n + 12 * n) * args.steps

@@ -92,11 +92,12 @@ int pcd_compress_labels(pcd_ctx *ctx, int *num_labels);
  * compressed labels and *num_labels (one device int32) receives k, or -1
  * when a label lies outside [-1, n).  `stream` is a hipStream_t (NULL: the
  * null stream); the call only enqueues kernels and returns.  labels and
- * out_labels must be different arrays.  Scratch (first-occurrence and
- * new-id tables, scan partials) is a file-scope device array of about
+ * out_labels must be different arrays.  Up to 36,864 labels the scratch is one
+ * workgroup's LDS, and calls may overlap.  Above that, scratch (first-occurrence
+ * and new-id tables, scan partials) is a file-scope device array of about
  * 32 MiB that each device holds until the process ends: n is limited to
- * PCD_NOALLOC_MAX_VERTICES (PCD_E_INVALID above).  Every call on one device
- * shares that array, so calls that overlap in time on one device race.
+ * PCD_NOALLOC_MAX_VERTICES (PCD_E_INVALID above), and calls of these sizes that
+ * overlap in time on one device race.
  * No hipMalloc, hipFree, hipMemset or allocating library routine is called. */
 #define PCD_NOALLOC_MAX_VERTICES 4194304
 int pcd_compress_labels_noalloc(int n, const int32_t *labels, int32_t *out_labels, int32_t *num_labels,
@@ -135,7 +136,10 @@ int pcd_merging_step(pcd_ctx *ctx, pcd_rule rule, int rounds, uint64_t seed, int
  * (l, k, links) for l != k, sorted by (l, k) -- the table MergingRefinement
  * builds at refinement.cpp:228-238 and framework-cuda.cu:744-807 computes by
  * sort + reduce-by-key.  *num_pairs receives U; arrays (may be NULL) need U
- * entries; call first with NULL arrays to get U. */
+ * entries; call first with NULL arrays to get U.  The first call reserves 24
+ * bytes per CSR entry, and where it counts over community rows (tunables
+ * contract_rows_min, contract_rows_labels) 4 more per entry and 12 per vertex,
+ * which the merging step shares; they are kept until the graph is replaced. */
 int pcd_contract(pcd_ctx *ctx, int64_t *num_pairs, int32_t *l, int32_t *k, int32_t *links);
 
 /* Graph::count_triangles (graph.cpp:107-175): per-vertex tri (twice the

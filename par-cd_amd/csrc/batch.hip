@@ -225,7 +225,7 @@ __device__ inline void stats_rows_item(const WorkItem &w, const BatchGraph &g) {
 }
 
 // Statistics after a propagation step, from the moved vertices only (the
-// update of partition.hip's k_delta_small / k_delta_items): cur holds the
+// update of partition.hip's k_delta_all): cur holds the
 // labels the step read (L), next those it wrote (N), and the records of
 // graphs whose statistics follow the labels are brought from L to N under
 // L's ids; the compression that follows renumbers them.
@@ -330,7 +330,7 @@ __device__ inline void delta_rows_item(const WorkItem &w, const BatchGraph &g) {
 // waves, so that short lists do not all fall to the first ones.  A round of
 // small graphs is bound by its launches: six row lists in one launch twice, the
 // four passes over the vertices after the scan in one, and the first-occurrence
-// fill beside the update take 14 of 31 away.  256 block-model graphs of 50 to
+// fill beside the update take 14 of 33 away.  256 block-model graphs of 50 to
 // 20,000 vertices, admission and results included: 63.4 -> 57.4 ms.
 struct RowLists {
     const WorkItem *items[6];

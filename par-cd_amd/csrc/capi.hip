@@ -77,7 +77,7 @@ void kt_end(pcd_ctx *ctx, int slot) {
 }
 
 static const char *kslot_names[NUM_KSLOTS] = {
-    "compress", "stats_items", "stats_small", "metric", "lp_records", "lp_hub_partition", "lp_hub_count",
+    "compress", "stats_items", "metric", "lp_records", "lp_hub_partition", "lp_hub_count",
     "lp_b4096", "lp_b1024", "lp_w256", "lp_g64", "lp_g32", "lp_g16", "lp_g8", "lp_g4",
     "merge_keys", "merge_sort", "merge_rle", "merge_rounds", "triangles", "stats_delta", "lp_small",
     "lp_b512", "lp_hub_final", "merge_stats"};
@@ -587,15 +587,6 @@ extern "C" int pcd_collect_statistics(pcd_ctx *ctx, int *num_labels) {
     phase_end(ctx, PCD_PHASE_STATS);
     if (num_labels) *num_labels = ctx->k;
     return PCD_OK;
-}
-
-__global__ void k_split_stats(int k, const CommStats *st, int32_t *s, int32_t *iv, int32_t *ev) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < k; c += gridDim.x * blockDim.x) {
-        CommStats x = st[c];
-        s[c] = x.size;
-        iv[c] = x.int_vol;
-        ev[c] = x.ext_vol;
-    }
 }
 
 extern "C" int pcd_stats_download(pcd_ctx *ctx, int32_t *sizes, int32_t *int_volume, int32_t *ext_volume) {

@@ -136,7 +136,7 @@ constexpr int HUB_PARTIAL_BYTES = 32; // storage per (hub, partition) partial re
 
 // Kernel timer slots (HIP events around each launch when timing is on).
 enum KSlot {
-    KS_COMPRESS = 0, KS_STATS_ITEMS, KS_STATS_SMALL, KS_METRIC,
+    KS_COMPRESS = 0, KS_STATS_ITEMS, KS_METRIC,
     KS_LP_SELECT, KS_LP_HUB_INSERT, KS_LP_HUB_DECIDE, KS_LP_B4096, KS_LP_B1024, KS_LP_W256,
     KS_LP_G64, KS_LP_G32, KS_LP_G16, KS_LP_G8, KS_LP_G4,
     KS_MERGE_KEYS, KS_MERGE_SORT, KS_MERGE_RLE, KS_MERGE_ROUNDS, KS_TRIANGLES, KS_STATS_DELTA, KS_LP_SMALL,

@@ -11,8 +11,8 @@
 // label's first[] or NEW_LABEL, and the exclusive scan of those flags over
 // v is the reference's running counter.  The output is bit-identical.
 //
-// Every call on one device shares that device's array and overwrites what
-// the last call left there; calls that overlap in time on one device race.
+// Calls above NA_SOLO labels share their device's array and overwrite what the
+// last one left there; those that overlap in time on one device race.
 #include <algorithm>
 #include <mutex>
 
@@ -77,9 +77,12 @@ __global__ __launch_bounds__(NF_NT) void k_na_first(int n, const int32_t *labels
 // holds CH chunks of 64 consecutive labels in registers, read at once.  The
 // table in LDS holds the least vertex of every label, then the complement of
 // its new id (negative, so a later test for "am I the least" stays false).
-// Seven launches took 26 us for 4,000 labels and 30 us for 36,000, most of it
-// their floors; one takes 4 and 23 us, and beyond its table's LDS the tiled
-// form is the faster one.
+// Seven launches take 20-24 us whatever the labels, most of it their floors;
+// one takes 6 us for 4,000 labels in many communities, 12 for 20,000, 17 for
+// 28,000 and 24 for 36,000, the most its table in LDS holds.  Labels that fall
+// into one community queue on its word: 7, 27, 37 and 48 us.  A build costs what
+// it has registers for (4,096 labels in the builds for 4, 8, 12, 20, 28 and 36
+// thousand: 5.8, 6.0, 6.4, 8.5, 10.6 and 14.7 us), so there are six.
 constexpr int NA_CH = 36, NA_SOLO = NA_CH * 1024;
 template <int CH>
 __global__ __launch_bounds__(1024) void k_na_solo(int n, const int32_t *labels, int32_t *out, int32_t *num_labels) {
