@@ -282,6 +282,7 @@ struct pcd_ctx {
     uint8_t *d_tri_flag = nullptr;  // per entry: on a counted triangle
     int32_t *d_tri_list = nullptr;  // number of vertices with long prefixes, then the vertices
     int32_t *d_tri_chunked = nullptr;  // the same for prefixes of several tables, or null: no row is that long
+    int tri_chunked = -1;              // their number, once it is known
     int32_t *d_lowpos = nullptr, *d_it = nullptr, *d_itd = nullptr;
     double cc = 0.0;
 

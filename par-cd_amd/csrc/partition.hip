@@ -663,9 +663,12 @@ __device__ inline void delta_items(const DeltaArgs &d, int wg, int nwg, int *nex
 // 103 64 46; as k_delta_crowded 66 43 34 25 21 18 and 642 354 200 132 100 77).
 // Crowded steps are left to k_delta_crowded.
 constexpr int DELTA_NT = 256, DELTA_ITEM_COST = 512, DELTA_PER_CU = 24;
-// moved vertices that share a community with another of their wave, among the
-// sampled: about as many atomics on one record as take 5 us
-constexpr int CROWDED = 512 / CROWD_SAMPLE;
+// Moved vertices that share a community with another of their wave, among the
+// sampled, up to which a step is not crowded.  Steps that both kernels took:
+// counts up to 1, 38 us direct and 51 with accumulators (R-MAT-18, modularity),
+// 101 and 141 (R-MAT-22); 2 and 3, 64 and 46, 48 and 39 (Chung-Lu graphs, WCC);
+// from 4 on, 62 and 51 to 1465 and 120.
+constexpr int CROWDED = 2;
 __global__ __launch_bounds__(DELTA_NT) void k_delta_all(const int32_t *list, const int32_t *bounds, const int4 *items,
                                                         DeltaArgs d) {
     int bd[8];

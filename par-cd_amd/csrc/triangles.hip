@@ -458,7 +458,9 @@ __global__ __launch_bounds__(256) void k_wcc_partial(int n, const int32_t *label
     }
 }
 
-__global__ __launch_bounds__(256) void k_sum_partials_plain(const double *part, int np, double *out) {
+// (with `count` set, out[1] receives it: one copy brings both to the host)
+__global__ __launch_bounds__(256) void k_sum_partials_plain(const double *part, int np, double *out,
+                                                            const int32_t *count) {
     __shared__ double lds[256 / WAVE];
     double acc = 0;
     for (int i = threadIdx.x; i < np; i += blockDim.x) acc += part[i];
@@ -469,6 +471,7 @@ __global__ __launch_bounds__(256) void k_sum_partials_plain(const double *part, 
         double t = 0;
         for (int i = 0; i < 256 / WAVE; i++) t += lds[i];
         *out = t;
+        if (count) out[1] = *count;
     }
 }
 
@@ -499,6 +502,7 @@ static int ensure_tri_buffers(pcd_ctx *ctx) {
     ctx->d_tri_flag = (uint8_t *)take(flags);
     ctx->d_tri_list = take(words(cap + 1));
     ctx->d_tri_chunked = chunked ? take(words(chunked + 1)) : nullptr;
+    ctx->tri_chunked = -1;
     if (chunked) PCD_TRY(fill_i32(ctx, ctx->d_tri_chunked, 0, 1));
     hipLaunchKernelGGL(k_lowpos, dim3(grid_for(ctx, ctx->n, 256)), dim3(256), 0, ctx->stream, ctx->n, ctx->d_indices,
                        ctx->d_adj, ctx->d_lowpos, chunked ? ctx->d_tri_chunked + 1 : nullptr, ctx->d_tri_chunked);
@@ -530,7 +534,7 @@ static int count_pass(pcd_ctx *ctx, const int32_t *labels, int32_t *t, int32_t *
     // several rounds of workgroups: vertices differ a hundredfold in work
     const int64_t listed = std::min<int64_t>(n, E / (TRI_WAVE + 1)) + 1;  // at most
     const dim3 grid((unsigned)std::min<int64_t>(ctx->cu_count * 24, listed * TRI_PARTS)), block(TRI_BLOCK_NT);
-    if (ctx->d_tri_chunked)
+    if (ctx->d_tri_chunked && ctx->tri_chunked != 0)  // unknown (-1) until the first count is read back
         hipLaunchKernelGGL(k_triangles_block<true>, grid, block, 0, ctx->stream, a, ctx->d_tri_chunked + 1,
                            ctx->d_tri_chunked);
     hipLaunchKernelGGL(k_triangles_block<false>, grid, block, 0, ctx->stream, a, a.list, a.listed);
@@ -549,11 +553,12 @@ int triangles_dev(pcd_ctx *ctx) {
     hipLaunchKernelGGL(k_cc_partial, dim3(TSUM_BLOCKS), dim3(256), 0, ctx->stream, ctx->n, ctx->d_indices, ctx->d_tri,
                        ctx->d_dacc);
     hipLaunchKernelGGL(k_sum_partials_plain, dim3(1), dim3(256), 0, ctx->stream, ctx->d_dacc, TSUM_BLOCKS,
-                       ctx->d_result);
+                       ctx->d_result, ctx->d_tri_chunked);
     PCD_HIP(hipGetLastError());
-    PCD_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    PCD_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     PCD_HIP(hipStreamSynchronize(ctx->stream));
     ctx->cc = ctx->h_result[0];
+    if (ctx->d_tri_chunked) ctx->tri_chunked = (int)ctx->h_result[1];
     ctx->has_triangles = true;
     return PCD_OK;
 }
@@ -567,7 +572,7 @@ int wcc_metric_enqueue(pcd_ctx *ctx) {
     hipLaunchKernelGGL(k_wcc_partial, dim3(TSUM_BLOCKS), dim3(256), 0, ctx->stream, ctx->n, ctx->d_labels,
                        ctx->d_stats, ctx->d_tri, ctx->d_tri_deg, ctx->d_it, ctx->d_itd, ctx->d_dacc);
     hipLaunchKernelGGL(k_sum_partials_plain, dim3(1), dim3(256), 0, ctx->stream, ctx->d_dacc, TSUM_BLOCKS,
-                       ctx->d_result);
+                       ctx->d_result, (const int32_t *)nullptr);
     PCD_HIP(hipGetLastError());
     if (!ctx->capturing)
         PCD_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
