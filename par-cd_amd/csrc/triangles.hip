@@ -475,9 +475,12 @@ __global__ __launch_bounds__(256) void k_sum_partials_plain(const double *part, 
     }
 }
 
-// The arrays of the counts in one allocation, cut at 64 words: a user counts a
-// graph once, and seven allocations and three launches for the list were 12 of
-// the 100 us that call takes on up to some 10,000 entries.
+// The arrays of the counts.  A user counts a graph once, and seven allocations
+// and three launches for the list were 12 of the 100 us that call takes on up to
+// some 10,000 entries: up to TRI_ONE_ALLOC words share one allocation (cut at 64
+// words).  Larger arrays have one each; together they took longer to allocate
+// (1 M vertices, 15 M entries: the first count 2.6 ms in one, 2.1 in seven).
+constexpr int64_t TRI_ONE_ALLOC = 1 << 19;
 static int ensure_tri_buffers(pcd_ctx *ctx) {
     if (ctx->d_tri) return PCD_OK;
     const int64_t E = (int64_t)2 * ctx->m;
@@ -485,23 +488,32 @@ static int ensure_tri_buffers(pcd_ctx *ctx) {
     const int64_t cap = std::min<int64_t>(ctx->n, E / (TRI_WAVE + 1)) + 1;
     // and those above one table's
     const int64_t chunked = ctx->max_degree > TRI_CHUNK ? std::min<int64_t>(ctx->n, E / (TRI_CHUNK + 1)) + 1 : 0;
-    auto words = [](int64_t w) { return (w + 63) & ~(int64_t)63; };
-    const int64_t per_vertex = words((int64_t)ctx->n + 1), flags = words(E / 4 + 1);
-    int32_t *p = nullptr;
-    PCD_TRY(dev_alloc_t(ctx, &p, 5 * per_vertex + flags + words(cap + 1) + words(chunked + 1)));
-    int32_t *at = p + per_vertex;
-    auto take = [&](int64_t w) {
-        int32_t *x = at;
-        at += w;
-        return x;
-    };
-    ctx->d_tri_deg = take(per_vertex);
-    ctx->d_lowpos = take(per_vertex);
-    ctx->d_it = take(per_vertex);
-    ctx->d_itd = take(per_vertex);
-    ctx->d_tri_flag = (uint8_t *)take(flags);
-    ctx->d_tri_list = take(words(cap + 1));
-    ctx->d_tri_chunked = chunked ? take(words(chunked + 1)) : nullptr;
+    constexpr int ARRAYS = 8;
+    const int64_t n1 = (int64_t)ctx->n + 1, none = chunked ? chunked + 1 : 0;
+    const int64_t words[ARRAYS] = {n1, n1, n1, n1, n1, E / 4 + 1, cap + 1, none};
+    int64_t total = 0;
+    for (int64_t w : words) total += (w + 63) & ~(int64_t)63;
+    int32_t *array[ARRAYS] = {}, *block = nullptr;
+    if (total <= TRI_ONE_ALLOC) PCD_TRY(dev_alloc_t(ctx, &block, total));
+    for (int i = 0; i < ARRAYS; i++) {
+        if (words[i] == 0) continue;
+        if (block) {
+            array[i] = block;
+            block += (words[i] + 63) & ~(int64_t)63;
+            continue;
+        }
+        const int rc = dev_alloc_t(ctx, &array[i], words[i]);
+        if (rc == PCD_OK) continue;
+        for (int k = 0; k < i; k++) dev_free(ctx, array[k]);
+        return rc;
+    }
+    ctx->d_tri_deg = array[1];
+    ctx->d_lowpos = array[2];
+    ctx->d_it = array[3];
+    ctx->d_itd = array[4];
+    ctx->d_tri_flag = (uint8_t *)array[5];
+    ctx->d_tri_list = array[6];
+    ctx->d_tri_chunked = array[7];
     ctx->tri_chunked = -1;
     if (chunked) PCD_TRY(fill_i32(ctx, ctx->d_tri_chunked, 0, 1));
     hipLaunchKernelGGL(k_lowpos, dim3(grid_for(ctx, ctx->n, 256)), dim3(256), 0, ctx->stream, ctx->n, ctx->d_indices,
@@ -516,7 +528,7 @@ static int ensure_tri_buffers(pcd_ctx *ctx) {
     else
         PCD_TRY(device_scan(ctx, ctx->n, is_long, store, nullptr));
     PCD_HIP(hipGetLastError());
-    ctx->d_tri = p;  // set last: the others are there
+    ctx->d_tri = array[0];  // set last: the others are there
     return PCD_OK;
 }
 
