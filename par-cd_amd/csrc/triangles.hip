@@ -13,7 +13,7 @@
 // triangle uses this entry" matters, so a hit stores a flag byte instead of
 // adding to a counter in memory.  R-MAT-18 (3.8 M edges, 660 M lookups):
 // 6.4 ms with binary searches, an atomic per hit and a pass that summed the
-// counters with two atomics per edge; 1.2 ms so, 540 G lookups/s, bound by the
+// counters with two atomics per edge; 1.1 ms so, 600 G lookups/s, bound by the
 // instructions and LDS reads of a lookup.  With labels given, only edges and triangles inside one
 // community count (rules.cpp:172,185): neighbours of other communities are
 // left out of the prefix.
@@ -279,11 +279,11 @@ __device__ inline void tri_clip(const TriArgs &a, int lo, int hi, int &s, int &l
 // a list and a launch of their own: the parts below are then counted over them
 // alone (R-MAT-19 with shuffled ids, clipped, 57 -> 18 ms), and the clipping in
 // one kernel with the others cost these 10 % (R-MAT-20 3.5 -> 3.9 ms).  Where
-// the list is short,
-// up to TRI_PARTS workgroups share a vertex, each with its own table and a part
-// of the rows: the rows of one wave are a serial chain.  That and the smaller
-// units of k_triangles_wave, whole call: R-MAT-11 237 -> 97 us, R-MAT-13 332 ->
-// 166, R-MAT-15 435 -> 304, R-MAT-18 unchanged.
+// the list is short, up to TRI_PARTS workgroups share a vertex, each with its
+// own table and a part of the rows: the rows of one wave are a serial chain.
+// With that and the smaller units of k_triangles_wave a repeated call takes 100
+// us for R-MAT-11, 172 for R-MAT-13 (237 and 332 without, 142 and 270 with a
+// binary search per lookup); R-MAT-18 is unchanged.
 constexpr int TRI_PARTS = 16, TRI_BLOCK_NT = 256;
 template <bool CHUNKS>
 __global__ __launch_bounds__(TRI_BLOCK_NT) void k_triangles_block(TriArgs a, const int32_t *list,
